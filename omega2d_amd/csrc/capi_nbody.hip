@@ -159,7 +159,8 @@ int o2d_hip_morton_order_dev_d(const o2d_env* env, int64_t n, const double* x, c
   if (n > 0 && (!x || !y || !keys || !order)) return fail(O2D_ERR_ARG, "NULL array");
   Device* d;
   O2D_TRY(device(env->device, &d));
-  return morton_order(d, dev_stream(env), n, x, y, false, x0, y0, inv_extent, keys, order);
+  return morton_order(d, dev_stream(env), n, x, y, false, x0, y0, inv_extent, keys, order,
+                      nullptr, true);
 }
 
 }  // extern "C"

@@ -22,10 +22,11 @@ int check_pp(const o2d_env* env, int64_t ns, const void* sx, const void* sy, con
              const void* sr, int64_t nt, const void* tx, const void* ty, const void* tu,
              const void* tv, const void* tw, const void* te);
 
-// 32-bit Morton keys and stable order (bbox: derive the box on device from x, y)
+// 32-bit Morton keys and stable order (bbox: derive the box on device from x, y); keys_out
+// holds the sorted keys when want_keys, else scratch. sort.hip
 int morton_order(Device* d, hipStream_t s, int64_t n, const double* x, const double* y,
                  bool bbox, double x0, double y0, double inv, uint32_t* keys_out,
-                 uint32_t* order_out, Workspace* ws = nullptr);
+                 uint32_t* order_out, Workspace* ws, bool want_keys);
 
 int panels_on_points_dev(Device* d, hipStream_t s, int64_t nnodes, const double* nx,
                          const double* ny, int64_t np, const uint32_t* idx, const double* vs,

@@ -22,8 +22,6 @@
 // Both forms split the source range into chunks when there are too few target workgroups to
 // fill the GPU; chunk partials are then reduced in a fixed order by a second kernel (no float
 // atomics, so results are reproducible run to run).
-#include <hipcub/hipcub.hpp>
-
 #include <algorithm>
 #include <cstring>
 
@@ -460,29 +458,8 @@ __global__ __launch_bounds__(kBlock) void reduce_chunks_kernel(int64_t nchunk, i
   if (pw) ow[o] += sw;
 }
 
-// ---------------------------------------------------------------------------- Morton order
+// ---------------------------------------------------------------------------- staging
 
-struct BBox {
-  double x0, y0, inv_extent, pad;
-};
-
-__device__ __forceinline__ uint32_t spread16(uint32_t v) {
-  v &= 0xFFFFu;
-  v = (v | (v << 8)) & 0x00FF00FFu;
-  v = (v | (v << 4)) & 0x0F0F0F0Fu;
-  v = (v | (v << 2)) & 0x33333333u;
-  v = (v | (v << 1)) & 0x55555555u;
-  return v;
-}
-
-__device__ __forceinline__ double warp_min(double v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-  return v;
-}
-__device__ __forceinline__ double warp_max(double v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
-}
 __device__ __forceinline__ double warp_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
@@ -490,110 +467,6 @@ __device__ __forceinline__ double warp_sum(double v) {
 __device__ __forceinline__ float warp_maxf(float v) {
   for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
   return v;
-}
-
-// per-block min/max of x and y -> part[4*block + {0,1,2,3}] = xmin, ymin, xmax, ymax
-__global__ __launch_bounds__(kBlock) void bbox_partial_kernel(int64_t n, const double* __restrict__ x,
-                                                              const double* __restrict__ y,
-                                                              double* __restrict__ part) {
-  __shared__ double red[4][kBlock / 64];
-  double xmn = INFINITY, ymn = INFINITY, xmx = -INFINITY, ymx = -INFINITY;
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kBlock) {
-    xmn = fmin(xmn, x[i]);
-    xmx = fmax(xmx, x[i]);
-    ymn = fmin(ymn, y[i]);
-    ymx = fmax(ymx, y[i]);
-  }
-  xmn = warp_min(xmn);
-  ymn = warp_min(ymn);
-  xmx = warp_max(xmx);
-  ymx = warp_max(ymx);
-  const int wv = threadIdx.x / 64, ln = threadIdx.x % 64;
-  if (ln == 0) {
-    red[0][wv] = xmn;
-    red[1][wv] = ymn;
-    red[2][wv] = xmx;
-    red[3][wv] = ymx;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kBlock / 64; ++w) {
-      xmn = fmin(xmn, red[0][w]);
-      ymn = fmin(ymn, red[1][w]);
-      xmx = fmax(xmx, red[2][w]);
-      ymx = fmax(ymx, red[3][w]);
-    }
-    part[4 * blockIdx.x + 0] = xmn;
-    part[4 * blockIdx.x + 1] = ymn;
-    part[4 * blockIdx.x + 2] = xmx;
-    part[4 * blockIdx.x + 3] = ymx;
-  }
-}
-
-// one workgroup of kBlock threads folds the per-block partials (min/max are exact, so the
-// order does not matter)
-__global__ __launch_bounds__(kBlock) void bbox_final_kernel(int nblk, const double* __restrict__ part,
-                                                            BBox* __restrict__ out) {
-  __shared__ double red[4][kBlock / 64];
-  double xmn = INFINITY, ymn = INFINITY, xmx = -INFINITY, ymx = -INFINITY;
-  for (int b = threadIdx.x; b < nblk; b += kBlock) {
-    xmn = fmin(xmn, part[4 * b + 0]);
-    ymn = fmin(ymn, part[4 * b + 1]);
-    xmx = fmax(xmx, part[4 * b + 2]);
-    ymx = fmax(ymx, part[4 * b + 3]);
-  }
-  xmn = warp_min(xmn);
-  ymn = warp_min(ymn);
-  xmx = warp_max(xmx);
-  ymx = warp_max(ymx);
-  const int wv = threadIdx.x / 64, ln = threadIdx.x % 64;
-  if (ln == 0) {
-    red[0][wv] = xmn;
-    red[1][wv] = ymn;
-    red[2][wv] = xmx;
-    red[3][wv] = ymx;
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int w = 1; w < kBlock / 64; ++w) {
-    xmn = fmin(xmn, red[0][w]);
-    ymn = fmin(ymn, red[1][w]);
-    xmx = fmax(xmx, red[2][w]);
-    ymx = fmax(ymx, red[3][w]);
-  }
-  const double ext = fmax(xmx - xmn, ymx - ymn);
-  BBox b;
-  b.x0 = xmn;
-  b.y0 = ymn;
-  b.inv_extent = ext > 0.0 ? 1.0 / ext : 0.0;
-  b.pad = 0.0;
-  *out = b;
-}
-
-// q = clamp(floor(((x - x0) * inv) * 65536), 0, 65535) with unfused IEEE operations
-__device__ __forceinline__ uint32_t quant16(double v, double v0, double inv) {
-#pragma clang fp contract(off)
-  double q = floor(__dmul_rn(__dmul_rn(__dsub_rn(v, v0), inv), 65536.0));
-  q = q < 0.0 ? 0.0 : (q > 65535.0 ? 65535.0 : q);
-  return (uint32_t)q;
-}
-
-__global__ __launch_bounds__(kBlock) void morton_kernel(int64_t n, const double* __restrict__ x,
-                                                        const double* __restrict__ y,
-                                                        const BBox* __restrict__ bb,
-                                                        double x0, double y0, double inv,
-                                                        uint32_t* __restrict__ keys,
-                                                        uint32_t* __restrict__ order) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  if (bb) {
-    x0 = bb->x0;
-    y0 = bb->y0;
-    inv = bb->inv_extent;
-  }
-  keys[i] = spread16(quant16(x[i], x0, inv)) | (spread16(quant16(y[i], y0, inv)) << 1);
-  order[i] = (uint32_t)i;
 }
 
 // One wave per group of 64 sources (in Morton order): the fp64 centroid (a wave sum in a fixed
@@ -808,39 +681,6 @@ int gather_targets(hipStream_t s, int core, int64_t n, const uint32_t* order, co
 
 }  // namespace
 
-// Morton keys and the stable key order; bbox == true derives the box from the data on device.
-int morton_order(Device* d, hipStream_t s, int64_t n, const double* x, const double* y,
-                 bool bbox, double x0, double y0, double inv, uint32_t* keys_out,
-                 uint32_t* order_out, Workspace* ws) {
-  if (n <= 0) return 0;
-  void *kA, *oA, *bbp = nullptr;
-  O2D_TRY(take(d, ws, kKeysA, n * sizeof(uint32_t), s, &kA));
-  O2D_TRY(take(d, ws, kOrderA, n * sizeof(uint32_t), s, &oA));
-  BBox* bb = nullptr;
-  if (bbox) {
-    const int nblk = (int)std::min<int64_t>((n + kBlock - 1) / kBlock, 1024);
-    O2D_TRY(take(d, ws, kBBox, sizeof(double) * (4 * nblk + 4), s, &bbp));
-    double* part = static_cast<double*>(bbp);
-    bb = reinterpret_cast<BBox*>(part + 4 * nblk);
-    bbox_partial_kernel<<<nblk, kBlock, 0, s>>>(n, x, y, part);
-    bbox_final_kernel<<<1, kBlock, 0, s>>>(nblk, part, bb);
-    O2D_LAUNCH_CHECK();
-  }
-  morton_kernel<<<grid1(n), kBlock, 0, s>>>(n, x, y, bb, x0, y0, inv, static_cast<uint32_t*>(kA),
-                                            static_cast<uint32_t*>(oA));
-  O2D_LAUNCH_CHECK();
-  size_t tbytes = 0;
-  O2D_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tbytes, static_cast<uint32_t*>(kA),
-                                             keys_out, static_cast<uint32_t*>(oA), order_out,
-                                             (int)n, 0, 32, s));
-  void* tmp;
-  O2D_TRY(take(d, ws, kSortTemp, tbytes, s, &tmp));
-  O2D_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, tbytes, static_cast<uint32_t*>(kA), keys_out,
-                                             static_cast<uint32_t*>(oA), order_out, (int)n, 0, 32,
-                                             s));
-  return 0;
-}
-
 // The most source chunks whose fp64 partials (nf per target) fit what is left of *ws; no limit
 // when the temporaries come from the buffer pool.
 int64_t max_chunks(const Workspace* ws, int nf, int64_t nt) {
@@ -863,7 +703,7 @@ int prep_targets(Device* d, hipStream_t s, Workspace* ws, int core, int64_t nt, 
     O2D_TRY(take(d, ws, kTrgKeys, nt * sizeof(uint32_t), s, &kT));
     O2D_TRY(take(d, ws, kTrgOrder, nt * sizeof(uint32_t), s, &oT));
     O2D_TRY(morton_order(d, s, nt, tx, ty, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(kT),
-                         static_cast<uint32_t*>(oT), ws));
+                         static_cast<uint32_t*>(oT), ws, false));
     o = static_cast<const uint32_t*>(oT);
   }
   void *pp, *wp = nullptr;
@@ -902,7 +742,7 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
     const uint32_t* order = nullptr;
     if (sort) {
       O2D_TRY(morton_order(d, s, ns, sx, sy, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(kB),
-                           static_cast<uint32_t*>(oB), ws));
+                           static_cast<uint32_t*>(oB), ws, false));
       order = static_cast<const uint32_t*>(oB);
     }
     Src64* src = static_cast<Src64*>(sp);
@@ -962,7 +802,7 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
   O2D_TRY(take(d, ws, kTileCent, ngroups * sizeof(GroupInfo), s, &tcent));
   KernelTimer kprep(O2D_KT_SPLIT_PREP, s);
   O2D_TRY(morton_order(d, s, ns, sx, sy, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(kB),
-                       static_cast<uint32_t*>(oB), ws));
+                       static_cast<uint32_t*>(oB), ws, false));
   const uint32_t* order = static_cast<const uint32_t*>(oB);
   GroupInfo* cent = static_cast<GroupInfo*>(tcent);
   float4* src = static_cast<float4*>(tsrc);

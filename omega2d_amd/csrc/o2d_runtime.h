@@ -20,7 +20,7 @@ enum Slot : int {
   kStageF0, kStageF1, kStageF2, kStageF3, kStageF4, kStageF5, kStageF6, kStageF7,
   kStageF8, kStageF9, kStageF10,
   kPartials,
-  kKeysA, kKeysB, kOrderA, kOrderB, kSortTemp, kBBox,
+  kKeysA, kKeysB, kOrderA, kOrderB, kSortTemp, kSortTab, kBBox,
   kTileSrc, kTileCent,
   kTrgKeys, kTrgOrder, kTrgPos, kTrgW, kSrc64,
   kPanX, kPanY, kPanIdx, kPanVs, kPanSs,
@@ -92,8 +92,9 @@ int take(Device* d, Workspace* ws, Slot which, size_t bytes, hipStream_t s, void
 
 int check_env(const o2d_env* env);
 
-// The Morton order of n points (x, y device arrays): *order (n entries, in the kOrderB slot, so
-// valid until that slot is next used) lists the point indices along the curve. morton.hip.
+// The Morton order of n points (x, y device arrays; 8 bits per axis on their box, so that a group
+// of 64 points is compact; no result depends on it): *order (n entries, in the kOrderB slot, so
+// valid until that slot is next used) lists the point indices along the curve. sort.hip.
 int morton_order16(Device* d, hipStream_t s, int64_t n, const double* x, const double* y,
                    const uint32_t** order);
 

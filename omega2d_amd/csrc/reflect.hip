@@ -18,8 +18,6 @@
 //     already exceed the current acceptance bound by a margin far above its rounding error.
 // Node normals are the sums of the normals of the panels that share the node, added in panel
 // order (end 0 before end 1), from a stable sort of the panel ends by node.
-#include <hipcub/hipcub.hpp>
-
 #include <cfloat>
 #include <climits>
 #include <cmath>
@@ -27,6 +25,7 @@
 
 #include "nbody.h"
 #include "o2d_runtime.h"
+#include "sort.h"
 
 #pragma clang fp contract(off)
 
@@ -54,19 +53,6 @@ __device__ inline double next_down(double m) {  // nextafter(m, 0) for m >= 0
 }
 __device__ inline double next_up(double m) {    // nextafter(m, DBL_MAX) for 0 <= m <= DBL_MAX
   return m < DBL_MAX ? __longlong_as_double(__double_as_longlong(m) + 1) : m;
-}
-
-// key/value pairs (node, panel end) for the node-normal sort; out-of-range nodes are clamped
-// here and counted by panel_rec_kernel
-__global__ __launch_bounds__(kBlock) void end_keys_kernel(int64_t nends, int64_t nnodes,
-                                                          const uint32_t* __restrict__ idx,
-                                                          uint32_t* __restrict__ key,
-                                                          uint32_t* __restrict__ val) {
-  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (e >= nends) return;
-  const uint32_t k = idx[e];
-  key[e] = (int64_t)k < nnodes ? k : (uint32_t)(nnodes - 1);
-  val[e] = (uint32_t)e;
 }
 
 // node normal = sum over the node's panel ends in end order; the first end of each run sums it
@@ -845,29 +831,22 @@ int near_dev(Device* d, hipStream_t s, int mode, int method, double cutoff_mult,
     double *nnx = nullptr, *nny = nullptr;
     if (mode != kNearest) {
       const int64_t nends = 2 * np;
-      void *kA, *vA, *kB, *vB, *nn;
-      O2D_TRY(slot(d, kKeysA, nends * sizeof(uint32_t), s, &kA));
-      O2D_TRY(slot(d, kOrderA, nends * sizeof(uint32_t), s, &vA));
+      void *kB, *vB, *nn;
       O2D_TRY(slot(d, kKeysB, nends * sizeof(uint32_t), s, &kB));
       O2D_TRY(slot(d, kOrderB, nends * sizeof(uint32_t), s, &vB));
       O2D_TRY(slot(d, kNodeNorm, 2 * sizeof(double) * (size_t)nnodes, s, &nn));
       nnx = static_cast<double*>(nn);
       nny = nnx + nnodes;
-      end_keys_kernel<<<blocks(nends), kBlock, 0, s>>>(nends, nnodes, idx,
-                                                       static_cast<uint32_t*>(kA),
-                                                       static_cast<uint32_t*>(vA));
-      O2D_LAUNCH_CHECK();
       int bits = 1;
       while (bits < 32 && ((uint64_t)1 << bits) < (uint64_t)nnodes) ++bits;
-      size_t tbytes = 0;
-      O2D_HIP(hipcub::DeviceRadixSort::SortPairs(
-          nullptr, tbytes, static_cast<uint32_t*>(kA), static_cast<uint32_t*>(kB),
-          static_cast<uint32_t*>(vA), static_cast<uint32_t*>(vB), (int)nends, 0, bits, s));
-      void* tmp;
-      O2D_TRY(slot(d, kSortTemp, tbytes, s, &tmp));
-      O2D_HIP(hipcub::DeviceRadixSort::SortPairs(
-          tmp, tbytes, static_cast<uint32_t*>(kA), static_cast<uint32_t*>(kB),
-          static_cast<uint32_t*>(vA), static_cast<uint32_t*>(vB), (int)nends, 0, bits, s));
+      // the panel ends by node (out-of-range nodes are clamped here and counted by
+      // panel_rec_kernel)
+      KeyGen g{};
+      g.kind = kNode;
+      g.idx = idx;
+      g.nnodes = (uint32_t)nnodes;
+      O2D_TRY(sort_order(d, s, nullptr, nends, g, bits, static_cast<uint32_t*>(kB),
+                         static_cast<uint32_t*>(vB), true));
       node_normal_kernel<<<blocks(nends), kBlock, 0, s>>>(
           nends, static_cast<uint32_t*>(kB), static_cast<uint32_t*>(vB), pnx, pny, nnx, nny);
       O2D_LAUNCH_CHECK();

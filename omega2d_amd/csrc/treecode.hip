@@ -401,7 +401,7 @@ int tree_dev(Device* d, hipStream_t s, int core, double theta, int p, double tol
   {
     KernelTimer kt(O2D_KT_TREE_BUILD, s);
     O2D_TRY(morton_order(d, s, ns, sx, sy, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(tk),
-                         sorder));
+                         sorder, nullptr, false));
     tree_gather_kernel<<<(unsigned)((ns + kBlock - 1) / kBlock), kBlock, 0, s>>>(
         ns, sorder, sx, sy, ss, sr, core, xs, ys, ssorted, ws);
     O2D_LAUNCH_CHECK();
@@ -416,7 +416,7 @@ int tree_dev(Device* d, hipStream_t s, int core, double theta, int p, double tol
       O2D_LAUNCH_CHECK();
     }
     O2D_TRY(morton_order(d, s, nt, tx, ty, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(tk),
-                         torder));
+                         torder, nullptr, false));
     kt.stop();
   }
   // each wave's walk is a chain of dependent loads, so the walk wants many waves per SIMD, and
