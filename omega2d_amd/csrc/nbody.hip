@@ -87,21 +87,11 @@ __device__ __forceinline__ void tile_pairs64(const Src64* __restrict__ tile, con
         au[t] = __builtin_fma(-g, dy, au[t]);
         av[t] = __builtin_fma(g, dx, av[t]);
       } else {
-        double kk, bbb;
-        core_kg64<CORE>(dx, dy, d2, w, kk, bbb);
-        kk *= q.s;
-        bbb *= q.s;
-        au[t] = __builtin_fma(-kk, dy, au[t]);
-        av[t] = __builtin_fma(kk, dx, av[t]);
-        if constexpr (RES == O2D_VELANDVORT) {
-          // (bbb dx^2 + K) - (-bbb dy^2 - K)   src/Kernels.h:176-178
-          aw[t] += __builtin_fma(bbb, d2, 2.0 * kk);
-        } else {
-          // sqrt(dudx^2 + asym^2/4)           src/Kernels.h:225-230
-          const double dudx = -bbb * dx * dy;
-          const double asym = bbb * (dx * dx - dy * dy);
-          aw[t] += sqrt(__builtin_fma(dudx, dudx, 0.25 * asym * asym));
-        }
+        double aux;
+        const double g = q.s * core_kw64<CORE, RES>(dx, dy, d2, w, aux);
+        au[t] = __builtin_fma(-g, dy, au[t]);
+        av[t] = __builtin_fma(g, dx, av[t]);
+        aw[t] = __builtin_fma(RES == O2D_VELANDVORT ? q.s : __builtin_fabs(q.s), aux, aw[t]);
       }
     }
   }

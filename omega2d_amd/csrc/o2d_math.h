@@ -118,15 +118,23 @@ __device__ __forceinline__ double core_k64(double dx, double dy, double d2, doub
   }
 }
 
-// K and bbb = 2 dK/d(d^2) in the reference's gradient forms (src/CoreFunc.h:64-81, 156-180,
-// 208-229, 256-274, 301-321). Gaussian at d2 == 0: bbb = 0 (the reference yields NaN there).
-template <int CORE>
-__device__ __forceinline__ void core_kg64(double dx, double dy, double d2, double w, double& k,
-                                          double& bbb) {
+// K and the vorticity or shear factor of a pair's sums, both without the source strength. With
+// bbb = 2 dK/d(d^2) (src/CoreFunc.h:64-81, 156-180, 208-229, 256-274, 301-321) the reference adds
+// s (bbb d^2 + 2 K) to the vorticity and sqrt((s bbb dx dy)^2 + (s bbb (dx^2 - dy^2))^2 / 4) =
+// |s| |bbb| d^2 / 2 to the shear (src/Kernels.h:139-231; dx^2 dy^2 + (dx^2 - dy^2)^2 / 4 = d^4 / 4).
+// The algebraic cores take the closed forms that follow (the table above core_kw32), which
+// need no square root and do not cancel; the Gaussian its gradient form, with bbb = 0 at
+// d2 == 0 (the reference yields NaN there). The fp64 loops are bound by vector issue, and the
+// square root was most of it: 100,003 V2 particles on themselves with shear 14.7 -> 6.3 ms
+// (25 issue slots a pair; 7.35 ms with |bbb| d^2 / 2 from the gradient form).
+template <int CORE, int RES>
+__device__ __forceinline__ double core_kw64(double dx, double dy, double d2, double w,
+                                            double& aux) {
+  constexpr bool kVort = RES == O2D_VELANDVORT;
   if constexpr (CORE == O2D_CORE_RM) {
     const double r = rcp64(d2 + w);
-    k = r;
-    bbb = -2.0 * r * r;
+    aux = (kVort ? 2.0 * w : d2) * r * r;
+    return r;
   } else if constexpr (CORE == O2D_CORE_GAUSSIAN) {
     const double cf = rcp64(w);
     const double x = d2 * cf;
@@ -134,23 +142,27 @@ __device__ __forceinline__ void core_kg64(double dx, double dy, double d2, doubl
     const double e = exp(-x);
     const int br = gauss_branch(x, dx, dy, w);
     const double r = br > 0 ? ood2 : (br < 0 ? cf : ood2 * (1.0 - e));
-    k = r;
-    bbb = (d2 == 0.0) ? 0.0 : (-2.0 * r * ood2 + 2.0 * cf * ood2 * e);
+    const double bbb = (d2 == 0.0) ? 0.0 : (-2.0 * r * ood2 + 2.0 * cf * ood2 * e);
+    aux = kVort ? __builtin_fma(bbb, d2, 2.0 * r) : 0.5 * __builtin_fabs(bbb) * d2;
+    return r;
   } else if constexpr (CORE == O2D_CORE_WL) {
     const double dd = d2 + w;
-    const double ood2s = rcp64(dd * dd);
-    const double r = (dd + w) * ood2s;
-    k = r;
-    bbb = (2.0 - 4.0 * r * dd) * ood2s;
+    const double r = rcp64(dd);
+    const double q = w * r;  // K = (1 + q) r
+    if constexpr (kVort) aux = 4.0 * q * q * r;
+    else aux = __builtin_fma(3.0, w, d2) * r * (d2 * r) * r;
+    return __builtin_fma(q, r, r);
   } else if constexpr (CORE == O2D_CORE_V2) {
     const double r = rsq64(__builtin_fma(d2, d2, w));
-    k = r;
-    bbb = -2.0 * r * r * r * d2;
+    const double q = d2 * r;
+    aux = kVort ? 2.0 * w * r * (r * r) : r * q * q;
+    return r;
   } else {
-    const double ds6 = __builtin_fma(d2 * d2, d2, w);
-    const double r = rcbrt(ds6);
-    k = r;
-    bbb = -2.0 * d2 * d2 * r * rcp64(ds6);
+    const double r = rcbrt(__builtin_fma(d2 * d2, d2, w));
+    const double q = r * r;
+    const double p = d2 * r;
+    aux = kVort ? 2.0 * w * q * q : p * p * p * r;
+    return r;
   }
 }
 
