@@ -29,6 +29,10 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kTile = 256;
 constexpr int kTpl = 2;
+#ifndef O2D_TREE_PAIRS
+#define O2D_TREE_PAIRS 1e8
+#endif
+constexpr double kTreePairs = O2D_TREE_PAIRS;
 
 struct alignas(16) Probe {
   double x, y, gu, gv;
@@ -200,6 +204,8 @@ int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx
                 const double* tx, const double* ty, const double* gu, const double* gv,
                 double* gx, double* gy, double* gs, double* gr) {
   if (ns == 0 || nt == 0) return 0;
+  if (core == O2D_CORE_GAUSSIAN && (double)ns * (double)nt >= kTreePairs)
+    return gauss_adjoint_tree_dev(d, s, ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, gx, gy, gs, gr);
   const int64_t swgs = (ns + kBlock * kTpl - 1) / (kBlock * kTpl);
   const int64_t ntiles = (nt + kTile - 1) / kTile;
   const int64_t want = O2D_WANT_ADJ * (int64_t)d->num_cu;

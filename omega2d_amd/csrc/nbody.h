@@ -57,6 +57,20 @@ int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx
                 const double* tx, const double* ty, const double* gu, const double* gv,
                 double* gx, double* gy, double* gs, double* gr);
 
+// the fp64 Gaussian velocity sum and its adjoint with the sources beyond the compact cutoff taken
+// by clusters, to rounding (treecode.hip); and the pairs from which that is faster than the pair
+// by pair sums: particles on themselves 147 us against 152 at 8,000, 228 against 247 at 16,000, 310
+// against 597 at 32,000; 30,000 on 3,000 points 209 us against 172, 250,000 on 4,096 439 us
+// against 658
+constexpr double kTreePairs = 2e8;
+int gauss_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const double* sy,
+                   const double* ss, const double* sr, int64_t nt, const double* tx,
+                   const double* ty, const double* tr, double* tu, double* tv);
+int gauss_adjoint_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx,
+                           const double* sy, const double* ss, const double* sr, int64_t nt,
+                           const double* tx, const double* ty, const double* gu,
+                           const double* gv, double* gx, double* gy, double* gs, double* gr);
+
 // Gaussian vorticity of particles at targets (fp64, +=), device pointers
 int vorticity_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const double* sy,
                   const double* ss, const double* sr, int64_t nt, const double* tx,

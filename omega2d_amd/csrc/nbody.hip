@@ -59,6 +59,10 @@ constexpr int kGroup = 64;   // sources sharing one centroid in the split form
 #endif
 constexpr int kMinChunkTiles = 16;
 constexpr int kStage = 4;  // source tiles brought into LDS per stage of the split kernel
+#ifndef O2D_TREE_PAIRS
+#define O2D_TREE_PAIRS 1e8
+#endif
+constexpr double kTreePairs = O2D_TREE_PAIRS;
 constexpr int kTpl64 = O2D_TPL64;  // targets per lane, plain form
 constexpr int kTpl32 = O2D_TPL32;  // targets per lane, split form
 
@@ -715,6 +719,9 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
   // the radix sort of the Morton keys takes an int count
   if (ns > 0x7fffffffLL || nt > 0x7fffffffLL)
     return fail(O2D_ERR_SIZE, "more than 2^31 - 1 sources or targets");
+  if (prec == O2D_PLAIN_FP64 && core == O2D_CORE_GAUSSIAN && res == O2D_VELONLY && !ws &&
+      (double)ns * (double)nt >= kTreePairs)
+    return gauss_tree_dev(d, s, ns, sx, sy, ss, sr, nt, tx, ty, tr, tu, tv);
   const bool trp = tr != nullptr;
   // targets that are the sources themselves (a collection acting on itself) share their order
   const bool self = tx == sx && ty == sy && nt == ns;

@@ -31,7 +31,8 @@ enum Slot : int {
   kGradX, kGradY, kGradS, kGradR,
   kNearPart, kNodeNorm, kPanRec, kCutTable, kNearCounts, kNearTiles,
   kInv, kSolveTmp,
-  kTreeKeys, kTreeOrder, kTreeTOrder, kTreeSrc, kTreeCells, kTreeMom,
+  kTreeKeys, kTreeOrder, kTreeTOrder, kTreeSrc, kTreeCells, kTreeBox, kTreeMom,
+  kTreeTrg, kTreeSuper,
   kPan2X, kPan2Y, kPan2Idx, kPanGeom2,
   kLuPairs, kPanClus, kPanClusG, kPanClusS, kVortSrc,
   kNumSlots

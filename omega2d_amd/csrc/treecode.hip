@@ -1,21 +1,41 @@
-// treecode.hip - O(N log N) particles-on-points velocity, the summation the reference reserves
-// as summation_t barneshut (src/ExecEnv.h:26-31) behind the same operator as the direct sum.
+// treecode.hip - O(N log N) particle sums: the summation the reference reserves as summation_t
+// barneshut (src/ExecEnv.h:26-31) behind the same operator as the direct sum, and, at an
+// acceptance where the remainder is below rounding, the fp64 Gaussian velocity sum and its
+// adjoint beyond the compact cutoff, where K = 1/d^2 exactly (src/CoreFunc.h:120-122).
+//
+// With q_j the charge of source j (its strength; gv - i gu for the adjoint, whose sources are the
+// probes), far sources act on a target z through S = sum_j q_j / (z - z_j), and for the adjoint
+// also S2 = sum_j q_j / (z - z_j)^2 = -dS/dz. The unscaled velocity is u - i v = -i S.
 //
 // Tree: sources in Morton order, cut into leaves of kLeaf consecutive sources; each coarser
-// level groups kFan consecutive cells, so every cell is one contiguous Morton range and the tree
-// needs no pointers. Per cell: bounding-box centre c, radius r (covers every source), largest
-// radius term, and the complex moments M_k = sum_j s_j (z_j - c)^k, k < p (fp64). Parents get
-// their moments by the binomial shift of their children's.
+// level groups kFan consecutive cells, so every cell is one contiguous Morton range. Per cell: box
+// centre c, radius r (covers every source), largest radius term, and the moments
+// M_k = sum_j q_j ((z_j - c) / r)^k, k < p, in fp64 (scaled by the radius, so that no power
+// overflows or vanishes). Parents shift their children's. A cell with a charge or radius that
+// is not finite gets r = inf, is never used through its moments, and reaches the sum pair by pair.
 //
-// Evaluation: one wave per 64 Morton-ordered targets walks the tree from the root with a stack
-// in LDS. A cell is used through its moments when, for every lane of the wave,
-//   r <= theta |z - c|                      (truncation of the Laurent series)
-//   the core equals 1/d^2 for every pair within core_tol, from d_min = |z - c| - r: exactly
-//   beyond the Gaussian's compact cutoff (d^2 > 16 w, src/CoreFunc.h:120-122); for the other
-//   cores through the bound on |K d^2 - 1| (RM w/d^2, WL w^2/d^4, V2 w/(2 d^4), V3 w/(3 d^6)).
-// Otherwise the cell is opened, and a leaf is summed directly with the exact core in fp64.
-// With S = sum_k M_k / (z - c)^(k+1), the unscaled velocity is u - i v = -i S, i.e.
-// u = Im S, v = Re S.
+// Evaluation, from the largest clusters of targets to the smallest:
+//   super groups   one workgroup per kSuper Morton-ordered targets opens the tree from the root,
+//                  every cell of a round tested by its own thread. Cells that are far for all the
+//                  targets become one local expansion about the targets' centre, L_l =
+//                  sum_j q_j / ..., (z - c_T)^l; cells no larger than half the super group that
+//                  are not far form its frontier;
+//   groups         one wave per 64 targets (one per lane) starts at the frontier. 64 cells are
+//                  tested at a time, one per lane, against the box of the wave's targets: far
+//                  cells are evaluated through their moments by every lane, leaves that are not
+//                  far pair by pair in fp64 with the exact core, the rest is opened.
+// A cell of radius r is far from targets at distance D or more from its centre when r <= theta D
+// and the core equals 1/d^2 for every pair within core_tol, from d_min = D - r: exactly beyond the
+// Gaussian's compact cutoff (d^2 > 16 w); for the other cores through the bound on |K d^2 - 1|
+// (RM w/d^2, WL w^2/d^4, V2 w/(2 d^4), V3 w/(3 d^6)). A local expansion of radius R at distance d
+// from the cell's centre also needs R <= theta (d - r).
+//
+// What bounds it: issue of the near pairs and of the moment sums. One wave that popped one cell
+// at a time from its own stack spent most of its time waiting for that cell's record and moments;
+// testing 64 cells at once takes a handful of dependent loads per wave, records of known cells
+// come as scalar loads, and the far cells of 1,024 targets are summed once, not sixteen times.
+// 1M blob particles on themselves plus 65,536 tracers (theta 0.6, order 28): 7.6 -> 3.1 ms, of which
+// the particles' groups 2.0, the tracers' 0.47, the two trees and orders 0.5.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -28,18 +48,40 @@ namespace o2d {
 
 namespace {
 
-constexpr int kLeaf = 64;     // sources per leaf
-constexpr int kFan = 4;       // children per cell
-constexpr int kMaxP = 32;     // largest expansion order
-constexpr int kMaxLevels = 15;  // 2^31 sources make 14 levels
-constexpr int kTBlock = 256;  // 4 waves, each with its own 64 targets
-constexpr int kStack = 96;    // per-wave stack entries (depth <= (kFan - 1) * levels + 1)
+constexpr int kLeaf = 32;       // sources per leaf
+constexpr int kFan = 4;         // children per cell
+constexpr int kMaxP = 32;       // largest expansion order; cells store this many moments
+constexpr int kMaxLevels = 16;  // 2^31 sources make 14 levels
 constexpr int kBlock = 256;
+constexpr int kWaves = kBlock / 64;
+constexpr int kGroupWaves = 1, kGroupBlock = 64 * kGroupWaves;  // a wave ends by itself
+constexpr int kSuper = 1024;    // targets per super group
+constexpr int kSuperBlock = 512;
+constexpr int kSuperWaves = kSuperBlock / 64;
+constexpr int kQueue = 1024;    // cells of one round of a super group
+constexpr int kFront = 512;     // frontier cells of a super group
+constexpr int kStack = 512;     // cells a group's wave has still to test
+constexpr int kStackSpare = 3 * kMaxLevels;  // what opening one cell at a time can add
+// acceptance at which the remainder of kMaxP moments is below rounding: a far cell's is at most
+// 3^-kMaxP = 5e-16 of sum |q_j| / D. (0.3 took 2.0 ms instead of 1.73 for 262,147 blob particles
+// on themselves and 9,973 tracers, 0.36, whose remainder is 6e-15, 1.59 ms; the error against 64
+// bits did not move, 5e-16, a quarter of the pair by pair sum's.)
+constexpr double kExactTheta = 1.0 / 3.0;
+// local expansions add a truncation of their own: they take cells from a little further away
+constexpr double kLocalShare = 0.85;
+// and groups take cells from a little further than theta says, so that the sum over many more
+// cells than the coarser groups of an earlier form used keeps its error
+constexpr double kThetaShare = 0.955;
+// waves per CU the group kernel aims for by sharing a group's cells and leaves out: every share
+// opens the same cells, so more of them cost more (1M particles: 32 and 64 equal; 10,000 tracers
+// in groups of 16: 264 us at 16, 369 at 32)
+constexpr int kWaves64 = 32, kWaves16 = 16;
+// fewer super groups than this leave most of the chip idle for longer than they save
+constexpr int64_t kMinSupers = 16;
 
-struct Cell {
-  double cx, cy, r, wmax;
-  double x0, y0, x1, y1;  // bounding box of the cell's sources
-};
+// A cell: head = (centre x, y, radius, largest radius term), kids = (first child, children); a
+// leaf has no children, and its first child is its index among the leaves. (As one struct the
+// records went through scratch memory wherever they were read ahead.)
 
 struct Levels {
   int n;                      // number of levels (level 0 = leaves, n - 1 = root)
@@ -47,330 +89,944 @@ struct Levels {
   int64_t cnt[kMaxLevels];    // cells per level
 };
 
-__global__ __launch_bounds__(kBlock) void tree_gather_kernel(
-    int64_t n, const uint32_t* __restrict__ order, const double* __restrict__ x,
-    const double* __restrict__ y, const double* __restrict__ s, const double* __restrict__ r,
-    int core, double* __restrict__ ox, double* __restrict__ oy, double* __restrict__ os,
-    double* __restrict__ ow) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t j = order[i];
-  ox[i] = x[j];
-  oy[i] = y[j];
-  if (os) os[i] = s[j];
-  if (ow) {
-    const double rr = r ? r[j] : 0.0;
-    ow[i] = core == O2D_CORE_V2   ? rterm<O2D_CORE_V2>(rr)
-            : core == O2D_CORE_V3 ? rterm<O2D_CORE_V3>(rr)
-                                  : rterm<O2D_CORE_RM>(rr);
-  }
-}
-
-// wave-wide reductions (every lane receives the result)
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
-  return v;
-}
-__device__ __forceinline__ double wave_min(double v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = fmin(v, __shfl_xor(v, m));
-  return v;
-}
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = fmax(v, __shfl_xor(v, m));
-  return v;
-}
-
-// leaves, one wave each (lane j holds source j of the leaf): bounding box, centre, radius,
-// largest radius term and the moments M_k = sum_j s_j (z_j - c)^k of <= kLeaf sources, each
-// moment a wave sum; lane k keeps M_k
-__global__ __launch_bounds__(kBlock) void tree_leaf_kernel(
-    int64_t ns, int64_t nleaf, int p, const double* __restrict__ x, const double* __restrict__ y,
-    const double* __restrict__ s, const double* __restrict__ w, Cell* __restrict__ cell,
-    double2* __restrict__ mom) {
-  const int lane = threadIdx.x & 63;
-  const int64_t c = (int64_t)blockIdx.x * (kBlock / 64) + threadIdx.x / 64;
-  if (c >= nleaf) return;  // whole waves leave together
-  const int64_t j = c * kLeaf + lane;
-  const bool in = j < ns;
-  const double xj = in ? x[j] : 0.0, yj = in ? y[j] : 0.0;
-  const double x0 = wave_min(in ? xj : INFINITY), x1 = wave_max(in ? xj : -INFINITY);
-  const double y0 = wave_min(in ? yj : INFINITY), y1 = wave_max(in ? yj : -INFINITY);
-  const double wm = wave_max(in ? w[j] : 0.0);
-  const double cx = 0.5 * (x0 + x1), cy = 0.5 * (y0 + y1);
-  const double dx = xj - cx, dy = yj - cy;
-  const double r2 = wave_max(in ? dx * dx + dy * dy : 0.0);
-  double pr = in ? s[j] : 0.0, pi = 0.0;  // s (z - c)^k
-  double mr = 0.0, mi = 0.0;
-  for (int k = 0; k < p; ++k) {
-    const double sr = wave_sum(pr), si = wave_sum(pi);
-    if (lane == k) {
-      mr = sr;
-      mi = si;
-    }
-    const double nr = pr * dx - pi * dy;
-    pi = pr * dy + pi * dx;
-    pr = nr;
-  }
-  // rounding of the offsets: a relative margin keeps r an upper bound
-  if (lane == 0) cell[c] = Cell{cx, cy, sqrt(r2) * (1.0 + 1e-12), wm, x0, y0, x1, y1};
-  if (lane < p) mom[c * p + lane] = make_double2(mr, mi);
-}
-
-// one coarser level, one wave per cell: bounding-box union, covering radius, and moments
-// shifted to the new centre, lane k forming M'_k = sum_children sum_{l <= k} C(k, l) M_l d^(k-l)
-// with d = c_child - c (the children's moments staged in LDS)
-__global__ __launch_bounds__(kBlock) void tree_up_kernel(int64_t nchild, int64_t ncell, int p,
-                                                         const Cell* __restrict__ child,
-                                                         const double2* __restrict__ cmom,
-                                                         Cell* __restrict__ cell,
-                                                         double2* __restrict__ mom) {
-  __shared__ double2 sm[kBlock / 64][kFan * kMaxP];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x / 64;
-  const int64_t c = (int64_t)blockIdx.x * (kBlock / 64) + wv;
-  if (c >= ncell) return;  // whole waves leave together; no block-wide barrier below
-  const int64_t k0 = c * kFan;
-  const int nch = (int)((k0 + kFan < nchild) ? kFan : nchild - k0);
-  for (int e = lane; e < nch * p; e += 64) sm[wv][e] = cmom[k0 * p + e];
-  double x0 = child[k0].x0, y0 = child[k0].y0, x1 = child[k0].x1, y1 = child[k0].y1, wm = 0.0;
-  for (int k = 0; k < nch; ++k) {
-    x0 = fmin(x0, child[k0 + k].x0);
-    y0 = fmin(y0, child[k0 + k].y0);
-    x1 = fmax(x1, child[k0 + k].x1);
-    y1 = fmax(y1, child[k0 + k].y1);
-    wm = fmax(wm, child[k0 + k].wmax);
-  }
-  const double cx = 0.5 * (x0 + x1), cy = 0.5 * (y0 + y1);
-  // the staged moments are read by other lanes of the same wave
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  double r = 0.0, ar = 0.0, ai = 0.0;
-  for (int ch = 0; ch < nch; ++ch) {
-    const double dx = child[k0 + ch].cx - cx, dy = child[k0 + ch].cy - cy;
-    r = fmax(r, sqrt(dx * dx + dy * dy) + child[k0 + ch].r);
-    if (lane < p) {
-      const int k = lane;
-      // l from k down to 0: C(k, l) M_l d^(k - l), with d^(k-l) and C(k, l) by recurrence
-      double dpr = 1.0, dpi = 0.0, binom = 1.0;
-      for (int l = k; l >= 0; --l) {
-        const double2 ml = sm[wv][ch * p + l];
-        ar += binom * (ml.x * dpr - ml.y * dpi);
-        ai += binom * (ml.x * dpi + ml.y * dpr);
-        const double nr = dpr * dx - dpi * dy;
-        dpi = dpr * dy + dpi * dx;
-        dpr = nr;
-        binom = binom * (double)l / (double)(k - l + 1);
-      }
-    }
-  }
-  if (lane == 0) cell[c] = Cell{cx, cy, r * (1.0 + 1e-12), wm, x0, y0, x1, y1};
-  if (lane < p) mom[c * p + lane] = make_double2(ar, ai);
-}
-
-// may the moments of a cell stand for its sources at a target d_min away?
-template <int CORE>
-__device__ __forceinline__ bool core_far(double dm2, double w, double tol) {
-  if constexpr (CORE == O2D_CORE_GAUSSIAN) {
-    return dm2 > 16.0 * w * (1.0 + 1e-12);
-  } else if constexpr (CORE == O2D_CORE_RM) {
-    return w <= tol * dm2;
-  } else if constexpr (CORE == O2D_CORE_WL) {
-    return w * w <= tol * dm2 * dm2;
-  } else if constexpr (CORE == O2D_CORE_V2) {
-    return w <= 2.0 * tol * dm2 * dm2;
-  } else {
-    return w <= 3.0 * tol * dm2 * dm2 * dm2;
-  }
-}
-
-struct TreeArgs {
-  Levels lv;
-  const Cell* cell;
-  const double2* mom;
-  const double* sx;
-  const double* sy;
-  const double* ss;
-  const double* sw;
-  int64_t ns;
-  int p;
-  double theta;
-  double tol;
-  // the walk may be split over ksplit waves per target group: wave k starts from the cells of
-  // level slevel whose index is k mod ksplit and writes its partial sums to part
-  int ksplit;
-  int slevel;
-  double* part;  // [2][ksplit][nt]: u then v partials (ksplit > 1)
+// a source as the pair loops read it: position, then strength and radius term (velocity) or the
+// two upstream gradients (adjoint)
+struct alignas(16) Src {
+  double x, y, a, b;
 };
 
-// makes an in-wave LDS write visible to the other lanes of the wave before they read it, and
-// keeps later writes behind earlier reads
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-struct alignas(16) LeafSrc {
+// a target: position, strength, then its radius term (velocity) or radius (adjoint). A collection
+// acting on itself reads its sources' records as its targets'.
+struct alignas(16) Trg {
   double x, y, s, w;
 };
+static_assert(sizeof(Src) == sizeof(Trg), "one array serves both");
 
-// Every lane of a wave walks the same cells. The popped stack entry is made wave-uniform
-// (readfirstlane), so cell records come in through scalar loads; a leaf's sources and a cell's
-// moments are loaded once per wave, one element per lane (coalesced), into the wave's LDS and
-// read back as broadcasts, instead of one dependent load per pair or per coefficient.
-template <int CORE>
-__global__ __launch_bounds__(kTBlock) void tree_eval_kernel(TreeArgs a, int64_t nt,
-                                                            const uint32_t* __restrict__ torder,
-                                                            const double* __restrict__ tx,
-                                                            const double* __restrict__ ty,
-                                                            const double* __restrict__ tr,
-                                                            double* __restrict__ tu,
-                                                            double* __restrict__ tv) {
-  constexpr int kWaves = kTBlock / 64;
-  __shared__ unsigned stack[kWaves][kStack];
-  __shared__ LeafSrc lsrc[kWaves][kLeaf];
-  __shared__ double2 lmom[kWaves][kMaxP];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x & 63;
-  unsigned* st = stack[wave];
-  LeafSrc* ls = lsrc[wave];
-  double2* lm = lmom[wave];
-  const int64_t i = (int64_t)blockIdx.x * kTBlock + threadIdx.x;
-  const bool valid = i < nt;
-  const uint32_t ti = valid ? torder[i] : 0u;
-  const double x = valid ? tx[ti] : 0.0, y = valid ? ty[ti] : 0.0;
-  const double wt = (valid && tr) ? rterm<CORE>(tr[ti]) : 0.0;
-  double u = 0.0, v = 0.0;     // direct part
-  double sr = 0.0, si = 0.0;   // S, the far part
-  const double th2 = a.theta * a.theta;
-  const int p = a.p;
-  // a wave with no valid lane (the tail of the grid) has nothing to do
-  if (__any(valid)) {
-    int sp = 0;
-    if (a.ksplit == 1) {
-      const int root = a.lv.n - 1;
-      if (lane == 0) st[0] = (unsigned)root << 27;  // (level << 27) | index; the root is index 0
-      sp = 1;
-    } else {
-      // cells k, k + ksplit, ... of level slevel, the smallest index on top
-      const int k = blockIdx.y;
-      const int ck = (int)((a.lv.cnt[a.slevel] - k + a.ksplit - 1) / a.ksplit);
-      if (lane < ck)
-        st[lane] = ((unsigned)a.slevel << 27) | (unsigned)(k + (ck - 1 - lane) * a.ksplit);
-      sp = ck;
+// C(n + m, m) for n, m < kMaxP, rounded once from the exact integers
+struct Binomials {
+  double v[kMaxP * kMaxP];
+};
+constexpr Binomials make_binomials() {
+  Binomials b{};
+  unsigned long long row[kMaxP] = {};
+  for (int m = 0; m < kMaxP; ++m) row[m] = 1;
+  for (int n = 0; n < kMaxP; ++n) {
+    for (int m = 0; m < kMaxP; ++m) {
+      if (n > 0 && m > 0) row[m] += row[m - 1];  // C(n+m, m) = C(n-1+m, m) + C(n+m-1, m-1)
+      b.v[n * kMaxP + m] = (double)row[m];
     }
-    wave_lds_sync();
-    while (sp > 0) {
-      const unsigned e = __builtin_amdgcn_readfirstlane(st[--sp]);
-      const int lev = (int)(e >> 27), idx = (int)(e & ((1u << 27) - 1));
-      const int64_t ci = a.lv.off[lev] + idx;
-      const Cell c = a.cell[ci];
-      const double dx = x - c.cx, dy = y - c.cy;
-      const double d2 = dx * dx + dy * dy;
-      const double dm = sqrt(d2) - c.r;  // distance to the nearest possible source of the cell
-      // every pair with this cell is beyond the core's cutoff (or within core_tol of 1/d^2)
-      const bool cfar = !valid || (dm > 0.0 && core_far<CORE>(dm * dm, c.wmax + wt, a.tol));
-      const bool acc = cfar && (!valid || c.r * c.r <= th2 * d2);
-      if (__all(acc)) {
-        if (lane < p) lm[lane] = a.mom[ci * p + lane];
-        wave_lds_sync();
-        if (valid) {
-          // t = 1/(z - c); S += sum_k M_k t^(k+1) by Horner
-          const double q = 1.0 / d2;
-          const double tre = dx * q, tim = -dy * q;
-          double hr = lm[p - 1].x, hi = lm[p - 1].y;
+  }
+  return b;
+}
+__constant__ Binomials kBinomials = make_binomials();
+
+__device__ __forceinline__ double rterm_any(int core, double r) {
+  return core == O2D_CORE_V2   ? rterm<O2D_CORE_V2>(r)
+         : core == O2D_CORE_V3 ? rterm<O2D_CORE_V3>(r)
+                               : rterm<O2D_CORE_RM>(r);
+}
+
+// LDS writes of this wave visible to its own later reads, and no compiler reordering across
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// lane l's x, in every lane
+__device__ __forceinline__ double lane_f64(double x, int l) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)b, l);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// reductions over lanes that differ in the bits below `width`
+template <int width>
+__device__ __forceinline__ double lanes_min(double v) {
+#pragma unroll
+  for (int m = width / 2; m >= 1; m >>= 1) v = fmin(v, __shfl_xor(v, m));
+  return v;
+}
+template <int width>
+__device__ __forceinline__ double lanes_max(double v) {
+#pragma unroll
+  for (int m = width / 2; m >= 1; m >>= 1) v = fmax(v, __shfl_xor(v, m));
+  return v;
+}
+
+__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
+  return make_double2(__builtin_fma(a.x, b.x, -a.y * b.y), __builtin_fma(a.x, b.y, a.y * b.x));
+}
+// f = f z + m
+__device__ __forceinline__ void horner(double2& f, double2 z, double2 m) {
+  const double fx = __builtin_fma(f.x, z.x, __builtin_fma(-f.y, z.y, m.x));
+  f.y = __builtin_fma(f.x, z.y, __builtin_fma(f.y, z.x, m.y));
+  f.x = fx;
+}
+// z^k, k < kMaxP
+__device__ __forceinline__ double2 cpow(double2 z, int k) {
+  double2 r = make_double2(1.0, 0.0);
+#pragma unroll
+  for (int b = 1; b < kMaxP; b <<= 1) {
+    const double2 t = cmul(r, z);
+    const bool set = (k & b) != 0;  // component by component: as structs they go through memory
+    r.x = set ? t.x : r.x;
+    r.y = set ? t.y : r.y;
+    if (2 * b < kMaxP) z = cmul(z, z);
+  }
+  return r;
+}
+// 1 / (x + i y)
+__device__ __forceinline__ double2 cinv(double x, double y) {
+  const double q = rcp64(__builtin_fma(x, x, y * y));
+  return make_double2(x * q, -y * q);
+}
+
+// ---------------------------------------------------------------------------- the tree
+
+// One wave per 64 sources in Morton order (kLeafs leaves): gathers their records (padding a
+// short last leaf with charges of 0 at its last source) and forms each leaf's cell, box and
+// moments. The powers of eight orders at a time pass through LDS, and each (leaf, order) sum is
+// taken by a few lanes: a wave sum per order through shuffles took 130 us for 1M sources.
+// ADJ: a is gv's and b gu's array, and radii play no part.
+template <bool ADJ>
+__global__ __launch_bounds__(kBlock) void tree_leaf_kernel(
+    int64_t ns, int64_t nleaf, int p, const uint32_t* __restrict__ order,
+    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ a,
+    const double* __restrict__ b, int core, Src* __restrict__ src, double4* __restrict__ head,
+    uint2* __restrict__ kids, double4* __restrict__ box, double2* __restrict__ mom) {
+  constexpr int kLeafs = 64 / kLeaf, kChunk = 8;
+  constexpr int kShare = 64 / (kLeafs * kChunk);  // lanes per (leaf, order)
+  static_assert(kShare >= 1 && kLeaf % kShare == 0, "whole shares");
+  __shared__ double2 buf[kWaves][kChunk][64 + 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t first = ((int64_t)blockIdx.x * kWaves + wave) * 64;
+  if (first >= nleaf * kLeaf) return;  // whole waves; no workgroup barrier below
+  const int64_t i = first + lane;
+  const bool in = i < ns;
+  const uint32_t o = order[in ? i : ns - 1];
+  Src q;
+  q.x = x[o];
+  q.y = y[o];
+  q.a = in ? a[o] : 0.0;
+  if constexpr (ADJ) q.b = in ? b[o] : 0.0;
+  else q.b = in ? rterm_any(core, b[o]) : 1.0;
+  if (i < nleaf * kLeaf) src[i] = q;
+  const double x0 = lanes_min<kLeaf>(in ? q.x : INFINITY), x1 = lanes_max<kLeaf>(in ? q.x : -INFINITY);
+  const double y0 = lanes_min<kLeaf>(in ? q.y : INFINITY), y1 = lanes_max<kLeaf>(in ? q.y : -INFINITY);
+  const double wm = ADJ ? 0.0 : lanes_max<kLeaf>(in ? q.b : 0.0);
+  const double cx = 0.5 * (x0 + x1), cy = 0.5 * (y0 + y1);
+  const double dx = q.x - cx, dy = q.y - cy;
+  // a charge that is not finite (its product with 0 is not 0) makes r infinite; an infinite radius
+  // term keeps the cell from being far by itself, and a NaN one reaches the pairs near it, as in
+  // the pair by pair sum, whose tiles beyond the largest finite term do not look at it
+  const bool odd = in && !(q.a * 0.0 + (ADJ ? q.b * 0.0 : 0.0) == 0.0);
+  const double r2 = lanes_max<kLeaf>(odd ? INFINITY : (in ? dx * dx + dy * dy : 0.0));
+  // rounding of the offsets: a relative margin keeps r an upper bound
+  const double r = sqrt(r2) * (1.0 + 1e-12);
+  const double inv = r > 0.0 ? 1.0 / r : 0.0;
+  const double2 d = make_double2(dx * inv, dy * inv);
+  double2 pw = ADJ ? make_double2(q.a, -q.b) : make_double2(q.a, 0.0);
+  if (!in) pw = make_double2(0.0, 0.0);
+  const int64_t leaf = first / kLeaf + lane / kLeaf;
+  if ((lane & (kLeaf - 1)) == 0 && leaf < nleaf) {
+    head[leaf] = make_double4(cx, cy, r, wm);
+    kids[leaf] = make_uint2((uint32_t)leaf, 0);
+    box[leaf] = make_double4(x0, y0, x1, y1);
+  }
+  // lane = ((share * kLeafs) + lf) * kChunk + k
+  const int k = lane % kChunk, lf = (lane / kChunk) % kLeafs, share = lane / (kChunk * kLeafs);
+  for (int k0 = 0; k0 < kMaxP; k0 += kChunk) {
+#pragma unroll
+    for (int e = 0; e < kChunk; ++e) {
+      buf[wave][e][lane] = pw;
+      pw = cmul(pw, d);
+    }
+    wave_sync();
+    double2 m = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int j = 0; j < kLeaf / kShare; ++j) {
+      const double2 t = buf[wave][k][lf * kLeaf + share * (kLeaf / kShare) + j];
+      m.x += t.x;
+      m.y += t.y;
+    }
+#pragma unroll
+    for (int s = kChunk * kLeafs; s < 64; s <<= 1) {
+      m.x += __shfl_xor(m.x, s);
+      m.y += __shfl_xor(m.y, s);
+    }
+    const int64_t c = first / kLeaf + lf;
+    if (share == 0 && c < nleaf)
+      mom[c * kMaxP + k0 + k] = k0 + k < p ? m : make_double2(0.0, 0.0);
+    wave_sync();
+  }
+}
+
+// One cell from its children (global cells child0 .. child0 + nch - 1), by one wave: the union of
+// the boxes, a covering radius (of the children's circles or of the box, whichever is smaller),
+// and the moments, M'_k = sum_children sum_{l <= k} C(k, l) (r_c / r)^l M_l ((c_c - c) / r)^(k - l).
+// Half-waves take a child each, lane k its order k; sa, sd: the wave's 2 x kMaxP scratch entries.
+__device__ __forceinline__ void tree_parent(uint32_t self, uint32_t child0, int nch, int p,
+                                            const double* __restrict__ binom, double2* sa,
+                                            double2* sd, double4* head, uint2* kids,
+                                            double4* box, double2* mom) {
+  const int lane = threadIdx.x & 63, k = lane & (kMaxP - 1), h = lane / kMaxP;
+  double4 b = box[child0];
+  double wm = head[child0].w;
+  for (int c = 1; c < nch; ++c) {
+    const double4 e = box[child0 + c];
+    b.x = fmin(b.x, e.x);
+    b.y = fmin(b.y, e.y);
+    b.z = fmax(b.z, e.z);
+    b.w = fmax(b.w, e.w);
+    wm = fmax(wm, head[child0 + c].w);
+  }
+  const double cx = 0.5 * (b.x + b.z), cy = 0.5 * (b.y + b.w);
+  double r = 0.0;
+  bool odd = false;
+  for (int c = 0; c < nch; ++c) {
+    const double4 q = head[child0 + c];
+    const double dx = q.x - cx, dy = q.y - cy;
+    r = fmax(r, sqrt(dx * dx + dy * dy) + q.z);
+    odd = odd || !(q.z < INFINITY);
+  }
+  const double ex = b.z - cx, ey = b.w - cy;
+  r = odd ? INFINITY : fmin(r, sqrt(ex * ex + ey * ey)) * (1.0 + 1e-12);
+  const double inv = r > 0.0 ? 1.0 / r : 0.0;
+  double2 acc = make_double2(0.0, 0.0);
+  for (int c0 = 0; c0 < kFan; c0 += 2) {
+    const int c = c0 + h;
+    double2 a = make_double2(0.0, 0.0), d = a;
+    if (c < nch) {
+      const double4 q = head[child0 + c];
+      const double2 m = mom[(int64_t)(child0 + c) * kMaxP + k];
+      const double ratio = cpow(make_double2(q.z * inv, 0.0), k).x;
+      a = make_double2(m.x * ratio, m.y * ratio);
+      d = cpow(make_double2((q.x - cx) * inv, (q.y - cy) * inv), k);
+    }
+    wave_sync();
+    sa[lane] = a;
+    sd[lane] = d;
+    wave_sync();
 #pragma unroll 4
-          for (int k = p - 2; k >= 0; --k) {
-            const double2 mk = lm[k];
-            const double nr = hr * tre - hi * tim + mk.x;
-            hi = hr * tim + hi * tre + mk.y;
-            hr = nr;
-          }
-          sr += hr * tre - hi * tim;
-          si += hr * tim + hi * tre;
-        }
-        wave_lds_sync();
-      } else if (lev == 0) {
-        const int64_t j0 = (int64_t)idx * kLeaf;
-        const int nj = (int)((j0 + kLeaf < a.ns) ? kLeaf : a.ns - j0);
-        if (lane < nj) {
-          const int64_t j = j0 + lane;
-          ls[lane] = LeafSrc{a.sx[j], a.sy[j], a.ss[j], a.sw[j]};
-        }
-        wave_lds_sync();
-        if (CORE == O2D_CORE_GAUSSIAN && __all(cfar)) {
-          // the whole leaf is beyond the compact cutoff for every lane: K = 1/d^2
-          if (valid) {
-#pragma unroll 8
-            for (int k = 0; k < nj; ++k) {
-              const LeafSrc q = ls[k];
-              const double ex = x - q.x, ey = y - q.y;
-              const double g = q.s * rcp64(__builtin_fma(ex, ex, ey * ey));
-              u = __builtin_fma(-g, ey, u);
-              v = __builtin_fma(g, ex, v);
-            }
-          }
-        } else if (valid) {
-#pragma unroll 4
-          for (int k = 0; k < nj; ++k) {
-            const LeafSrc q = ls[k];
-            const double ex = x - q.x, ey = y - q.y;
-            const double e2 = __builtin_fma(ex, ex, ey * ey);
-            const double g = q.s * core_k64<CORE>(ex, ey, e2, wsum(q.w, wt));
-            u = __builtin_fma(-g, ey, u);
-            v = __builtin_fma(g, ex, v);
-          }
-        }
-        wave_lds_sync();
-      } else {
-        const int64_t first = (int64_t)idx * kFan;
-        const int64_t cnt = a.lv.cnt[lev - 1];
-        // lane k writes child kFan-1-k, so the first child ends on top of the stack
-        int nc = 0;
-        for (int k = 0; k < kFan; ++k) nc += (first + k < cnt) ? 1 : 0;
-        if (lane < nc)
-          st[sp + lane] = ((unsigned)(lev - 1) << 27) | (unsigned)(first + nc - 1 - lane);
-        sp += nc;
-        wave_lds_sync();
+    for (int l = 0; l < kMaxP; ++l) {
+      if (l <= k) {
+        const double2 al = sa[h * kMaxP + l], dl = sd[h * kMaxP + k - l];
+        const double bn = binom[l * kMaxP + k - l];
+        const double2 t = make_double2(al.x * bn, al.y * bn);
+        acc.x = __builtin_fma(t.x, dl.x, __builtin_fma(-t.y, dl.y, acc.x));
+        acc.y = __builtin_fma(t.x, dl.y, __builtin_fma(t.y, dl.x, acc.y));
       }
     }
   }
-  if (valid) {
-    if (a.ksplit == 1) {
-      tu[ti] += u + si;
-      tv[ti] += v + sr;
-    } else {
-      a.part[(int64_t)blockIdx.y * nt + ti] = u + si;
-      a.part[(int64_t)(a.ksplit + blockIdx.y) * nt + ti] = v + sr;
+  acc.x += __shfl_xor(acc.x, kMaxP);
+  acc.y += __shfl_xor(acc.y, kMaxP);
+  if (h == 0) mom[(int64_t)self * kMaxP + k] = k < p ? acc : make_double2(0.0, 0.0);
+  if (lane == 0) {
+    head[self] = make_double4(cx, cy, r, wm);
+    kids[self] = make_uint2(child0, (uint32_t)nch);
+    box[self] = b;
+  }
+}
+
+// Two coarser levels per launch: a workgroup's four waves form four cells of level l + 1, then
+// its first wave their parent of level l + 2 (when there is one: cnt2 > 0)
+__global__ __launch_bounds__(kBlock) void tree_up_kernel(uint32_t off0, uint32_t cnt0, uint32_t off1,
+                                                         uint32_t cnt1, uint32_t off2,
+                                                         uint32_t cnt2, int p, double4* head,
+                                                         uint2* kids, double4* box,
+                                                         double2* mom) {
+  __shared__ double binom[kMaxP * kMaxP];
+  __shared__ double2 sa[kWaves][64], sd[kWaves][64];
+  static_assert(kWaves == kFan, "a workgroup forms the children of one cell");
+  const int wave = threadIdx.x >> 6;
+  for (int e = threadIdx.x; e < kMaxP * kMaxP; e += kBlock) binom[e] = kBinomials.v[e];
+  __syncthreads();
+  const uint32_t c1 = blockIdx.x * kFan + wave;
+  if (c1 < cnt1) {
+    const uint32_t k0 = c1 * kFan;
+    const int nch = (int)(k0 + kFan < cnt0 ? kFan : cnt0 - k0);
+    tree_parent(off1 + c1, off0 + k0, nch, p, binom, sa[wave], sd[wave], head, kids, box,
+                mom);
+  }
+  if (cnt2 == 0) return;  // uniform
+  __threadfence_block();
+  __syncthreads();
+  if (wave != 0) return;
+  const uint32_t k0 = blockIdx.x * kFan;
+  const int nch = (int)(k0 + kFan < cnt1 ? kFan : cnt1 - k0);
+  tree_parent(off2 + blockIdx.x, off1 + k0, nch, p, binom, sa[0], sd[0], head, kids, box, mom);
+}
+
+// the targets in Morton order
+template <bool ADJ>
+__global__ __launch_bounds__(kBlock) void tree_targets_kernel(int64_t n, const uint32_t* __restrict__ order,
+                                                              const double* __restrict__ x,
+                                                              const double* __restrict__ y,
+                                                              const double* __restrict__ r,
+                                                              const double* __restrict__ s,
+                                                              int core, Trg* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t o = order[i];
+  Trg t;
+  t.x = x[o];
+  t.y = y[o];
+  if constexpr (ADJ) {
+    t.w = r[o];
+    t.s = s[o];
+  } else {
+    t.w = r ? rterm_any(core, r[o]) : 0.0;
+    t.s = 0.0;
+  }
+  out[i] = t;
+}
+
+// ---------------------------------------------------------------------------- far tests
+
+// the pair distance from which the core equals 1/d^2 to within tol (exactly for the Gaussian) for
+// radius terms up to w, with a margin far above the rounding of the tests that use it
+template <int CORE>
+__device__ __forceinline__ double core_reach(double w, double tol) {
+  if constexpr (CORE == O2D_CORE_GAUSSIAN) {
+    return 4.0 * sqrt(w) * (1.0 + 1e-12);
+  } else if constexpr (CORE == O2D_CORE_RM) {
+    return sqrt(w / tol) * (1.0 + 1e-12);
+  } else if constexpr (CORE == O2D_CORE_WL) {
+    return sqrt(w / sqrt(tol)) * (1.0 + 1e-12);
+  } else if constexpr (CORE == O2D_CORE_V2) {
+    return sqrt(sqrt(w / (2.0 * tol))) * (1.0 + 1e-12);
+  } else {
+    return cbrt(sqrt(w / (3.0 * tol))) * (1.0 + 1e-12);
+  }
+}
+
+// a radius as the largest radius term of the pairs' targets: the adjoint's targets carry radii
+template <int CORE, bool ADJ>
+__device__ __forceinline__ double target_term(const Trg& t) {
+  return ADJ ? rterm<CORE>(t.w) : t.w;
+}
+
+// ---------------------------------------------------------------------------- super groups
+
+struct Super {
+  double cx, cy, r;  // the local expansion's centre and the radius that scales it
+  int64_t nfront;    // frontier cells, or -1: the groups start from the root, without the expansion
+};
+
+// One workgroup per kSuper targets. Cells of a round are tested by one thread each; accepted
+// ones are dealt to the waves, whose local expansions are added in wave order at the end, so
+// nothing depends on scheduling. A wave takes a cell's moments into lanes 0..kMaxP-1, a_k =
+// M_k (r / D)^k with D = c_T - c, and its lanes form sum_k C(k + l, l) a_k, half of the k each;
+// the upper half-wave scales by (-R / D)^l / D and keeps the sums.
+template <int CORE, bool ADJ>
+__global__ __launch_bounds__(kSuperBlock) void tree_super_kernel(
+    int64_t nt, const Trg* __restrict__ trg, const double4* __restrict__ head,
+    const uint2* __restrict__ kids, const double2* __restrict__ mom, uint32_t root, double theta, double tol,
+    Super* __restrict__ super, double2* __restrict__ local, uint32_t* __restrict__ front) {
+  __shared__ double binom[kMaxP * kMaxP];
+  __shared__ uint32_t queue[2][kQueue], taken[kSuperBlock];
+  __shared__ int counts[kSuperWaves][3];
+  __shared__ double2 am[kSuperWaves][kMaxP];
+  __shared__ double2 sums[kSuperWaves][kMaxP];
+  __shared__ double red[kSuperWaves][5];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int k = lane & (kMaxP - 1), h = lane / kMaxP;
+  for (int e = t; e < kMaxP * kMaxP; e += kSuperBlock) binom[e] = kBinomials.v[e];
+  // the targets' box, its centre and the radius that covers them (NaN positions are left out:
+  // those targets' sums are NaN whatever is done with the cells)
+  const int64_t t0 = (int64_t)blockIdx.x * kSuper;
+  double x0 = INFINITY, x1 = -INFINITY, y0 = INFINITY, y1 = -INFINITY, wt = 0.0;
+  double px[kSuper / kSuperBlock], py[kSuper / kSuperBlock];
+  bool odd = false;
+#pragma unroll
+  for (int e = 0; e < kSuper / kSuperBlock; ++e) {
+    const int64_t i = t0 + e * kSuperBlock + t;
+    const Trg q = trg[i < nt ? i : nt - 1];
+    const double w = target_term<CORE, ADJ>(q);
+    px[e] = q.x;
+    py[e] = q.y;
+    x0 = fmin(x0, q.x);
+    x1 = fmax(x1, q.x);
+    y0 = fmin(y0, q.y);
+    y1 = fmax(y1, q.y);
+    wt = fmax(wt, w);
+    odd = odd || !(w < INFINITY);
+  }
+  if (odd) wt = INFINITY;  // nothing is far from a target whose radius is not finite
+  x0 = lanes_min<64>(x0);
+  x1 = lanes_max<64>(x1);
+  y0 = lanes_min<64>(y0);
+  y1 = lanes_max<64>(y1);
+  wt = lanes_max<64>(wt);
+  if (lane == 0) {
+    red[wave][0] = x0;
+    red[wave][1] = x1;
+    red[wave][2] = y0;
+    red[wave][3] = y1;
+    red[wave][4] = wt;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kSuperWaves; ++w) {
+    x0 = fmin(x0, red[w][0]);
+    x1 = fmax(x1, red[w][1]);
+    y0 = fmin(y0, red[w][2]);
+    y1 = fmax(y1, red[w][3]);
+    wt = fmax(wt, red[w][4]);
+  }
+  const double cx = 0.5 * (x0 + x1), cy = 0.5 * (y0 + y1);
+  double r2 = 0.0;
+#pragma unroll
+  for (int e = 0; e < kSuper / kSuperBlock; ++e) {
+    const double dx = px[e] - cx, dy = py[e] - cy;
+    r2 = fmax(r2, dx * dx + dy * dy);
+  }
+  r2 = lanes_max<64>(r2);
+  __syncthreads();
+  if (lane == 0) red[wave][0] = r2;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kSuperWaves; ++w) r2 = fmax(r2, red[w][0]);
+  const double R = sqrt(r2) * (1.0 + 1e-12);
+
+  uint32_t* fr = front + (int64_t)blockIdx.x * kFront;
+  int nf = 0, nq = 1, cur = 0;
+  bool over = !(R < INFINITY);  // a target at infinity must not reach the others
+  if (t == 0) queue[0][0] = root;
+  double2 acc = make_double2(0.0, 0.0);  // lane kMaxP + l: L_l
+  __syncthreads();
+  while (nq > 0 && !over) {
+    int nnext = 0;
+    for (int base = 0; base < nq && !over; base += kSuperBlock) {
+      const bool live = base + t < nq;
+      const uint32_t ci = live ? queue[cur][base + t] : root;
+      const double4 c = head[ci];
+      const uint2 kd = kids[ci];
+      const double dx = cx - c.x, dy = cy - c.y;
+      const double d = sqrt(dx * dx + dy * dy);
+      const double near = d - R;  // the nearest a target can be to the cell's centre
+      const bool far = live && near > c.z + core_reach<CORE>(c.w + wt, tol) &&
+                       c.z <= theta * near && R <= theta * (d - c.z);
+      const bool keep = live && !far && (kd.y == 0 || c.z <= 0.5 * R);
+      const int nc = live && !far && !keep ? (int)kd.y : 0;
+      // places in the three lists: ballots within the wave, the waves' counts before it
+      const unsigned long long below = (1ull << lane) - 1ull;
+      const unsigned long long mf = __ballot(far), mk = __ballot(keep);
+      const unsigned long long b0 = __ballot(nc & 1), b1 = __ballot(nc & 2), b2 = __ballot(nc & 4);
+      int pf = __popcll(mf & below), pk = __popcll(mk & below);
+      int pc = __popcll(b0 & below) + 2 * __popcll(b1 & below) + 4 * __popcll(b2 & below);
+      if (lane == 0) {
+        counts[wave][0] = __popcll(mf);
+        counts[wave][1] = __popcll(mk);
+        counts[wave][2] = __popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2);
+      }
+      __syncthreads();
+      int nfar = 0, nkeep = 0, nchild = 0;
+#pragma unroll
+      for (int w = 0; w < kSuperWaves; ++w) {
+        pf += w < wave ? counts[w][0] : 0;
+        pk += w < wave ? counts[w][1] : 0;
+        pc += w < wave ? counts[w][2] : 0;
+        nfar += counts[w][0];
+        nkeep += counts[w][1];
+        nchild += counts[w][2];
+      }
+      if (nf + nkeep > kFront || nnext + nchild > kQueue) {
+        over = true;  // uniform
+      } else {
+        if (far) taken[pf] = ci;
+        if (keep) fr[nf + pk] = ci;
+        for (int e = 0; e < nc; ++e) queue[cur ^ 1][nnext + pc + e] = kd.x + e;
+      }
+      nf += nkeep;
+      nnext += nchild;
+      __syncthreads();
+      if (over) break;
+      // the accepted cells, dealt to the waves; the next one's record and moments are on their
+      // way while one is shifted
+      int j = wave;
+      double4 nxt = make_double4(0.0, 0.0, 0.0, 0.0);
+      double2 nm = make_double2(0.0, 0.0);
+      if (j < nfar) {
+        const uint32_t cj = taken[j];
+        nxt = head[cj];
+        nm = mom[(int64_t)cj * kMaxP + k];
+      }
+      while (j < nfar) {
+        const double4 q = nxt;
+        const double2 m = nm;
+        j += kSuperWaves;
+        if (j < nfar) {
+          const uint32_t cj = taken[j];
+          nxt = head[cj];
+          nm = mom[(int64_t)cj * kMaxP + k];
+        }
+        const double2 id = cinv(cx - q.x, cy - q.y);  // 1 / D
+        const double sc = h == 0 ? q.z : -R;
+        const double2 pw = cpow(make_double2(sc * id.x, sc * id.y), k);
+        const double2 a = cmul(m, pw);
+        wave_sync();
+        if (h == 0) am[wave][k] = a;
+        wave_sync();
+        double2 s = make_double2(0.0, 0.0);
+#pragma unroll 8
+        for (int e = 0; e < kMaxP / 2; ++e) {
+          const int kk = h * (kMaxP / 2) + e;
+          const double bn = binom[kk * kMaxP + k];
+          const double2 ak = am[wave][kk];
+          s.x = __builtin_fma(bn, ak.x, s.x);
+          s.y = __builtin_fma(bn, ak.y, s.y);
+        }
+        s.x += __shfl_xor(s.x, kMaxP);
+        s.y += __shfl_xor(s.y, kMaxP);
+        const double2 f = cmul(cmul(pw, id), s);
+        acc.x += f.x;
+        acc.y += f.y;
+      }
+      __syncthreads();
+    }
+    cur ^= 1;
+    nq = nnext;
+  }
+  if (h == 1) sums[wave][k] = acc;
+  __syncthreads();
+  if (t < kMaxP) {
+    double2 s = sums[0][t];
+    for (int w = 1; w < kSuperWaves; ++w) {
+      s.x += sums[w][t].x;
+      s.y += sums[w][t].y;
+    }
+    local[(int64_t)blockIdx.x * kMaxP + t] = s;
+  }
+  if (t == 0) super[blockIdx.x] = Super{cx, cy, R, over ? -1 : nf};
+}
+
+// ---------------------------------------------------------------------------- groups
+
+struct GroupArgs {
+  int64_t nt;
+  int g;           // targets per wave
+  int p;           // moments used, and terms of the local expansion
+  int ksplit;      // waves per group: wave k takes every ksplit-th far cell and leaf
+  uint32_t start;  // starting cells when there are no super groups (or one gave up): start ..
+  uint32_t nstart; // start + nstart - 1, all of one level
+  double theta, tol;
+};
+
+// One wave per G targets and share (blockIdx.y) of their far cells and leaves; every share opens
+// the same cells. The wave's 64 / G slices
+// hold the same targets and take different cells and leaves; their sums are added in slice order.
+// ou..: the outputs in the targets' input order, or (part != null) partial sums by position,
+// [component][ksplit][nt].
+template <int CORE, bool ADJ, int G>
+__global__ __launch_bounds__(kGroupBlock, 4) void tree_group_kernel(
+    GroupArgs a, const Trg* __restrict__ trg, const uint32_t* __restrict__ torder,
+    const double4* __restrict__ head, const uint2* __restrict__ kids,
+    const double2* __restrict__ mom, const Src* __restrict__ src,
+    const Super* __restrict__ super, const double2* __restrict__ local,
+    const uint32_t* __restrict__ front, double* __restrict__ o0, double* __restrict__ o1,
+    double* __restrict__ o2, double* __restrict__ o3, double* __restrict__ part) {
+  constexpr int kSlices = 64 / G;
+  constexpr int kItem = 2 * kLeaf;  // double2 elements of a leaf's records
+  static_assert(kMaxP <= kItem && kItem % G == 0 && kMaxP % (G < kMaxP ? G : kMaxP) == 0,
+                "whole loads per slice");
+  __shared__ uint32_t stacks[kGroupWaves][kStack];
+  // per slice the moments or the sources being worked on (rows apart by other than a multiple of
+  // the banks, so that the slices' reads do not meet)
+  __shared__ double2 buffers[kGroupWaves][kSlices][kItem + (kSlices > 1 ? 1 : 0)];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int slice = lane / G, mine = lane % G;
+  const int64_t group = (int64_t)blockIdx.x * kGroupWaves + wave;
+  if (group * G >= a.nt) return;  // whole waves; no workgroup barrier below
+  uint32_t* st = stacks[wave];
+  double2* data = buffers[wave][slice];
+  const int64_t i = group * G + mine;
+  const Trg tg = trg[i < a.nt ? i : a.nt - 1];
+  const double x = tg.x, y = tg.y;
+  const double wmine = target_term<CORE, ADJ>(tg);
+  const double x0 = lanes_min<G>(x), x1 = lanes_max<G>(x);
+  const double y0 = lanes_min<G>(y), y1 = lanes_max<G>(y);
+  const double wt = __any(!(wmine < INFINITY)) ? INFINITY : lanes_max<G>(wmine);
+  const double itheta = 1.0 / (kThetaShare * a.theta);
+  const int p = a.p;
+  const float logtail = 2.0f * (float)p * __builtin_amdgcn_logf((float)(0.9 * a.theta));
+  // pairs: velocity u, v; adjoint dJ/ds, dJ/dx, dJ/dy, dJ/dr (the last three over the strength)
+  double n0 = 0.0, n1 = 0.0, n2 = 0.0, n3 = 0.0;
+  double2 S = make_double2(0.0, 0.0), S2 = S;  // far cells: S, and for the adjoint S2
+
+  const uint32_t* init = nullptr;
+  int64_t ninit = a.nstart;
+  if (super) {
+    const int64_t sg = group * G / kSuper;
+    const Super sp = super[sg];
+    if (sp.nfront >= 0) {
+      init = front + sg * kFront;
+      ninit = sp.nfront;
+      if (blockIdx.y == 0) {  // the super group's local expansion at this target (slice 0's sums)
+        double2* L = buffers[wave][0];
+        if (lane < kMaxP) L[lane] = local[sg * kMaxP + lane];
+        wave_sync();
+        const double ir = sp.r > 0.0 ? 1.0 / sp.r : 0.0;
+        const double2 z = make_double2((x - sp.cx) * ir, (y - sp.cy) * ir);
+        double2 f = L[p - 1], g = make_double2(0.0, 0.0);
+#pragma unroll 4
+        for (int l = p - 2; l >= 0; --l) {
+          if constexpr (ADJ) horner(g, z, f);
+          horner(f, z, L[l]);
+        }
+        if (slice != 0) f = g = make_double2(0.0, 0.0);
+        S = f;
+        if constexpr (ADJ) S2 = make_double2(-g.x * ir, -g.y * ir);  // -dS/dz
+      }
+    }
+  }
+  // the next set bit of `bits` for every slice: this lane's in `from` (-1 when there is none
+  // left), the lowest bits to the lowest slices
+  auto deal = [&](unsigned long long& bits, int& from) {
+    from = -1;
+#pragma unroll
+    for (int q = 0; q < kSlices; ++q) {
+      const int b = bits ? __builtin_ctzll(bits) : -1;
+      bits = bits ? bits & (bits - 1) : bits;
+      from = slice == q ? b : from;
+    }
+  };
+  // lane l's value (l the same in every lane of the wave when there is one slice)
+  auto lane_of = [&](double v, int l) {
+    if constexpr (kSlices == 1) return lane_f64(v, l);
+    else return __shfl(v, l < 0 ? 0 : l, 64);
+  };
+  auto int_of = [&](int v, int l) {
+    if constexpr (kSlices == 1) return __builtin_amdgcn_readlane(v, l);
+    else return __shfl(v, l < 0 ? 0 : l, 64);
+  };
+  int sp = 0;
+  int64_t next = 0;  // the next starting cell
+  // this share's far cells and leaves: every ksplit-th of each kind
+  unsigned nfar = 0, nleaf = 0;
+  auto share = [&](unsigned long long bits, unsigned& seen) {
+    if (a.ksplit == 1) return bits;
+    const unsigned at = seen + __popcll(bits & ((1ull << lane) - 1ull));
+    seen += __popcll(bits);
+    return bits & __ballot(at % (unsigned)a.ksplit == blockIdx.y);
+  };
+  for (;;) {
+    if (sp < 64 && next < ninit) {
+      const int64_t at = next + lane;
+      if (at < ninit) st[sp + lane] = init ? init[at] : a.start + (uint32_t)at;
+      sp += ninit - next < 64 ? (int)(ninit - next) : 64;
+      next += 64;
+      wave_sync();
+    }
+    if (sp == 0) break;
+    // as many of the top cells as the stack has room to open
+    int m = (kStack - kStackSpare - sp) / 3;
+    m = m < 1 ? 1 : (m < 64 ? m : 64);
+    m = m < sp ? m : sp;
+    sp -= m;
+    const bool live = lane < m;
+    const uint32_t ci = st[sp + (live ? lane : 0)];
+    const double4 c = head[ci];
+    const uint2 kd = kids[ci];
+    const uint32_t first = kd.x, nkids = kd.y;
+    // squared distances to the centre from which the core is 1/d^2 for every pair, and from which
+    // the cell is far
+    const double reach = c.z + core_reach<CORE>(c.w + wt, a.tol), open = c.z * itheta;
+    const double rcore = reach * reach, rfar = fmax(rcore, open * open);
+    // the box's squared distance, a little low so that no target is nearer
+    const double bx = fmax(fmax(x0 - c.x, c.x - x1), 0.0);
+    const double by = fmax(fmax(y0 - c.y, c.y - y1), 0.0);
+    const double b2d = (bx * bx + by * by) * (1.0 - 1e-12);
+    unsigned long long fbits = __ballot(live && b2d >= rfar);
+    unsigned long long cbits = CORE == O2D_CORE_GAUSSIAN ? __ballot(live && b2d >= rcore) : 0ull;
+    // cells too near the box may still be far from every target (a box that spans a jump of the
+    // curve is mostly empty): target by target
+    for (unsigned long long bits = __ballot(live) & ~fbits; bits;) {
+      int from;
+      deal(bits, from);
+      const double ex = x - lane_of(c.x, from), ey = y - lane_of(c.y, from);
+      const double e2 = __builtin_fma(ex, ex, ey * ey) * (1.0 - 1e-12);
+      const double tfar = lane_of(rfar, from), tcore = lane_of(rcore, from);  // by every lane
+      const unsigned long long mf = __ballot(from >= 0 && e2 >= tfar);
+      const unsigned long long mc =
+          CORE == O2D_CORE_GAUSSIAN ? __ballot(from >= 0 && e2 >= tcore) : 0ull;
+      constexpr unsigned long long kAll = G == 64 ? ~0ull : (1ull << (G & 63)) - 1ull;
+#pragma unroll
+      for (int q = 0; q < kSlices; ++q) {
+        const int f = __builtin_amdgcn_readlane(from, q * G);
+        if (((mf >> (q * G)) & kAll) == kAll) fbits |= 1ull << f;
+        if (((mc >> (q * G)) & kAll) == kAll) cbits |= 1ull << f;
+      }
+    }
+    const bool far = (fbits >> lane) & 1ull;
+    // orders that this cell needs at its distance: (r / d)^terms <= (0.9 theta)^p, so that cells
+    // nearer the limit keep all p and the others stay well below its truncation
+    int terms = p;
+    if (far && b2d >= rfar) {
+      const float ratio = __builtin_amdgcn_logf((float)(c.z * c.z) / (float)b2d);
+      const float need = __builtin_ceilf(logtail / ratio);
+      terms = need < (float)p ? (need > 2.0f ? (int)need : 2) : p;
+      terms = terms < p ? terms : p;
+    }
+    const bool leaf = live && !far && nkids == 0;
+    const int nc = live && !far && !leaf ? (int)nkids : 0;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const unsigned long long b0 = __ballot(nc & 1), b1 = __ballot(nc & 2), b2 = __ballot(nc & 4);
+    const int pc = __popcll(b0 & below) + 2 * __popcll(b1 & below) + 4 * __popcll(b2 & below);
+    wave_sync();  // the popped entries have been read
+    for (int e = 0; e < nc; ++e) st[sp + pc + e] = first + e;
+    sp += __popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2);
+    wave_sync();
+
+    // The batch's far cells, then its leaves beyond the core, then the others, one a slice at a
+    // time. Moments and records are loaded, an element per lane and load, while those before are
+    // worked on, and go through LDS, which the slice's lanes read as broadcasts (as scalar loads
+    // they arrive a few at a time: 18 ms, against 10, before the cells were tested by target)
+    const uint32_t item = far ? ci : first;  // the cell, or the leaf
+    const unsigned long long lbits = share(__ballot(leaf), nleaf);
+    const unsigned long long mine_far = share(fbits, nfar);
+    constexpr int kMomLoads = kMaxP > G ? kMaxP / G : 1, kLeafLoads = kItem / G;
+    double2 nxt[kLeafLoads];
+    auto load_mom = [&](int from) {
+      const uint32_t id = __shfl(item, from < 0 ? 0 : from, 64);
+      const double2* m = mom + (int64_t)id * kMaxP;
+      if (from >= 0) {
+#pragma unroll
+        for (int e = 0; e < kMomLoads; ++e) nxt[e] = m[(e * G + mine) & (kMaxP - 1)];
+      }
+    };
+    auto load_leaf = [&](int from) {
+      const uint32_t id = __shfl(item, from < 0 ? 0 : from, 64);
+      const double2* m = reinterpret_cast<const double2*>(src) + (int64_t)id * kItem;
+      if (from >= 0) {
+#pragma unroll
+        for (int e = 0; e < kLeafLoads; ++e) nxt[e] = m[e * G + mine];
+      }
+    };
+    {
+      unsigned long long bits = mine_far;
+      int from = -1, then = -1;
+      if (bits) {
+        deal(bits, then);
+        load_mom(then);
+      }
+      for (bool more = mine_far != 0ull; more;) {
+        from = then;
+        wave_sync();  // the cells before have been read
+#pragma unroll
+        for (int e = 0; e < kMomLoads; ++e)
+          if (e * G + mine < kMaxP) data[e * G + mine] = nxt[e];
+        more = bits != 0ull;
+        if (more) {
+          deal(bits, then);
+          load_mom(then);
+        }
+        wave_sync();
+        // through its moments: t = r / (z - c), S += sum_k M_k t^k / (z - c)
+        const double qr = lane_of(c.z, from), qx = lane_of(c.x, from), qy = lane_of(c.y, from);
+        const int np = int_of(terms, from);
+        if (from >= 0) {
+          const double2 id = cinv(x - qx, y - qy);
+          const double2 z = make_double2(qr * id.x, qr * id.y);
+          double2 f = data[np - 1], g = make_double2(0.0, 0.0);
+#pragma unroll 4
+          for (int k = np - 2; k >= 0; --k) {
+            if constexpr (ADJ) horner(g, z, f);
+            horner(f, z, data[k]);
+          }
+          const double2 s1 = cmul(f, id);
+          S.x += s1.x;
+          S.y += s1.y;
+          if constexpr (ADJ) {  // S2 = (f + t f') / (z - c)^2
+            const double2 fz = cmul(g, z);
+            const double2 s2 = cmul(make_double2(f.x + fz.x, f.y + fz.y), cmul(id, id));
+            S2.x += s2.x;
+            S2.y += s2.y;
+          }
+        }
+      }
+    }
+    // leaves pair by pair: first those beyond the Gaussian's cutoff for every pair, without the
+    // test per pair
+    auto leaves = [&](unsigned long long bits, auto inner) {
+      int from = -1, then = -1;
+      if (!bits) return;
+      deal(bits, then);
+      load_leaf(then);
+      for (bool more = true; more;) {
+        from = then;
+        wave_sync();
+#pragma unroll
+        for (int e = 0; e < kLeafLoads; ++e) data[e * G + mine] = nxt[e];
+        more = bits != 0ull;
+        if (more) {
+          deal(bits, then);
+          load_leaf(then);
+        }
+        wave_sync();
+        if (from >= 0) inner(reinterpret_cast<const Src*>(data));
+      }
+    };
+    if constexpr (CORE == O2D_CORE_GAUSSIAN) {
+      leaves(lbits & cbits, [&](const Src* ls) {
+#pragma unroll 8
+        for (int k = 0; k < kLeaf; ++k) {
+          const Src q = ls[k];
+          if constexpr (ADJ) {
+            const double dx = q.x - x, dy = q.y - y;
+            const double kk = rcp64(__builtin_fma(dx, dx, dy * dy));
+            const double tr = dx * kk, ti = -dy * kk;
+            n0 = __builtin_fma(q.a, tr, __builtin_fma(q.b, ti, n0));
+            const double sr2 = __builtin_fma(tr, tr, -ti * ti), si2 = 2.0 * tr * ti;
+            n1 = __builtin_fma(q.a, sr2, __builtin_fma(q.b, si2, n1));
+            n2 = __builtin_fma(q.b, sr2, __builtin_fma(-q.a, si2, n2));
+          } else {
+            const double ex = x - q.x, ey = y - q.y;
+            const double g = q.a * rcp64(__builtin_fma(ex, ex, ey * ey));
+            n0 = __builtin_fma(-g, ey, n0);
+            n1 = __builtin_fma(g, ex, n1);
+          }
+        }
+      });
+    }
+    leaves(lbits & ~cbits, [&](const Src* ls) {
+#pragma unroll 4
+      for (int k = 0; k < kLeaf; ++k) {
+        const Src q = ls[k];
+        if constexpr (ADJ) {
+          const double dx = q.x - x, dy = q.y - y;
+          const double d2 = __builtin_fma(dx, dx, dy * dy);
+          double kk, bbb, dks;
+          core_adj64<CORE>(dx, dy, d2, tg.w, kk, bbb, dks);
+          const double w = __builtin_fma(q.a, dx, -q.b * dy);
+          n0 = __builtin_fma(kk, w, n0);
+          n3 = __builtin_fma(dks, w, n3);
+          const double bxy = bbb * dx * dy;
+          n1 += __builtin_fma(q.b, bxy, -q.a * __builtin_fma(bbb, dx * dx, kk));
+          n2 += __builtin_fma(q.b, __builtin_fma(bbb, dy * dy, kk), -q.a * bxy);
+        } else {
+          const double ex = x - q.x, ey = y - q.y;
+          const double e2 = __builtin_fma(ex, ex, ey * ey);
+          const double w = wsum(q.b, tg.w);
+          double k0;
+          if constexpr (CORE == O2D_CORE_GAUSSIAN)  // near leaves hold most of the pairs inside cores
+            k0 = e2 > kGaussFar * (1.0 + kCutMargin) * w ? rcp64(e2) : gauss_inside64(ex, ey, e2, w);
+          else
+            k0 = core_k64<CORE>(ex, ey, e2, w);
+          const double g = q.a * k0;
+          n0 = __builtin_fma(-g, ey, n0);
+          n1 = __builtin_fma(g, ex, n1);
+        }
+      }
+    });
+    wave_sync();
+  }
+#pragma unroll
+  for (int o = G; o < 64; o <<= 1) {  // the slices' sums
+    n0 += __shfl_xor(n0, o, 64);
+    n1 += __shfl_xor(n1, o, 64);
+    S.x += __shfl_xor(S.x, o, 64);
+    S.y += __shfl_xor(S.y, o, 64);
+    if constexpr (ADJ) {
+      n2 += __shfl_xor(n2, o, 64);
+      n3 += __shfl_xor(n3, o, 64);
+      S2.x += __shfl_xor(S2.x, o, 64);
+      S2.y += __shfl_xor(S2.y, o, 64);
+    }
+  }
+  if (slice != 0) return;
+  if (i >= a.nt) return;
+  if constexpr (ADJ) {
+    // t = 1/(z_probe - z) = -1/(z - z_probe): sum G t = -S, sum G t^2 = S2
+    n0 -= S.x;
+    n1 = tg.s * (n1 + S2.x);
+    n2 = tg.s * (n2 - S2.y);
+    n3 *= tg.s;
+  } else {
+    n0 += S.y;
+    n1 += S.x;
+  }
+  if (part) {
+    const int64_t stride = (int64_t)a.ksplit * a.nt, at = (int64_t)blockIdx.y * a.nt + i;
+    part[at] = n0;
+    part[stride + at] = n1;
+    if constexpr (ADJ) {
+      part[2 * stride + at] = n2;
+      part[3 * stride + at] = n3;
+    }
+  } else {
+    const uint32_t o = torder[i];
+    o0[o] += n0;
+    o1[o] += n1;
+    if constexpr (ADJ) {
+      o2[o] += n2;
+      o3[o] += n3;
     }
   }
 }
 
-// tu[i] += sum over k (in order) of the split walk's partials
-__global__ __launch_bounds__(kBlock) void tree_reduce_kernel(int64_t nt, int ksplit,
+// outputs[torder[i]] += the shares' partial sums, in order (nf components)
+__global__ __launch_bounds__(kBlock) void tree_reduce_kernel(int64_t nt, int ksplit, int nf,
                                                              const double* __restrict__ part,
-                                                             double* __restrict__ tu,
-                                                             double* __restrict__ tv) {
+                                                             const uint32_t* __restrict__ torder,
+                                                             double* __restrict__ o0,
+                                                             double* __restrict__ o1,
+                                                             double* __restrict__ o2,
+                                                             double* __restrict__ o3) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i >= nt) return;
-  double su = 0.0, sv = 0.0;
-  for (int k = 0; k < ksplit; ++k) {
-    su += part[(int64_t)k * nt + i];
-    sv += part[(int64_t)(ksplit + k) * nt + i];
+  const uint32_t o = torder[i];
+  double* const out[4] = {o0, o1, o2, o3};
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    if (f >= nf) break;
+    double s = 0.0;
+    for (int k = 0; k < ksplit; ++k) s += part[((int64_t)f * ksplit + k) * nt + i];
+    out[f][o] += s;
   }
-  tu[i] += su;
-  tv[i] += sv;
 }
 
-}  // namespace
+inline unsigned blocks(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
-int tree_dev(Device* d, hipStream_t s, int core, double theta, int p, double tol, int64_t ns,
-             const double* sx, const double* sy, const double* ss, const double* sr, int64_t nt,
-             const double* tx, const double* ty, const double* tr, double* tu, double* tv) {
-  if (ns == 0 || nt == 0) return 0;
-  // levels
+struct Problem {
+  int core;
+  int p;
+  double theta, tol;
+  double theta_local;  // for local expansions, whose truncation adds to the moments'
+  // sources, and their charges: strength and radius (velocity) or gv and gu (adjoint)
+  int64_t ns;
+  const double *sx, *sy, *sa, *sb;
+  // targets: radius (may be null for the velocity) and strength (adjoint)
+  int64_t nt;
+  const double *tx, *ty, *tr, *ts;
+  double *o0, *o1, *o2, *o3;
+  int timed;  // kernel class of the evaluation
+};
+
+template <int CORE, bool ADJ>
+void launch_eval(const Problem& q, hipStream_t s, int64_t nsuper, const GroupArgs& ga,
+                 const Trg* trg, const uint32_t* torder, const double4* head, const uint2* kids,
+                 const double2* mom, const Src* src, uint32_t root, Super* super, double2* local, uint32_t* front,
+                 double* part) {
+  if (nsuper)
+    tree_super_kernel<CORE, ADJ><<<(unsigned)nsuper, kSuperBlock, 0, s>>>(
+        q.nt, trg, head, kids, mom, root, q.theta_local, q.tol, super, local, front);
+  const int64_t groups = (q.nt + ga.g - 1) / ga.g;
+  const dim3 grid((unsigned)((groups + kGroupWaves - 1) / kGroupWaves), (unsigned)ga.ksplit);
+  auto* sup = nsuper ? super : nullptr;
+  if (ga.g == 16)
+    tree_group_kernel<CORE, ADJ, 16><<<grid, kGroupBlock, 0, s>>>(
+        ga, trg, torder, head, kids, mom, src, sup, local, front, q.o0, q.o1, q.o2, q.o3, part);
+  else
+    tree_group_kernel<CORE, ADJ, 64><<<grid, kGroupBlock, 0, s>>>(
+        ga, trg, torder, head, kids, mom, src, sup, local, front, q.o0, q.o1, q.o2, q.o3, part);
+}
+
+template <bool ADJ>
+int tree_run(Device* d, hipStream_t s, const Problem& q) {
+  const int64_t ns = q.ns, nt = q.nt;
   Levels lv{};
   int64_t cnt = (ns + kLeaf - 1) / kLeaf, total = 0;
   for (;;) {
@@ -382,94 +1038,149 @@ int tree_dev(Device* d, hipStream_t s, int core, double theta, int p, double tol
     if (cnt == 1) break;
     cnt = (cnt + kFan - 1) / kFan;
   }
-  // a split walk starts from up to kFan cells of one level
-  if ((kFan - 1) * lv.n + kFan > kStack) return fail(O2D_ERR_SIZE, "tree too deep");
-  // buffers
-  void *ko, *to, *tk, *sbuf, *cb, *mb;
-  O2D_TRY(slot(d, kTreeKeys, sizeof(uint32_t) * (ns > nt ? ns : nt), s, &tk));
+  const bool self = !ADJ && q.tx == q.sx && q.ty == q.sy && nt == ns;
+  const bool same = self && q.tr == q.sb;  // sources and targets have the same records
+  const int64_t nsrc = lv.cnt[0] * kLeaf;
+  void *kb, *ko, *to, *sb, *cb, *bb, *mb;
+  O2D_TRY(slot(d, kTreeKeys, sizeof(uint32_t) * std::max(ns, nt), s, &kb));
   O2D_TRY(slot(d, kTreeOrder, sizeof(uint32_t) * ns, s, &ko));
-  O2D_TRY(slot(d, kTreeTOrder, sizeof(uint32_t) * nt, s, &to));
-  O2D_TRY(slot(d, kTreeSrc, sizeof(double) * 4 * ns, s, &sbuf));
-  O2D_TRY(slot(d, kTreeCells, sizeof(Cell) * total, s, &cb));
-  O2D_TRY(slot(d, kTreeMom, sizeof(double2) * p * total, s, &mb));
+  O2D_TRY(slot(d, kTreeSrc, sizeof(Src) * nsrc, s, &sb));
+  O2D_TRY(slot(d, kTreeCells, (sizeof(double4) + sizeof(uint2)) * total, s, &cb));
+  O2D_TRY(slot(d, kTreeBox, sizeof(double4) * total, s, &bb));
+  O2D_TRY(slot(d, kTreeMom, sizeof(double2) * kMaxP * total, s, &mb));
   uint32_t* sorder = static_cast<uint32_t*>(ko);
-  uint32_t* torder = static_cast<uint32_t*>(to);
-  double* xs = static_cast<double*>(sbuf);
-  double *ys = xs + ns, *ssorted = ys + ns, *ws = ssorted + ns;
-  Cell* cells = static_cast<Cell*>(cb);
+  Src* src = static_cast<Src*>(sb);
+  double4* head = static_cast<double4*>(cb);
+  uint2* kids = reinterpret_cast<uint2*>(head + total);
+  double4* box = static_cast<double4*>(bb);
   double2* mom = static_cast<double2*>(mb);
+  const uint32_t* torder = sorder;
+  const Trg* trg;
   {
     KernelTimer kt(O2D_KT_TREE_BUILD, s);
-    O2D_TRY(morton_order(d, s, ns, sx, sy, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(tk),
+    O2D_TRY(morton_order(d, s, ns, q.sx, q.sy, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(kb),
                          sorder, nullptr, false));
-    tree_gather_kernel<<<(unsigned)((ns + kBlock - 1) / kBlock), kBlock, 0, s>>>(
-        ns, sorder, sx, sy, ss, sr, core, xs, ys, ssorted, ws);
+    const int64_t lwaves = (nsrc + 63) / 64;
+    tree_leaf_kernel<ADJ><<<(unsigned)((lwaves + kWaves - 1) / kWaves), kBlock, 0, s>>>(
+        ns, lv.cnt[0], q.p, sorder, q.sx, q.sy, q.sa, q.sb, q.core, src, head, kids, box, mom);
     O2D_LAUNCH_CHECK();
-    constexpr int kCellsPerBlock = kBlock / 64;  // one wave per cell
-    tree_leaf_kernel<<<(unsigned)((lv.cnt[0] + kCellsPerBlock - 1) / kCellsPerBlock), kBlock, 0,
-                       s>>>(ns, lv.cnt[0], p, xs, ys, ssorted, ws, cells, mom);
-    O2D_LAUNCH_CHECK();
-    for (int l = 1; l < lv.n; ++l) {
-      tree_up_kernel<<<(unsigned)((lv.cnt[l] + kCellsPerBlock - 1) / kCellsPerBlock), kBlock, 0, s>>>(
-          lv.cnt[l - 1], lv.cnt[l], p, cells + lv.off[l - 1], mom + lv.off[l - 1] * p,
-          cells + lv.off[l], mom + lv.off[l] * p);
+    for (int l = 0; l + 1 < lv.n; l += 2) {
+      const bool two = l + 2 < lv.n;
+      tree_up_kernel<<<(unsigned)((lv.cnt[l + 1] + kFan - 1) / kFan), kBlock, 0, s>>>(
+          (uint32_t)lv.off[l], (uint32_t)lv.cnt[l], (uint32_t)lv.off[l + 1],
+          (uint32_t)lv.cnt[l + 1], two ? (uint32_t)lv.off[l + 2] : 0u,
+          two ? (uint32_t)lv.cnt[l + 2] : 0u, q.p, head, kids, box, mom);
       O2D_LAUNCH_CHECK();
     }
-    O2D_TRY(morton_order(d, s, nt, tx, ty, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(tk),
-                         torder, nullptr, false));
+    if (!self) {
+      O2D_TRY(slot(d, kTreeTOrder, sizeof(uint32_t) * nt, s, &to));
+      O2D_TRY(morton_order(d, s, nt, q.tx, q.ty, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(kb),
+                           static_cast<uint32_t*>(to), nullptr, false));
+      torder = static_cast<const uint32_t*>(to);
+    }
+    if (same) {
+      trg = reinterpret_cast<const Trg*>(src);
+    } else {
+      void* tb;
+      O2D_TRY(slot(d, kTreeTrg, sizeof(Trg) * nt, s, &tb));
+      tree_targets_kernel<ADJ><<<blocks(nt), kBlock, 0, s>>>(nt, torder, q.tx, q.ty, q.tr, q.ts,
+                                                             q.core, static_cast<Trg*>(tb));
+      O2D_LAUNCH_CHECK();
+      trg = static_cast<const Trg*>(tb);
+    }
     kt.stop();
   }
-  // each wave's walk is a chain of dependent loads, so the walk wants many waves per SIMD, and
-  // the groups' costs vary widely: below 256 waves per CU, split the walk of each group over up
-  // to 64 waves, each from its share of one level's cells (measured on the 1M blob workload: the
-  // tracers' 1,024 groups over 64 waves each and the particles' 16,384 groups over 4 each took
-  // 6.1 ms, against 7.5 ms for 4 and 1)
-  const int64_t waves = (nt + 63) / 64, want = 256 * (int64_t)d->num_cu;
-  int ksplit = 1, slevel = lv.n - 1;
-  if (waves < want && lv.n > 1) {
-    ksplit = (int)std::min<int64_t>(64, (want + waves - 1) / waves);
-    for (int l = lv.n - 1; l >= 0; --l)
-      if (lv.cnt[l] >= ksplit) {
-        slevel = l;
-        break;
-      }
-    if (lv.cnt[slevel] < ksplit) ksplit = (int)lv.cnt[slevel];
-  }
+  GroupArgs ga{};
+  ga.nt = nt;
+  ga.p = q.p;
+  ga.theta = q.theta;
+  ga.tol = q.tol;
+  const int64_t nsup = (nt + kSuper - 1) / kSuper;
+  const int64_t nsuper = nsup >= kMinSupers ? nsup : 0;
+  // waves per group: enough for O2D_TREE_WAVES waves per CU
+  // targets much sparser than the sources: a box of 64 would hold many leaves that few of its
+  // targets are near (65,536 tracers among 1M particles: 0.47 ms in groups of 16, 0.51 of 32,
+  // 0.72 of 64; the particles on themselves 3.2, 2.4 and 2.0 ms)
+  ga.g = nt < ns / 4 ? 16 : 64;
+  const int64_t groups = (nt + ga.g - 1) / ga.g, want = (int64_t)(ga.g == 64 ? kWaves64 : kWaves16) * d->num_cu;
+  ga.ksplit = groups >= want ? 1 : (int)std::min<int64_t>(32, (want + groups - 1) / groups);
+  // starting cells without a frontier: the lowest level that is tested in one go
+  int sl = lv.n - 1;
+  while (sl > 0 && lv.cnt[sl - 1] <= 64) --sl;
+  ga.start = (uint32_t)lv.off[sl];
+  ga.nstart = (uint32_t)lv.cnt[sl];
+  const int nf = ADJ ? 4 : 2;
   double* part = nullptr;
-  if (ksplit > 1) {
+  if (ga.ksplit > 1) {
     void* pp;
-    O2D_TRY(slot(d, kPartials, sizeof(double) * 2 * ksplit * nt, s, &pp));
+    O2D_TRY(slot(d, kPartials, sizeof(double) * nf * ga.ksplit * nt, s, &pp));
     part = static_cast<double*>(pp);
   }
-  TreeArgs a{lv, cells, mom, xs, ys, ssorted, ws, ns, p, theta, tol, ksplit, slevel, part};
-  const dim3 grid((unsigned)((nt + kTBlock - 1) / kTBlock), (unsigned)ksplit);
-  KernelTimer kt(O2D_KT_TREE_EVAL, s);
-  switch (core) {
-    case O2D_CORE_RM:
-      tree_eval_kernel<O2D_CORE_RM><<<grid, kTBlock, 0, s>>>(a, nt, torder, tx, ty, tr, tu, tv);
-      break;
-    case O2D_CORE_GAUSSIAN:
-      tree_eval_kernel<O2D_CORE_GAUSSIAN><<<grid, kTBlock, 0, s>>>(a, nt, torder, tx, ty, tr, tu,
-                                                                   tv);
-      break;
-    case O2D_CORE_WL:
-      tree_eval_kernel<O2D_CORE_WL><<<grid, kTBlock, 0, s>>>(a, nt, torder, tx, ty, tr, tu, tv);
-      break;
-    case O2D_CORE_V2:
-      tree_eval_kernel<O2D_CORE_V2><<<grid, kTBlock, 0, s>>>(a, nt, torder, tx, ty, tr, tu, tv);
-      break;
+  Super* super = nullptr;
+  double2* local = nullptr;
+  uint32_t* front = nullptr;
+  if (nsuper) {
+    void* up;
+    O2D_TRY(slot(d, kTreeSuper,
+                 (sizeof(Super) + sizeof(double2) * kMaxP + sizeof(uint32_t) * kFront) * nsuper, s,
+                 &up));
+    local = static_cast<double2*>(up);
+    super = reinterpret_cast<Super*>(local + kMaxP * nsuper);
+    front = reinterpret_cast<uint32_t*>(super + nsuper);
+  }
+  const uint32_t root = (uint32_t)lv.off[lv.n - 1];
+  KernelTimer kt(q.timed, s);
+#define O2D_EVAL(C) \
+  launch_eval<C, ADJ>(q, s, nsuper, ga, trg, torder, head, kids, mom, src, root, super, local, front, part)
+  switch (q.core) {
+    case O2D_CORE_GAUSSIAN: O2D_EVAL(O2D_CORE_GAUSSIAN); break;
     default:
-      tree_eval_kernel<O2D_CORE_V3><<<grid, kTBlock, 0, s>>>(a, nt, torder, tx, ty, tr, tu, tv);
+      if constexpr (!ADJ) {
+        if (q.core == O2D_CORE_RM) O2D_EVAL(O2D_CORE_RM);
+        else if (q.core == O2D_CORE_WL) O2D_EVAL(O2D_CORE_WL);
+        else if (q.core == O2D_CORE_V2) O2D_EVAL(O2D_CORE_V2);
+        else O2D_EVAL(O2D_CORE_V3);
+      }
       break;
   }
+#undef O2D_EVAL
   kt.stop();
   O2D_LAUNCH_CHECK();
-  if (ksplit > 1) {
-    tree_reduce_kernel<<<(unsigned)((nt + kBlock - 1) / kBlock), kBlock, 0, s>>>(nt, ksplit, part,
-                                                                               tu, tv);
+  if (part) {
+    tree_reduce_kernel<<<blocks(nt), kBlock, 0, s>>>(nt, ga.ksplit, nf, part, torder, q.o0, q.o1,
+                                                     q.o2, q.o3);
     O2D_LAUNCH_CHECK();
   }
   return 0;
+}
+
+}  // namespace
+
+int tree_dev(Device* d, hipStream_t s, int core, double theta, int p, double tol, int64_t ns,
+             const double* sx, const double* sy, const double* ss, const double* sr, int64_t nt,
+             const double* tx, const double* ty, const double* tr, double* tu, double* tv) {
+  if (ns == 0 || nt == 0) return 0;
+  const Problem q{core, p, theta, tol, kLocalShare * theta, ns, sx, sy, ss, sr, nt, tx, ty, tr, nullptr,
+                  tu, tv, nullptr, nullptr, O2D_KT_TREE_EVAL};
+  return tree_run<false>(d, s, q);
+}
+
+int gauss_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const double* sy,
+                   const double* ss, const double* sr, int64_t nt, const double* tx,
+                   const double* ty, const double* tr, double* tu, double* tv) {
+  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kExactTheta, 0.0, kLocalShare * kExactTheta, ns, sx, sy, ss, sr, nt,
+                  tx, ty, tr, nullptr, tu, tv, nullptr, nullptr,
+                  tr ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT};
+  return tree_run<false>(d, s, q);
+}
+
+int gauss_adjoint_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx,
+                           const double* sy, const double* ss, const double* sr, int64_t nt,
+                           const double* tx, const double* ty, const double* gu,
+                           const double* gv, double* gx, double* gy, double* gs, double* gr) {
+  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kExactTheta, 0.0, kLocalShare * kExactTheta, nt, tx, ty, gv, gu, ns,
+                  sx, sy, sr, ss, gs, gx, gy, gr, O2D_KT_ADJOINT};
+  return tree_run<true>(d, s, q);
 }
 
 }  // namespace o2d
