@@ -29,10 +29,6 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kTile = 256;
 constexpr int kTpl = 2;
-#ifndef O2D_TREE_PAIRS
-#define O2D_TREE_PAIRS 1e8
-#endif
-constexpr double kTreePairs = O2D_TREE_PAIRS;
 
 struct alignas(16) Probe {
   double x, y, gu, gv;

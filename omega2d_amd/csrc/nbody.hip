@@ -59,10 +59,6 @@ constexpr int kGroup = 64;   // sources sharing one centroid in the split form
 #endif
 constexpr int kMinChunkTiles = 16;
 constexpr int kStage = 4;  // source tiles brought into LDS per stage of the split kernel
-#ifndef O2D_TREE_PAIRS
-#define O2D_TREE_PAIRS 1e8
-#endif
-constexpr double kTreePairs = O2D_TREE_PAIRS;
 constexpr int kTpl64 = O2D_TPL64;  // targets per lane, plain form
 constexpr int kTpl32 = O2D_TPL32;  // targets per lane, split form
 
