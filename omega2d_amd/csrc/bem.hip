@@ -281,8 +281,11 @@ int bem_factor_dev(Device* d, hipStream_t s, int64_t n, const double* A, int64_t
   rocblas_handle h;
   O2D_TRY(blas_of(d, s, &h));
   if (n <= lu_max_order()) {
-    O2D_TRY(lu_factor_dev(d, s, (int)n, static_cast<double*>(lu), (int)n,
-                          static_cast<int*>(piv), static_cast<int*>(info)));
+    void* perm;
+    O2D_TRY(slot(d, kLuPerm, sizeof(int) * n, s, &perm));
+    O2D_TRY(lu_factor_dev(d, s, (int)n, static_cast<double*>(lu), (int)n, static_cast<int*>(piv),
+                          static_cast<int*>(perm), static_cast<int*>(info)));
+    O2D_TRY(lu_prepare_solve(d, s, (int)n, static_cast<const double*>(lu)));
   } else if (rocsolver_dgetrf(h, (rocblas_int)n, (rocblas_int)n, static_cast<double*>(lu),
                               (rocblas_int)n, static_cast<rocblas_int*>(piv),
                               static_cast<rocblas_int*>(info)) != rocblas_status_success) {
@@ -305,16 +308,14 @@ __global__ __launch_bounds__(kBlock) void identity_kernel(int64_t n, double* __r
     a[e] = (e % (n + 1) == 0) ? 1.0 : 0.0;
 }
 
-// Solves A x = b with the kept factors. A matrix solved against more than once with the same
-// factors is worth inverting: the second solve builds A^-1 from them, as the solution of A X = I
-// (rocsolver getrs with n right-hand sides: the row interchanges, then two triangular solves
-// with n columns on the fp64 matrix cores; 1.2 ms at order 2049 and 5.3 ms at 4097, where
-// rocsolver getri took 4.8 and 22.7 ms), about the cost of one solve by two latency-bound
-// triangular solves (1.1 and 2.8 ms). Every solve from then on is one dgemv, an HBM-bound read
-// of n^2 doubles (0.09 and 0.17 ms). A body that does not move keeps its inverse for the whole
-// run; a body in relative motion, refactored every step and solved once per Runge-Kutta stage,
-// builds it at its second stage.
-constexpr int kSolvesBeforeInverse = 1;
+// Solves A x = b with the kept factors. A matrix solved against many times with the same factors
+// is worth inverting: the fourth solve builds A^-1 from them, as the solution of A X = I (rocsolver
+// getrs with n right-hand sides: the row interchanges, then two triangular solves with n columns
+// on the fp64 matrix cores; 1.2 ms at order 2049 and 5.3 ms at 4097), and every solve from then on
+// is one matrix-vector product (0.013 ms at 2049, against 0.27 by two triangular solves). A body that
+// does not move keeps its inverse for the whole run; a body in relative motion, refactored every
+// step and solved once per Runge-Kutta stage, never builds it: its two or three solves cost less.
+constexpr int kSolvesBeforeInverse = 3;
 
 int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* x) {
   if (!d->lu_ready || d->lu_n != n)
@@ -336,22 +337,11 @@ int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* 
     d->inv_ready = true;
   }
   ++d->lu_solves;
-  if (d->inv_ready) {
-    const double* src = b;
-    if (x == b) {  // dgemv needs distinct input and output vectors
-      void* t;
-      O2D_TRY(slot(d, kSolveTmp, sizeof(double) * n, s, &t));
-      O2D_HIP(hipMemcpyAsync(t, b, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-      src = static_cast<const double*>(t);
-    }
-    const double one = 1.0, zero = 0.0;
-    if (rocblas_set_pointer_mode(h, rocblas_pointer_mode_host) != rocblas_status_success ||
-        rocblas_dgemv(h, rocblas_operation_none, (rocblas_int)n, (rocblas_int)n, &one,
-                      static_cast<const double*>(d->buf[kInv]), (rocblas_int)n, src, 1, &zero, x,
-                      1) != rocblas_status_success)
-      return fail(O2D_ERR_HIP, "rocblas_dgemv failed");
-    return 0;
-  }
+  if (d->inv_ready)
+    return matvec_dev(d, s, (int)n, static_cast<const double*>(d->buf[kInv]), b, x);
+  if (n <= lu_max_order())
+    return lu_solve_dev(d, s, (int)n, static_cast<const double*>(d->buf[kLU]),
+                        static_cast<const int*>(d->buf[kLuPerm]), b, x);
   if (x != b) O2D_HIP(hipMemcpyAsync(x, b, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   if (rocsolver_dgetrs(h, rocblas_operation_none, (rocblas_int)n, 1, static_cast<double*>(d->buf[kLU]),
                        (rocblas_int)n, static_cast<const rocblas_int*>(d->buf[kPivots]), x,

@@ -433,7 +433,8 @@ __global__ __launch_bounds__(kPT) void lu_panel_kernel(int n, int P, int nb,
   }
 }
 
-// The block's row pairs on every column, one wave per column, all loads of a column before its
+// The block's row pairs on every column (and, as column n, on the row permutation perm that the
+// solves gather their right-hand side by), one wave per column, all loads of a column before its
 // stores (rows that move form closed cycles). On a trailing column (j >= P + kNB) the block rows
 // are then solved with L11 (A12 <- L11^-1 A12, L11 unit lower, read from l11 in column-major
 // order): pair l < kNB has destination P + l, so lane l already holds that row's new value, and
@@ -443,16 +444,24 @@ __global__ __launch_bounds__(kPT) void lu_panel_kernel(int n, int P, int nb,
 __global__ __launch_bounds__(256) void lu_swap_solve_kernel(int n, int P, double* __restrict__ A,
                                                             int lda,
                                                             const int* __restrict__ bpairs,
-                                                            const double* __restrict__ l11) {
+                                                            const double* __restrict__ l11,
+                                                            int* __restrict__ perm) {
   static_assert(kNB == 64 && kMaxPairs == 2 * 64, "a lane per block row, two pairs per lane");
   const int lane = threadIdx.x & 63;
   const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (j >= n) return;  // the whole wave
+  if (j > n) return;  // the whole wave
   const int cnt = bpairs[0];
-  double* cp = A + (size_t)j * lda;
   const bool ok0 = lane < cnt, ok1 = lane + 64 < cnt;
   const int d0 = ok0 ? bpairs[1 + 2 * lane] : 0, s0 = ok0 ? bpairs[2 + 2 * lane] : 0;
   const int d1 = ok1 ? bpairs[1 + 2 * (lane + 64)] : 0, s1 = ok1 ? bpairs[2 + 2 * (lane + 64)] : 0;
+  if (j == n) {  // the row permutation so far, moved as a column is
+    const int p0 = ok0 ? perm[s0] : 0, p1 = ok1 ? perm[s1] : 0;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (ok0) perm[d0] = p0;
+    if (ok1) perm[d1] = p1;
+    return;
+  }
+  double* cp = A + (size_t)j * lda;
   const double v0 = ok0 ? cp[s0] : 0.0;
   const double v1 = ok1 ? cp[s1] : 0.0;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every load of the column has returned
@@ -476,7 +485,12 @@ __global__ __launch_bounds__(256) void lu_swap_solve_kernel(int n, int P, double
   cp[P + lane] = v;
 }
 
-__global__ void lu_zero_info_kernel(int* info) { *info = 0; }
+// info = 0 and perm the identity
+__global__ __launch_bounds__(256) void lu_start_kernel(int n, int* __restrict__ perm, int* info) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) perm[i] = i;
+  if (i == 0) *info = 0;
+}
 
 // the panel kernel for q rows per thread, q <= Q
 template <int Q>
@@ -518,8 +532,10 @@ static int aux_of(Device* d, hipStream_t s, hipStream_t* B, rocblas_handle* hb) 
 int64_t lu_max_order() { return kMaxOrder; }
 
 // In-place LU of the n x n column-major matrix A (leading dimension lda), pivots to ipiv
-// (1-based), info (device int) = 0 or the first zero pivot (1-based).
-int lu_factor_dev(Device* d, hipStream_t s, int n, double* A, int lda, int* ipiv, int* info) {
+// (1-based), the row permutation they compose to perm (row i of the factors is row perm[i] of A),
+// info (device int) = 0 or the first zero pivot (1-based).
+int lu_factor_dev(Device* d, hipStream_t s, int n, double* A, int lda, int* ipiv, int* perm,
+                  int* info) {
   if (n <= 0) return 0;
   if (n > kMaxOrder) return fail(O2D_ERR_SIZE, "blocked LU takes n <= %d", kMaxOrder);
   rocblas_handle h;
@@ -531,7 +547,7 @@ int lu_factor_dev(Device* d, hipStream_t s, int n, double* A, int lda, int* ipiv
                &pb));
   double* l11 = static_cast<double*>(pb);
   int* bpairs = reinterpret_cast<int*>(l11 + kNB * kNB);
-  lu_zero_info_kernel<<<1, 1, 0, s>>>(info);
+  lu_start_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, perm, info);
   O2D_LAUNCH_CHECK();
   // look-ahead: a large trailing update of block k is split into the next block's columns, on
   // s, and the rest, on the second stream, so the next panel (one workgroup) runs beside it. The
@@ -551,7 +567,7 @@ int lu_factor_dev(Device* d, hipStream_t s, int n, double* A, int lda, int* ipiv
     O2D_LAUNCH_CHECK();
     if (rest_pending) O2D_HIP(hipStreamWaitEvent(s, e_rest, 0));
     rest_pending = false;
-    lu_swap_solve_kernel<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(n, P, A, lda, bpairs, l11);
+    lu_swap_solve_kernel<<<(unsigned)(n / 4 + 1), 256, 0, s>>>(n, P, A, lda, bpairs, l11, perm);
     O2D_LAUNCH_CHECK();
     const int pend = P + nb;
     const int nr = n - pend;

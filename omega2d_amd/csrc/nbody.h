@@ -46,7 +46,14 @@ int bem_factor_dev(Device* d, hipStream_t s, int64_t n, const double* A, int64_t
 
 // blocked LU with partial pivoting (lu.hip), n <= lu_max_order(); ipiv 1-based, info device int
 int64_t lu_max_order();
-int lu_factor_dev(Device* d, hipStream_t s, int n, double* A, int lda, int* ipiv, int* info);
+int lu_factor_dev(Device* d, hipStream_t s, int n, double* A, int lda, int* ipiv, int* perm,
+                  int* info);
+// solves with those factors (lusolve.hip): lu_prepare_solve once per factorisation
+int lu_prepare_solve(Device* d, hipStream_t s, int n, const double* lu);
+int lu_solve_dev(Device* d, hipStream_t s, int n, const double* lu, const int* perm,
+                 const double* b, double* x);
+// x = A b, A n x n column-major
+int matvec_dev(Device* d, hipStream_t s, int n, const double* a, const double* b, double* x);
 int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* x);
 
 int rk_move_dev(Device* d, hipStream_t s, int64_t n, double dt, int nstage, const double* w,

@@ -26,7 +26,7 @@ enum Slot : int {
   kPanX, kPanY, kPanIdx, kPanVs, kPanSs,
   kPanGeom,
   kMatA, kRhs,
-  kLU, kPivots, kInfo,
+  kLU, kPivots, kInfo, kLuPerm, kLuDinv,
   kRkPtrs, kRkStage,
   kGradX, kGradY, kGradS, kGradR,
   kNearPart, kNodeNorm, kPanRec, kCutTable, kNearCounts, kNearTiles,
