@@ -111,7 +111,7 @@ __device__ __forceinline__ double exp_neg_core(double x) {
   return ldexp(__builtin_fma(r, q, 1.0), (int)n);
 }
 
-// Gaussian at or beyond the cutoffs, or within kCutMargin of one (few pairs)
+// Gaussian within kCutMargin of a cutoff, beyond the far one, or not a number (few pairs)
 __device__ __noinline__ double gauss_edge64(double dx, double dy, double d2, double w) {
   const double cf = rcp64(w);
   const double x = d2 * cf;
@@ -121,15 +121,17 @@ __device__ __noinline__ double gauss_edge64(double dx, double dy, double d2, dou
   return br > 0 ? ood2 : (1.0 - exp_neg_core(x)) * ood2;
 }
 
-// Gaussian inside (or at) its compact cutoff (src/CoreFunc.h:117-131): between the cutoffs first,
-// then the pairs at them. Inline for loops whose pairs are mostly inside the core (100,000
-// particles all inside each other's cores: 17 ms, against 22 out of line and 24.6 with the
-// library's exp), out of line for loops that meet few of them (a 262k blob sum takes 4% longer
-// with it inline).
+// Gaussian inside (or at) its compact cutoff (src/CoreFunc.h:117-131): between the cutoffs, below
+// the near one (a particle on itself), then the pairs at them. Inline for loops whose pairs are
+// mostly inside the core (100,000 particles all inside each other's cores: 17 ms, against 22 out
+// of line and 24.6 with the library's exp), out of line for loops that meet few of them (a 262k
+// blob sum takes 4% longer with it inline).
 __device__ __forceinline__ double gauss_inside64(double dx, double dy, double d2, double w) {
-  const double x = d2 * rcp64(w);
+  const double cf = rcp64(w);
+  const double x = d2 * cf;
   if (x > kGaussNear * (1.0 + kCutMargin) && x < kGaussFar * (1.0 - kCutMargin))
     return (1.0 - exp_neg_core(x)) * rcp64(d2);
+  if (x < kGaussNear * (1.0 - kCutMargin)) return cf;
   return gauss_edge64(dx, dy, d2, w);
 }
 __device__ __noinline__ double gauss_core64(double dx, double dy, double d2, double w) {
