@@ -200,7 +200,7 @@ int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx
                 const double* tx, const double* ty, const double* gu, const double* gv,
                 double* gx, double* gy, double* gs, double* gr) {
   if (ns == 0 || nt == 0) return 0;
-  if (core == O2D_CORE_GAUSSIAN && (double)ns * (double)nt >= kTreePairs)
+  if (core == O2D_CORE_GAUSSIAN && (double)ns * (double)nt >= kTreePairsAdjoint)
     return gauss_adjoint_tree_dev(d, s, ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, gx, gy, gs, gr);
   const int64_t swgs = (ns + kBlock * kTpl - 1) / (kBlock * kTpl);
   const int64_t ntiles = (nt + kTile - 1) / kTile;

@@ -65,11 +65,12 @@ int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx
                 double* gx, double* gy, double* gs, double* gr);
 
 // the fp64 Gaussian velocity sum and its adjoint with the sources beyond the compact cutoff taken
-// by clusters, to rounding (treecode.hip); and the pairs from which that is faster than the pair
-// by pair sums: particles on themselves 147 us against 152 at 8,000, 228 against 247 at 16,000, 310
-// against 597 at 32,000; 30,000 on 3,000 points 209 us against 172, 250,000 on 4,096 439 us
-// against 658
-constexpr double kTreePairs = 2e8;
+// by clusters, to rounding (treecode.hip), and the pairs from which they are faster than the pair
+// by pair sums. Clusters against pairs: particles on themselves 221 us against 203 at 16,000, 243
+// against 264 at 20,000, 299 against 590 at 32,000; 100,000 on 3,000 points 279 against 250, 30,000
+// on 16,000 286 against 334. With the adjoint: 50,000 on 4,096 374 against 381, 100,000 on 1,000 372
+// against 312, on 3,000 409 against 518.
+constexpr double kTreePairs = 3.5e8, kTreePairsAdjoint = 2e8;
 int gauss_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const double* sy,
                    const double* ss, const double* sr, int64_t nt, const double* tx,
                    const double* ty, const double* tr, double* tu, double* tv);

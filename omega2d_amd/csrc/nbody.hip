@@ -58,6 +58,9 @@ constexpr int kGroup = 64;   // sources sharing one centroid in the split form
 #define O2D_WANT64 128
 #endif
 constexpr int kMinChunkTiles = 16;
+constexpr int kUnit = 64;         // sources in the shortest chunk of the fp64 form for small sums
+constexpr int64_t kFewWgs = 16;  // pairs of a target set and a source tile per CU below which a sum
+                                 // is small
 constexpr int kStage = 4;  // source tiles brought into LDS per stage of the split kernel
 constexpr int kTpl64 = O2D_TPL64;  // targets per lane, plain form
 constexpr int kTpl32 = O2D_TPL32;  // targets per lane, split form
@@ -68,13 +71,14 @@ struct alignas(16) Src64 {
 
 // ---------------------------------------------------------------------------- plain fp64
 
-// the pair loop over one staged tile; TR adds each target's radius term per pair
-template <int CORE, int RES, bool TR, int TPL>
-__device__ __forceinline__ void tile_pairs64(const Src64* __restrict__ tile, const double* px,
-                                             const double* py, const double* pw, double* au,
-                                             double* av, double* aw) {
+// the pair loop over the first nk staged sources; TR adds each target's radius term per pair
+template <int CORE, int RES, bool TR, int TPL, bool FEW>
+__device__ __forceinline__ void tile_pairs64(const Src64* __restrict__ tile, int nk,
+                                             const double* px, const double* py,
+                                             const double* pw, double* au, double* av,
+                                             double* aw) {
 #pragma unroll 4
-  for (int k = 0; k < kTile; ++k) {
+  for (int k = 0; k < nk; ++k) {
     const Src64 q = tile[k];
 #pragma unroll
     for (int t = 0; t < TPL; ++t) {
@@ -83,7 +87,12 @@ __device__ __forceinline__ void tile_pairs64(const Src64* __restrict__ tile, con
       const double d2 = __builtin_fma(dx, dx, dy * dy);
       const double w = TR ? wsum(q.w, pw[t]) : q.w;
       if constexpr (RES == O2D_VELONLY) {
-        const double g = q.s * core_k64<CORE>(dx, dy, d2, w);
+        double k0;
+        if constexpr (CORE == O2D_CORE_GAUSSIAN && FEW)
+          k0 = d2 > kGaussFar * (1.0 + kCutMargin) * w ? rcp64(d2) : gauss_inside64(dx, dy, d2, w);
+        else
+          k0 = core_k64<CORE>(dx, dy, d2, w);
+        const double g = q.s * k0;
         au[t] = __builtin_fma(-g, dy, au[t]);
         av[t] = __builtin_fma(g, dx, av[t]);
       } else {
@@ -99,8 +108,20 @@ __device__ __forceinline__ void tile_pairs64(const Src64* __restrict__ tile, con
 
 // src: the staged sources in Morton order; tq, tw: the targets' positions and radius terms in
 // Morton order (tw unused unless TR); torder[i]: the input index of sorted target i (torder
-// null: the targets are in input order)
-template <int CORE, int RES, bool TR, int TPL>
+// null: the targets are in input order).
+//
+// Bound by the fp64 vector units (a Rosenhead-Moore or far Gaussian pair is 11 fp64 operations and
+// a reciprocal), by latency where the sum is small:
+//
+// FEW: the form for sums too small to fill the chip with whole tiles (fewer than kFewWgs pairs of
+// 512 targets and 256 sources per CU). There the launch lasts as long as one workgroup's own loop,
+// so a lane holds one target, a chunk can be as short as kUnit sources, and the Gaussian's inside
+// is inline: a call costs its whole latency, and the tile a wave's own targets lie in makes one for
+// most of its sources. Whole calls on themselves: 6,715 blob particles 209 us with two targets a
+// lane, whole tiles and calls, 132 with the inside inline, 84 in this form; 10,000 Rosenhead-Moore
+// particles 100 and 81. At kFewWgs (16,000 on themselves) 221 and 203 us; beyond it two targets
+// a lane halve the LDS reads per pair and win (a 262k blob sum is 4% slower inline).
+template <int CORE, int RES, bool TR, int TPL, bool FEW>
 __global__ __launch_bounds__(kBlock) void nbody64_kernel(
     int64_t ns, const Src64* __restrict__ src, int64_t nt, const double2* __restrict__ tq,
     const double* __restrict__ tw, const uint32_t* __restrict__ torder, int64_t chunk,
@@ -142,6 +163,7 @@ __global__ __launch_bounds__(kBlock) void nbody64_kernel(
   const int64_t je = jb + chunk < ns ? jb + chunk : ns;
   for (int64_t j0 = jb; j0 < je; j0 += kTile) {
     const int64_t j = j0 + tid;
+    const int nk = FEW && je - j0 < kTile ? (int)((je - j0 + 3) & ~int64_t(3)) : kTile;
     Src64 s = src[j < je ? j : je - 1];
     if (j >= je) s.s = 0.0;  // zero strength at the chunk's last source: contributes exactly 0
     if (uni) s.w = wsum(s.w, w0);
@@ -189,7 +211,7 @@ __global__ __launch_bounds__(kBlock) void nbody64_kernel(
       }
       if (__all(far)) {
 #pragma unroll 4
-        for (int k = 0; k < kTile; ++k) {
+        for (int k = 0; k < nk; ++k) {
           const Src64 q = tile[k];
 #pragma unroll
           for (int t = 0; t < TPL; ++t) {
@@ -204,9 +226,9 @@ __global__ __launch_bounds__(kBlock) void nbody64_kernel(
       }
     }
     if (uni)
-      tile_pairs64<CORE, RES, false, TPL>(tile, px, py, pw, au, av, aw);
+      tile_pairs64<CORE, RES, false, TPL, FEW>(tile, nk, px, py, pw, au, av, aw);
     else
-      tile_pairs64<CORE, RES, TR, TPL>(tile, px, py, pw, au, av, aw);
+      tile_pairs64<CORE, RES, TR, TPL, FEW>(tile, nk, px, py, pw, au, av, aw);
   }
 
 #pragma unroll
@@ -425,7 +447,10 @@ void nbody32_kernel(
   }
 }
 
-// out[order[i]] += sum over chunks c (in order) of part[c*nt + i] (order null: the identity)
+// out[order[i]] += sum over chunks c of part[c*nt + i] (order null: the identity). A workgroup takes
+// 64 targets, its four waves a quarter of the chunks each, in order, and their sums are added in
+// wave order. Bound by the latency of its loads: with a thread per target, 10,000 targets kept 157
+// waves busy with a loop over 40 chunks each (7.8 us, 4.9 us so).
 __global__ __launch_bounds__(kBlock) void reduce_chunks_kernel(int64_t nchunk, int64_t nt,
                                                                const uint32_t* __restrict__ order,
                                                                const double* __restrict__ pu,
@@ -434,18 +459,33 @@ __global__ __launch_bounds__(kBlock) void reduce_chunks_kernel(int64_t nchunk, i
                                                                double* __restrict__ ou,
                                                                double* __restrict__ ov,
                                                                double* __restrict__ ow) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= nt) return;
+  constexpr int kWaves = kBlock / 64;
+  __shared__ double sm[3][kWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t i = (int64_t)blockIdx.x * 64 + lane;
+  const int64_t share = (nchunk + kWaves - 1) / kWaves;
+  const int64_t c0 = wave * share, c1 = c0 + share < nchunk ? c0 + share : nchunk;
   double su = 0.0, sv = 0.0, sw = 0.0;
-  for (int64_t c = 0; c < nchunk; ++c) {
-    su += pu[c * nt + i];
-    sv += pv[c * nt + i];
-    if (pw) sw += pw[c * nt + i];
+  if (i < nt) {
+#pragma unroll 4
+    for (int64_t c = c0; c < c1; ++c) {
+      su += pu[c * nt + i];
+      sv += pv[c * nt + i];
+      if (pw) sw += pw[c * nt + i];
+    }
   }
+  sm[0][wave][lane] = su;
+  sm[1][wave][lane] = sv;
+  sm[2][wave][lane] = sw;
+  __syncthreads();
+  const int f = wave;  // a component per wave
+  if (f > (pw ? 2 : 1) || i >= nt) return;
+  double s = sm[f][0][lane];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) s += sm[f][w][lane];
   const int64_t o = order ? (int64_t)order[i] : i;
-  ou[o] += su;
-  ov[o] += sv;
-  if (pw) ow[o] += sw;
+  double* out = f == 0 ? ou : (f == 1 ? ov : ow);
+  out[o] += s;
 }
 
 // ---------------------------------------------------------------------------- staging
@@ -574,19 +614,24 @@ ChunkPlan plan_chunks(const Device* d, int64_t target_wgs, int64_t ntiles, int p
 }
 
 template <int CORE, int RES, bool TR>
-void launch64(dim3 grid, hipStream_t s, int64_t ns, const Src64* src, int64_t nt,
+void launch64(bool few, dim3 grid, hipStream_t s, int64_t ns, const Src64* src, int64_t nt,
               const double2* tq, const double* tw, const uint32_t* torder, int64_t chunk,
               double* ou, double* ov, double* ow, int direct) {
-  nbody64_kernel<CORE, RES, TR, kTpl64><<<grid, kBlock, 0, s>>>(ns, src, nt, tq, tw, torder, chunk,
-                                                               ou, ov, ow, direct);
+  if (few)
+    nbody64_kernel<CORE, RES, TR, 1, true><<<grid, kBlock, 0, s>>>(ns, src, nt, tq, tw, torder,
+                                                                   chunk, ou, ov, ow, direct);
+  else
+    nbody64_kernel<CORE, RES, TR, kTpl64, false><<<grid, kBlock, 0, s>>>(
+        ns, src, nt, tq, tw, torder, chunk, ou, ov, ow, direct);
 }
 
 template <int CORE>
-void dispatch64(int res, bool tr_present, dim3 grid, hipStream_t s, int64_t ns, const Src64* src,
-                int64_t nt, const double2* tq, const double* tw, const uint32_t* torder,
-                int64_t chunk, double* ou, double* ov, double* ow, int direct) {
+void dispatch64(int res, bool tr_present, bool few, dim3 grid, hipStream_t s, int64_t ns,
+                const Src64* src, int64_t nt, const double2* tq, const double* tw,
+                const uint32_t* torder, int64_t chunk, double* ou, double* ov, double* ow,
+                int direct) {
 #define O2D_L64(R, T) \
-  launch64<CORE, R, T>(grid, s, ns, src, nt, tq, tw, torder, chunk, ou, ov, ow, direct)
+  launch64<CORE, R, T>(few, grid, s, ns, src, nt, tq, tw, torder, chunk, ou, ov, ow, direct)
   if (res == O2D_VELONLY) {
     if (tr_present) O2D_L64(O2D_VELONLY, true);
     else O2D_L64(O2D_VELONLY, false);
@@ -753,11 +798,24 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
     O2D_TRY(prep_targets<double>(d, s, ws, core, nt, tx, ty, tr, sort, self ? order : nullptr,
                                  &torder, &tq, &twv));
 
-    const int64_t twgs = (nt + kBlock * kTpl64 - 1) / (kBlock * kTpl64);
+    int64_t twgs = (nt + kBlock * kTpl64 - 1) / (kBlock * kTpl64);
     const int64_t ntiles = (ns + kTile - 1) / kTile;
     const int nf = res == O2D_VELONLY ? 2 : 3;
-    ChunkPlan cp = plan_chunks(d, twgs, ntiles, O2D_WANT64, max_chunks(ws, nf, nt));
-    const int64_t chunk = cp.per_chunk * kTile;
+    const bool few = twgs * ntiles < kFewWgs * d->num_cu;
+    ChunkPlan cp;
+    int64_t chunk;
+    if (few) {
+      twgs = (nt + kBlock - 1) / kBlock;
+      const int64_t units = (ns + kUnit - 1) / kUnit;
+      int64_t n = std::min((kFewWgs * d->num_cu + twgs - 1) / twgs, units);
+      n = std::max<int64_t>(1, std::min(n, max_chunks(ws, nf, nt)));
+      const int64_t per = (units + n - 1) / n;
+      cp = ChunkPlan{(units + per - 1) / per, per};
+      chunk = per * kUnit;
+    } else {
+      cp = plan_chunks(d, twgs, ntiles, O2D_WANT64, max_chunks(ws, nf, nt));
+      chunk = cp.per_chunk * kTile;
+    }
     const dim3 grid((unsigned)twgs, (unsigned)cp.nchunk);
     double *ou = tu, *ov = tv, *ow = tw;
     const int direct = cp.nchunk == 1;
@@ -770,17 +828,17 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
     }
     KernelTimer kt(trp ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT, s);
     switch (core) {
-      case O2D_CORE_RM: dispatch64<O2D_CORE_RM>(res, trp, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
-      case O2D_CORE_GAUSSIAN: dispatch64<O2D_CORE_GAUSSIAN>(res, trp, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
-      case O2D_CORE_WL: dispatch64<O2D_CORE_WL>(res, trp, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
-      case O2D_CORE_V2: dispatch64<O2D_CORE_V2>(res, trp, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
-      default: dispatch64<O2D_CORE_V3>(res, trp, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
+      case O2D_CORE_RM: dispatch64<O2D_CORE_RM>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
+      case O2D_CORE_GAUSSIAN: dispatch64<O2D_CORE_GAUSSIAN>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
+      case O2D_CORE_WL: dispatch64<O2D_CORE_WL>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
+      case O2D_CORE_V2: dispatch64<O2D_CORE_V2>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
+      default: dispatch64<O2D_CORE_V3>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
     }
     kt.stop();
     O2D_LAUNCH_CHECK();
     if (!direct) {
-      reduce_chunks_kernel<<<grid1(nt), kBlock, 0, s>>>(cp.nchunk, nt, torder, ou, ov, ow, tu, tv,
-                                                        tw);
+      reduce_chunks_kernel<<<(unsigned)((nt + 63) / 64), kBlock, 0, s>>>(cp.nchunk, nt, torder, ou,
+                                                                         ov, ow, tu, tv, tw);
       O2D_LAUNCH_CHECK();
     }
     return 0;
@@ -839,8 +897,8 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
   kt.stop();
   O2D_LAUNCH_CHECK();
   if (!direct) {
-    reduce_chunks_kernel<<<grid1(nt), kBlock, 0, s>>>(cp.nchunk, nt, torder, ou, ov, ow, tu, tv,
-                                                      tw);
+    reduce_chunks_kernel<<<(unsigned)((nt + 63) / 64), kBlock, 0, s>>>(cp.nchunk, nt, torder, ou,
+                                                                       ov, ow, tu, tv, tw);
     O2D_LAUNCH_CHECK();
   }
   return 0;

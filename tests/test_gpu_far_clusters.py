@@ -1,5 +1,5 @@
-"""The fp64 Gaussian velocity sum and its adjoint from 2e8 pairs, where far sources are taken by
-clusters, against the oracle and against the pair by pair sum of the no-allocation entry.
+"""The fp64 Gaussian velocity sum and its adjoint from 3.5e8 and 2e8 pairs, where far sources are
+taken by clusters, against the oracle and against the pair by pair sum of the no-allocation entry.
 
 The bar is the fp64 form's, 1e-12 relative L2 (a far cluster's remainder is below 6e-16 of its
 sum of magnitudes). Sizes sit at the edges of the groups: 64 or 16 targets per wave (16 from four
@@ -67,8 +67,8 @@ def clusters(src, tgt, tr, tu=None, tv=None):
 
 @pytest.mark.parametrize("kind", ["blobs", "square", "line"])
 @pytest.mark.parametrize("sigma", [1e-4, (0.002, 0.03)])
-@pytest.mark.parametrize("ns,nt", [(14143, None), (20033, 16384), (12289, 16385), (65537, 16383),
-                                   (65537, 3111), (262144, 801), (801, 262144)])
+@pytest.mark.parametrize("ns,nt", [(18719, None), (22033, 16384), (21377, 16385), (65537, 16383),
+                                   (131075, 3111), (262144, 1601), (1601, 262144)])
 def test_clusters_match_pairs(ns, nt, sigma, kind):
     rng = np.random.default_rng(ns)
     draw = lambda n: (np.full(n, sigma) if np.isscalar(sigma)  # noqa: E731
@@ -93,8 +93,8 @@ def test_clusters_match_pairs(ns, nt, sigma, kind):
 def test_scaled_problem_scales(scale):
     # cluster moments are taken relative to the cluster's radius: no power over- or underflows
     rng = np.random.default_rng(3)
-    x, y = layout(rng, 16000, "blobs")
-    s, r = rng.normal(size=16000), np.full(16000, 1e-3)
+    x, y = layout(rng, 20000, "blobs")
+    s, r = rng.normal(size=20000), np.full(20000, 1e-3)
     a = clusters((x, y, s, r), None, "self")
     b = clusters((x * scale, y * scale, s, r * scale), None, "self")
     assert rel_l2(np.concatenate(b) * scale, np.concatenate(a)) <= BAR
@@ -102,7 +102,7 @@ def test_scaled_problem_scales(scale):
 
 def test_accumulates_and_all_points_coincide():
     rng = np.random.default_rng(4)
-    n = 15000
+    n = 19000
     src = (np.full(n, 0.5), np.full(n, -0.25), rng.normal(size=n), np.full(n, 0.01))
     t0 = rng.normal(size=n), rng.normal(size=n)
     u, v = clusters(src, (rng.uniform(1, 2, n), rng.uniform(1, 2, n)), None, *t0)
@@ -119,7 +119,7 @@ def test_values_that_are_not_finite(what, value):
     NaN where a tile or leaf is near enough to be tested pair by pair, which is not the same set
     in both; elsewhere neither sum looks at it.)"""
     rng = np.random.default_rng(6)
-    ns, nt = 16100, 16200
+    ns, nt = 19100, 19200
     src = [*layout(rng, ns, "blobs"), rng.normal(size=ns), np.full(ns, 1e-3)]
     tgt, tr = list(layout(rng, nt, "blobs")), np.full(nt, 1e-3)
     {"strength": src[2], "source": src[0], "target": tgt[1], "source radius": src[3],
