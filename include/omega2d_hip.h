@@ -231,6 +231,16 @@ int o2d_hip_rk_move_d(const o2d_env* env, int64_t n, double dt, int32_t nstage, 
 int o2d_hip_rk_move_dev_d(const o2d_env* env, int64_t n, double dt, int32_t nstage,
                           const double* w, const double* const* u, const double* const* v,
                           double* x, double* y);
+/* The same update out of place on device arrays, x = x0 + dt * sum_s w[s] * u_s (x0, y0 may be
+ * x, y); uc, vc (both or neither NULL): the combined stage velocity sum_s w[s] * u_s. */
+int o2d_hip_rk_advance_dev_d(const o2d_env* env, int64_t n, double dt, int32_t nstage,
+                             const double* w, const double* const* u, const double* const* v,
+                             const double* x0, const double* y0, double* x, double* y, double* uc,
+                             double* vc);
+/* u = fsx + u * factor and v = fsy + v * factor on device arrays, each operation rounded
+ * (ElementBase::finalize_vels, src/ElementBase.h:215-221, where factor is 1 / (2 pi)). */
+int o2d_hip_finalize_dev_d(const o2d_env* env, int64_t n, double fsx, double fsy, double factor,
+                           double* u, double* v);
 
 /* ---- adjoint (no reference counterpart) -------------------------------------------------- */
 

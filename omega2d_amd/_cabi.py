@@ -89,6 +89,9 @@ SIGNATURES = {
     "o2d_hip_bem_solve_dev_d": [_envp, _i64, _vp, _vp],
     "o2d_hip_rk_move_d": [_envp, _i64, _dbl, _i32, _vp, _vp, _vp, _vp, _vp],
     "o2d_hip_rk_move_dev_d": [_envp, _i64, _dbl, _i32, _vp, _vp, _vp, _vp, _vp],
+    "o2d_hip_rk_advance_dev_d": [_envp, _i64, _dbl, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                 _vp],
+    "o2d_hip_finalize_dev_d": [_envp, _i64, _dbl, _dbl, _dbl, _vp, _vp],
     "o2d_hip_points_on_points_adjoint_d": [_envp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp,
                                            _vp, _vp, _vp, _vp, _vp],
     "o2d_hip_points_on_points_adjoint_dev_d": [_envp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp,

@@ -56,8 +56,9 @@ int lu_solve_dev(Device* d, hipStream_t s, int n, const double* lu, const int* p
 int matvec_dev(Device* d, hipStream_t s, int n, const double* a, const double* b, double* x);
 int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* x);
 
-int rk_move_dev(Device* d, hipStream_t s, int64_t n, double dt, int nstage, const double* w,
-                const double* const* u, const double* const* v, double* x, double* y);
+int rk_move_dev(hipStream_t s, int64_t n, double dt, int nstage, const double* w,
+                const double* const* u, const double* const* v, const double* x0,
+                const double* y0, double* x, double* y, double* uc, double* vc);
 
 int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx,
                 const double* sy, const double* ss, const double* sr, int64_t nt,

@@ -11,8 +11,9 @@ import torch
 from ._cabi import VELANDSHEAR, VELANDVORT, VELONLY, TreeOpts, call, make_env
 
 __all__ = ["points_on_points", "panels_on_points", "points_on_panels", "bem_assemble",
-           "bem_factor", "bem_solve", "rk_move", "points_on_points_adjoint", "morton_order",
-           "points_on_points_tree", "points_vorticity", "nearest_distances", "reflect", "clear_inner", "env_for"]
+           "bem_factor", "bem_solve", "rk_move", "rk_advance", "finalize",
+           "points_on_points_adjoint", "morton_order", "points_on_points_tree",
+           "points_vorticity", "nearest_distances", "reflect", "clear_inner", "env_for"]
 
 
 def _ptr(t):
@@ -121,6 +122,31 @@ def rk_move(x, y, us, vs, w, dt):
     call("o2d_hip_rk_move_dev_d", ctypes.byref(env), x.numel(), float(dt), len(us), wv, up, vp,
          _ptr(x), _ptr(y))
     return x, y
+
+
+def rk_advance(x0, y0, us, vs, w, dt, x=None, y=None, combined=False):
+    """The update of rk_move out of place: x = x0 + dt sum w u (new tensors unless x, y are given,
+    which may be x0, y0). combined: also the velocity sum w u, as two more tensors."""
+    x = torch.empty_like(x0) if x is None else x
+    y = torch.empty_like(y0) if y is None else y
+    uc, vc = (torch.empty_like(x0), torch.empty_like(y0)) if combined else (None, None)
+    dev = _check(x0, y0, x, y, *us, *vs)
+    env = env_for(dev)
+    wv = (ctypes.c_double * len(w))(*[float(a) for a in w])
+    up = (ctypes.c_void_p * len(us))(*[u.data_ptr() for u in us])
+    vp = (ctypes.c_void_p * len(vs))(*[v.data_ptr() for v in vs])
+    call("o2d_hip_rk_advance_dev_d", ctypes.byref(env), x.numel(), float(dt), len(us), wv, up, vp,
+         _ptr(x0), _ptr(y0), _ptr(x), _ptr(y), _ptr(uc), _ptr(vc))
+    return (x, y, uc, vc) if combined else (x, y)
+
+
+def finalize(u, v, fs, factor):
+    """In place u = fs[0] + u * factor, v = fs[1] + v * factor."""
+    dev = _check(u, v)
+    env = env_for(dev)
+    call("o2d_hip_finalize_dev_d", ctypes.byref(env), u.numel(), float(fs[0]), float(fs[1]),
+         float(factor), _ptr(u), _ptr(v))
+    return u, v
 
 
 def points_on_points_adjoint(sx, sy, ss, sr, tx, ty, gu, gv, *, core="gauss", out=None):

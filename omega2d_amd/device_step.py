@@ -179,24 +179,26 @@ class Stepper:
         """Finalized velocities of the particles at (x, y) (src/Convection.h:172-243)."""
         if self.body is not None:
             self.body.solve(x, y, self.s, self.fs)
-        u = torch.zeros_like(x)
-        v = torch.zeros_like(x)
+        u, v = torch.zeros((2, *x.shape), dtype=x.dtype, device=x.device)
         dv.points_on_points(x, y, self.s, self.r, x, y, self.r, core=self.core,
                             precision=self.precision, tu=u, tv=v)
         if self.body is not None:
             self.body.add_vels(x, y, u, v)
-        return self.fs[0] + u * FACTOR, self.fs[1] + v * FACTOR
+        return dv.finalize(u, v, self.fs, FACTOR)
 
     def _clear(self, x, y):
         if self.body is not None:
             self.body.clear(x, y, self.s, self.r, self.ips)
 
-    def _moved(self, dt, w, us, vs, x0=None, y0=None):
-        x = (self.x if x0 is None else x0).clone()
-        y = (self.y if y0 is None else y0).clone()
-        dv.rk_move(x, y, us, vs, w, dt)
+    def _moved(self, dt, w, us, vs):
+        x, y = dv.rk_advance(self.x, self.y, us, vs, w, dt)
         self._clear(x, y)
         return x, y
+
+    def _combined(self, dt, w, us, vs):
+        _, _, u, v = dv.rk_advance(self.x, self.y, us, vs, w, dt, self.x, self.y, combined=True)
+        self._clear(self.x, self.y)
+        return u, v
 
     def step(self, dt, order=2):
         """One step of the given order (src/Convection.h:274-303, 390-466, 472-598). Returns
@@ -215,9 +217,7 @@ class Stepper:
             u1, v1 = self.vels(x1, y1)
             self.stages = [(u0, v0), (u1, v1)]
             w = [0.25, 0.75]
-            dv.rk_move(self.x, self.y, [u0, u1], [v0, v1], w, dt)
-            self._clear(self.x, self.y)
-            return w[0] * u0 + w[1] * u1, w[0] * v0 + w[1] * v1
+            return self._combined(dt, w, [u0, u1], [v0, v1])
         if order == 3:
             u0, v0 = self.vels(self.x, self.y)
             x1, y1 = self._moved(0.5 * dt, [1.0], [u0], [v0])
@@ -226,7 +226,5 @@ class Stepper:
             u2, v2 = self.vels(x2, y2)
             self.stages = [(u0, v0), (u1, v1), (u2, v2)]
             w = [2.0 / 9.0, 3.0 / 9.0, 4.0 / 9.0]
-            dv.rk_move(self.x, self.y, [u0, u1, u2], [v0, v1, v2], w, dt)
-            self._clear(self.x, self.y)
-            return (w[0] * u0 + w[1] * u1 + w[2] * u2, w[0] * v0 + w[1] * v1 + w[2] * v2)
+            return self._combined(dt, w, [u0, u1, u2], [v0, v1, v2])
         raise ValueError("order must be 1, 2 or 3")

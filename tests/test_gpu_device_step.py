@@ -106,3 +106,27 @@ def test_free_particle_steps_match_oracle(order, precision):
     tol = 1e-14 if precision == "fp64" else 1e-5 * dt * np.max(np.hypot(eu, ev))
     assert np.max(np.abs(x.cpu().numpy() - ex)) <= tol
     assert np.max(np.abs(y.cpu().numpy() - ey)) <= tol
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1000])
+@pytest.mark.parametrize("w", [[1.0], [0.25, 0.75], [2 / 9, 3 / 9, 4 / 9]])
+def test_advance_and_finalize_round_as_separate_operations(n, w):
+    # the same IEEE operations as torch's separate ones, so equal bit for bit
+    rng = np.random.default_rng(n)
+    x, y, *uv = [T(rng.normal(size=n)) for _ in range(2 + 2 * len(w))]
+    us, vs = uv[0::2], uv[1::2]
+    x0, y0 = x.clone(), y.clone()
+    ax, ay, cu, cv = ds.dv.rk_advance(x, y, us, vs, w, 0.01, combined=True)
+    assert torch.equal(x, x0) and torch.equal(y, y0)
+    for c, parts in ((cu, us), (cv, vs)):
+        ref = w[0] * parts[0]
+        for a, p in zip(w[1:], parts[1:]):
+            ref = ref + a * p
+        assert torch.equal(c, ref)
+    ds.dv.rk_move(x0, y0, us, vs, w, 0.01)
+    assert torch.equal(ax, x0) and torch.equal(ay, y0)
+    bx, by = ds.dv.rk_advance(x, y, us, vs, w, 0.01, x, y)
+    assert bx is x and by is y and torch.equal(x, x0) and torch.equal(y, y0)
+    u, v = us[0].clone(), vs[0].clone()
+    ds.dv.finalize(u, v, (1.5, -0.25), ds.FACTOR)
+    assert torch.equal(u, 1.5 + us[0] * ds.FACTOR) and torch.equal(v, -0.25 + vs[0] * ds.FACTOR)
