@@ -4,8 +4,8 @@
 // of pairs ran as a merge sort at these sizes (a block sort and up to sixteen merge launches,
 // 110 us for 200k or 1M points, 45 us for 10k), after three or four launches that made the keys.
 //
-// Up to kSmallMax keys one workgroup does everything in one launch, box included. Beyond, least
-// significant digits first, 8 bits a pass: the box (one launch), the keys with the first digit's
+// Up to kRankMax keys one launch does everything, box included, by counting for each key the keys
+// that go before it (rank_kernel). Beyond, least significant digits first, 8 bits a pass: the box (one launch), the keys with the first digit's
 // tile histograms (one launch), then one launch per digit. A scatter launch sums the
 // histogram rows of the tiles before its own (every tile reads all rows from cache, which at
 // kMaxTiles rows is a fraction of the launch's own cost), ranks its keys within the tile by
@@ -33,9 +33,9 @@ constexpr int kSW = kST / 64;
 constexpr int kDigits = 256;
 constexpr int kMaxTiles = 512;
 constexpr int kCountItems = 2;   // keys per thread up to which a pass counts the next digit
-constexpr int kSmallT = 1024;    // threads of the one-workgroup sort
-constexpr int kSmallW = kSmallT / 64;
-constexpr int kSmallMax = 4 * kSmallT;
+constexpr int kRankT = 1024;     // threads of a rank workgroup
+constexpr int kRankW = kRankT / 64;
+constexpr int kRankMax = 12 * kRankT;
 
 __device__ __forceinline__ uint32_t spread16(uint32_t v) {  // bits of v to the even positions
   v &= 0xFFFFu;
@@ -332,90 +332,79 @@ __global__ __launch_bounds__(kST) void scatter_kernel(int64_t n, int ntiles, int
   }
 }
 
-// the whole order in one workgroup, n <= ITEMS * kSmallT: keys and values pass through LDS
-// between digits
-template <int KIND, int ITEMS>
-__global__ __launch_bounds__(kSmallT) void small_kernel(KeyGen g, int n, int npass,
-                                                        uint32_t* __restrict__ keys_out,
-                                                        uint32_t* __restrict__ vals_out) {
-  __shared__ uint32_t sk[kSmallT * ITEMS], sv[kSmallT * ITEMS];
-  __shared__ uint32_t cnt[kSmallW][kDigits];
-  __shared__ uint32_t part[kDigits / 64];
-  __shared__ Box sm[kSmallW];
+// the whole order in one launch, n <= ITEMS * kRankT, by the place of each key: the keys below it,
+// and the equal ones before it. Every workgroup makes all keys in LDS and places EACH of them, one to
+// a lane; its waves share the blocks of 64 keys to compare with, and the 64 / EACH lanes with the same
+// key share a block. Bound by latency up to 4,096 keys (7 us is the launch, two dependent passes over
+// the points and their box), beyond by the integer units and LDS together: 8.4 us at 1,531 keys,
+// 11.9 at 4,096, 18.3 at 8,192, 25.3 at 10,000 and 28.9 at 12,288. A one-workgroup radix sort in LDS took 15.4 us at
+// 1,531 (four digits, three barriers each), the six launches of the tiled passes 30 us and their gaps
+// at 10,000; here 16,384 keys take 37 us, and n^2 comparisons no longer pay. Comparing 64 keys with
+// one scalar key and counting the mask's bits took 40 us at 10,000 (scalar registers), two keys a lane
+// 28.
+template <int KIND, int ITEMS, int EACH>
+__global__ __launch_bounds__(kRankT) void rank_kernel(KeyGen g, int n,
+                                                      uint32_t* __restrict__ keys_out,
+                                                      uint32_t* __restrict__ vals_out) {
+  __shared__ __align__(16) uint32_t sk[kRankT * ITEMS];
+  __shared__ uint32_t cnt[kRankW][64];
+  __shared__ Box sm[kRankW];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   Box b = empty_box();
   if (KIND != kNode && g.bbox) {
-    for (int i = t; i < n; i += kSmallT) grow(b, g.x[i], g.y[i], g.x[i], g.y[i]);
-    b = block_box<kSmallW>(b, sm);
+#pragma unroll 4
+    for (int k = 0; k < ITEMS; ++k) {
+      const int i = t + k * kRankT;
+      if (i < n) grow(b, g.x[i], g.y[i], g.x[i], g.y[i]);
+    }
+    b = block_box<kRankW>(b, sm);
   }
   double x0, y0, inv;
   key_frame<KIND>(g, b, x0, y0, inv);
-  const int first = wave * (64 * ITEMS) + lane;
-  uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
-#pragma unroll
+#pragma unroll 4
   for (int k = 0; k < ITEMS; ++k) {
-    const int i = first + 64 * k;
-    val[k] = (uint32_t)i;
-    key[k] = i < n ? make_key<KIND>(g, b, x0, y0, inv, i) : 0u;
+    const int i = t + k * kRankT;
+    // the padding goes after every key: it is only compared with keys before it, by <
+    sk[i] = i < n ? make_key<KIND>(g, b, x0, y0, inv, i) : 0xFFFFFFFFu;
   }
-  const unsigned long long below = (1ull << lane) - 1ull;
-  for (int p = 0; p < npass; ++p) {
-    const int shift = 8 * p;
-    for (int d = lane; d < kDigits; d += 64) cnt[wave][d] = 0;
-    wave_sync();
+  __syncthreads();
+  const int i = blockIdx.x * EACH + lane % EACH, nblk = (n + 63) / 64;
+  const int own = (blockIdx.x * EACH) / 64, part = (lane / EACH) * EACH;  // own: the keys' block
+  const uint32_t mine = sk[i];
+  uint32_t c = 0;
+  for (int blk = wave; blk < nblk; blk += kRankW) {
+    const int first = blk * 64 + part;
+    const uint4* q = reinterpret_cast<const uint4*>(sk + first);
+    if (blk < own) {
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const bool valid = first + 64 * k < n;
-      const uint32_t d = (key[k] >> shift) & (kDigits - 1);
-      const unsigned long long m = match8(d, __ballot(valid));
-      const uint32_t had = cnt[wave][d];
-      rank[k] = had + __popcll(m & below);
-      wave_sync();
-      if (valid && (m & below) == 0) cnt[wave][d] = had + __popcll(m);
-      wave_sync();
-    }
-    __syncthreads();
-    uint32_t total = 0;
-    if (t < kDigits) {
-#pragma unroll
-      for (int w = 0; w < kSmallW; ++w) {
-        const uint32_t c = cnt[w][t];
-        cnt[w][t] = total;
-        total += c;
+      for (int k = 0; k < EACH / 4; ++k) {
+        const uint4 o = q[k];
+        c += (o.x <= mine) + (o.y <= mine) + (o.z <= mine) + (o.w <= mine);
       }
-    }
-    const uint32_t start = digit_scan(total, part);
-    if (t < kDigits) {
+    } else if (blk > own) {
 #pragma unroll
-      for (int w = 0; w < kSmallW; ++w) cnt[w][t] += start;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      if (first + 64 * k < n) {
-        const uint32_t dst = cnt[wave][(key[k] >> shift) & (kDigits - 1)] + rank[k];
-        sk[dst] = key[k];
-        sv[dst] = val[k];
+      for (int k = 0; k < EACH / 4; ++k) {
+        const uint4 o = q[k];
+        c += (o.x < mine) + (o.y < mine) + (o.z < mine) + (o.w < mine);
       }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const int i = first + 64 * k;
-      if (i < n) {
-        key[k] = sk[i];
-        val[k] = sv[i];
+    } else {
+#pragma unroll 4
+      for (int k = 0; k < EACH; ++k) {
+        const uint32_t o = sk[first + k];
+        c += o < mine || (o == mine && first + k < i);
       }
     }
   }
+  cnt[wave][lane] = c;
+  __syncthreads();
+  if (t >= EACH || i >= n) return;
+  c = 0;
 #pragma unroll
-  for (int k = 0; k < ITEMS; ++k) {
-    const int i = first + 64 * k;
-    if (i < n) {
-      if (keys_out) keys_out[i] = key[k];
-      vals_out[i] = val[k];
-    }
-  }
+  for (int w = 0; w < kRankW; ++w)
+#pragma unroll
+    for (int p = 0; p < 64; p += EACH) c += cnt[w][lane + p];
+  if (keys_out) keys_out[c] = mine;
+  vals_out[c] = (uint32_t)i;
 }
 
 __global__ __launch_bounds__(kBoxBlock) void iota_kernel(int64_t n, uint32_t* __restrict__ v) {
@@ -423,14 +412,18 @@ __global__ __launch_bounds__(kBoxBlock) void iota_kernel(int64_t n, uint32_t* __
   if (i < n) v[i] = (uint32_t)i;
 }
 
+// 16 keys a workgroup while that leaves no more than one for each of 256 compute units, then 32 or 64
+// (each workgroup makes all keys: at 8,192 keys 16 took 25.5 us and 32 take 18.3)
 template <int KIND>
-void launch_small(hipStream_t s, const KeyGen& g, int n, int npass, uint32_t* ko, uint32_t* vo) {
-  if (n <= kSmallT)
-    small_kernel<KIND, 1><<<1, kSmallT, 0, s>>>(g, n, npass, ko, vo);
-  else if (n <= 2 * kSmallT)
-    small_kernel<KIND, 2><<<1, kSmallT, 0, s>>>(g, n, npass, ko, vo);
+void launch_rank(hipStream_t s, const KeyGen& g, int n, uint32_t* ko, uint32_t* vo) {
+  if (n <= 2 * kRankT)
+    rank_kernel<KIND, 2, 16><<<(n + 15) / 16, kRankT, 0, s>>>(g, n, ko, vo);
+  else if (n <= 4 * kRankT)
+    rank_kernel<KIND, 4, 16><<<(n + 15) / 16, kRankT, 0, s>>>(g, n, ko, vo);
+  else if (n <= 8 * kRankT)
+    rank_kernel<KIND, 8, 32><<<(n + 31) / 32, kRankT, 0, s>>>(g, n, ko, vo);
   else
-    small_kernel<KIND, 4><<<1, kSmallT, 0, s>>>(g, n, npass, ko, vo);
+    rank_kernel<KIND, 12, 64><<<(n + 63) / 64, kRankT, 0, s>>>(g, n, ko, vo);
 }
 
 template <int ITEMS>
@@ -490,12 +483,12 @@ int sort_order(Device* d, hipStream_t s, Workspace* ws, int64_t n, const KeyGen&
                uint32_t* keys_out, uint32_t* order_out, bool want_keys) {
   if (n <= 0) return 0;
   const int npass = (bits + 7) / 8;
-  if (n <= kSmallMax) {
+  if (n <= kRankMax) {
     uint32_t* ko = want_keys ? keys_out : nullptr;
     switch (g.kind) {
-      case kMorton32: launch_small<kMorton32>(s, g, (int)n, npass, ko, order_out); break;
-      case kMorton16: launch_small<kMorton16>(s, g, (int)n, npass, ko, order_out); break;
-      default: launch_small<kNode>(s, g, (int)n, npass, ko, order_out); break;
+      case kMorton32: launch_rank<kMorton32>(s, g, (int)n, ko, order_out); break;
+      case kMorton16: launch_rank<kMorton16>(s, g, (int)n, ko, order_out); break;
+      default: launch_rank<kNode>(s, g, (int)n, ko, order_out); break;
     }
     O2D_LAUNCH_CHECK();
     return 0;

@@ -1,7 +1,8 @@
 """The device key sort against numpy's stable argsort of the oracle's Morton keys, bit-exact, at
-the edges of its ranges: one workgroup (to 4,096 keys, in steps of 1,024), the tiled passes with
-2, 4, 8 and 16 keys per thread (from 4,097, 65,537, 262,145 and 1,048,577) and the library sort
-past 4,194,304 keys; spread keys, keys that share their high digits, and one key throughout."""
+the edges of its ranges: ranks by comparison (to 12,288 keys, with 2, 4, 8 and 12 keys per thread,
+16, 32 or 64 ranks per workgroup), the tiled passes with 2, 4, 8 and 16 keys per thread (from 12,289,
+65,537, 262,145 and 1,048,577) and the library sort past 4,194,304 keys; spread keys, keys that
+share their high digits, and one key throughout."""
 import numpy as np
 import pytest
 import torch
@@ -13,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("spread", ["wide", "clustered", "single"])
-@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 2049, 4096, 4097, 65536, 65537, 262145, 1048577,
+@pytest.mark.parametrize("n", [1, 15, 63, 65, 1024, 1025, 2048, 2049, 4096, 4097, 8191, 8192, 8193,
+                               12287, 12288, 12289, 65536, 65537, 262145, 1048577,
                                4194305])
 def test_morton_order_is_the_stable_order(n, spread):
     rng = np.random.default_rng(n)
