@@ -1,28 +1,23 @@
 // vorticity.hip - Gaussian vorticity of particles at targets, points_affect_points_vorticity
 // (src/InfluenceVort.h:47-126, the x86 loop :103-117):
 //   tw_i += sum_j 2 s_j exp(-d_ij^2 / r_j^2) / r_j^2      (unscaled; finalize_vels adds 1/2pi)
-// in fp64. Sources are staged through LDS as (x, y, 1/r^2, 2 s/r^2); each lane owns two
-// targets. A pair with d^2/r^2 > 746 contributes exactly +-0 (exp underflows to 0 in double), so
-// its exponential is skipped without changing the sum. Few targets split the source range into
-// chunks whose fp64 partials are summed in chunk order. With many sources and targets both go
-// in Morton order: a tile of 256 sources carries the box of its positions and its smallest
-// 1/r^2, each group of 256 targets (and each wave's 64) has a compact box, and a tile whose
-// every pair with a group lies beyond the underflow bound (by a margin far above the rounding
-// of both tests) is skipped for that group; it adds only +-0 terms. The exponential is a
-// table-driven exp(-x) on [0, 746). The Morton order changes the order of the fp64 additions, so sums move by
-// rounding only. A NaN position or radius adds NaN, as in the reference (its tile and its
-// targets' group are never skipped); a non-finite strength or a zero radius beyond the bound
-// adds nothing, where the reference's inf*0 gives NaN.
-#include <cfloat>
+// in fp64. A pair with d^2/r^2 > 746 contributes exactly +-0 (exp underflows to 0 in double), so
+// its exponential is skipped without changing the sum. The exponential is a table-driven exp(-x) on
+// [0, 746).
+//
+// Sources and targets go in Morton order, and a group of 16 targets meets only the boxes of 32 sources
+// that its own box can reach. The order is fixed, so sums are reproducible. (A kernel without orders
+// or boxes, two targets a lane, took 58 us at 1,000 particles against 22, 59 at 4,000 against 32, 45 for
+// 200 on 50,000 points against 41; it was faster for 200,000 on 50, 108 against 115, and where the
+// radii reach across the whole domain, 3,000 on 200,000: 442 against 521, 129 at ordinary radii.)
+//
+// A NaN position or radius adds NaN, as in the reference (its tile and its targets' group are never
+// skipped); a non-finite strength or a zero radius beyond the bound adds nothing, where the
+// reference's inf*0 gives NaN.
+#include <algorithm>
 
 #include "nbody.h"
 #include "o2d_runtime.h"
-
-// workgroups per CU the source chunks aim for (128: 17.1 -> 13.8 ms for 200k particles on
-// themselves, against 8)
-#ifndef O2D_WANT_VORT
-#define O2D_WANT_VORT 128
-#endif
 
 namespace o2d {
 
@@ -30,16 +25,20 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kTile = 256;
-constexpr int kTpl = 2;
 constexpr double kUnderflow = 746.0;  // exp(-x) == 0 in double for every x above this
-constexpr int64_t kPruneSources = 4096, kPruneTargets = 1024;  // from here the sort pays
-// pruned launch: source tiles per chunk, and the cap on the chunk partials' bytes
-#ifndef O2D_VORT_PRUNED_TILES
-#define O2D_VORT_PRUNED_TILES 2
-#endif
-constexpr int64_t kPartialBytes = int64_t(1) << 30;
+constexpr int kSub = 32;                   // sources per box of a tile
+constexpr int kSubs = kTile / kSub;
+constexpr int kGroup = 16;                 // targets per wave of vort_near_kernel
+constexpr int kNearT = 256;                // its threads
+constexpr int kNearTargets = 32;           // its targets: two groups, two waves each
+// rows of tiles that its grid is cut into: kNearWgs workgroups per CU, and at least kNearRows (the
+// workgroups of dense regions last longest, and without rows the launch waits for them): 200,000 wake
+// particles take 394 us a call with one row, 347 with two, 330 with four; 100,000 209, 173 (two)
+// and 148 (three); 20,000 51 with 12 workgroups per CU and 65 with 48
+constexpr int64_t kNearWgs = 12, kNearRows = 3;
+constexpr int64_t kPartialBytes = int64_t(1) << 30;  // the cap on the rows' partial sums
 
-struct VSrc {
+struct alignas(16) VSrc {
   double x, y, rr, c;  // position, 1/r^2, 2 s / r^2
 };
 
@@ -95,259 +94,213 @@ __device__ __forceinline__ VSrc vsrc_of(double x, double y, double s, double r) 
   return VSrc{x, y, rr, 2.0 * s * rr};
 }
 
-// the sources in the order sorder as staged records, and per tile of kTile the box of their
-// positions and their smallest 1/r^2: tbox[5 t ...] = (x min, x max, y min, y max, rr min).
-// One workgroup per tile. A NaN position or radius makes the tile's box unbounded.
+// the smallest and largest of v over aligned groups of 32 lanes
+__device__ __forceinline__ double min32(double v) {
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
+  return v;
+}
+__device__ __forceinline__ double max32(double v) { return -min32(-v); }
+
+// LDS writes of this wave visible to its own later reads, and no compiler reordering across
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A box of source positions with their smallest 1/r^2. A NaN position or radius makes it unbounded.
+struct VBox {
+  double x0, x1, y0, y1, rr;
+};
+
+// the sources in the order sorder as staged records, the box of every kSub of them (sub) and of
+// every tile of kTile (tile), padded to whole tiles with the last source at zero strength. One
+// workgroup per tile.
 __global__ __launch_bounds__(kBlock) void vort_gather_kernel(int64_t ns, const double* __restrict__ sx,
                                                              const double* __restrict__ sy,
                                                              const double* __restrict__ ss,
                                                              const double* __restrict__ sr,
                                                              const uint32_t* __restrict__ sorder,
                                                              VSrc* __restrict__ vs,
-                                                             double* __restrict__ tbox) {
-  __shared__ double sm[5][kBlock];
+                                                             VBox* __restrict__ sub,
+                                                             VBox* __restrict__ tile) {
+  static_assert(kTile == kBlock && kSub == 32, "a tile per workgroup, two boxes per wave");
+  __shared__ VBox sm[kSubs];
   const int t = threadIdx.x;
   const int64_t g = (int64_t)blockIdx.x * kBlock + t;
-  double x0 = DBL_MAX, x1 = -DBL_MAX, y0 = DBL_MAX, y1 = -DBL_MAX, r0 = DBL_MAX;
-  if (g < ns) {
-    const int64_t j = sorder ? (int64_t)sorder[g] : g;
-    const VSrc q = vsrc_of(sx[j], sy[j], ss[j], sr[j]);
-    vs[g] = q;
-    x0 = x1 = q.x;
-    y0 = y1 = q.y;
-    r0 = q.rr;
-    if (!(q.x == q.x) || !(q.y == q.y) || !(q.rr == q.rr)) {
-      x0 = y0 = -INFINITY;
-      x1 = y1 = INFINITY;
-      r0 = 0.0;
-    }
+  const int64_t j = sorder[g < ns ? g : ns - 1];
+  VSrc q = vsrc_of(sx[j], sy[j], ss[j], sr[j]);
+  if (g >= ns) q.c = 0.0;
+  vs[g] = q;
+  const bool bad = !(q.x == q.x) || !(q.y == q.y) || !(q.rr == q.rr);
+  VBox b;
+  b.x0 = min32(bad ? -INFINITY : q.x);
+  b.x1 = max32(bad ? INFINITY : q.x);
+  b.y0 = min32(bad ? -INFINITY : q.y);
+  b.y1 = max32(bad ? INFINITY : q.y);
+  b.rr = min32(bad ? 0.0 : q.rr);
+  if ((t & (kSub - 1)) == 0) {
+    sm[t / kSub] = b;
+    sub[(int64_t)blockIdx.x * kSubs + t / kSub] = b;
   }
-  sm[0][t] = x0;
-  sm[1][t] = x1;
-  sm[2][t] = y0;
-  sm[3][t] = y1;
-  sm[4][t] = r0;
   __syncthreads();
-  for (int w = kBlock / 2; w > 0; w >>= 1) {
-    if (t < w) {
-      sm[0][t] = fmin(sm[0][t], sm[0][t + w]);
-      sm[1][t] = fmax(sm[1][t], sm[1][t + w]);
-      sm[2][t] = fmin(sm[2][t], sm[2][t + w]);
-      sm[3][t] = fmax(sm[3][t], sm[3][t + w]);
-      sm[4][t] = fmin(sm[4][t], sm[4][t + w]);
-    }
-    __syncthreads();
+  if (t != 0) return;
+  for (int k = 1; k < kSubs; ++k) {
+    b.x0 = fmin(b.x0, sm[k].x0);
+    b.x1 = fmax(b.x1, sm[k].x1);
+    b.y0 = fmin(b.y0, sm[k].y0);
+    b.y1 = fmax(b.y1, sm[k].y1);
+    b.rr = fmin(b.rr, sm[k].rr);
   }
-  if (t < 5) tbox[5 * blockIdx.x + t] = sm[t][0];
+  tile[blockIdx.x] = b;
 }
 
-// the box of each kBlock consecutive targets in the order torder (the first or the second
-// targets of one vort_kernel workgroup's lanes): gbox[4 g ...] = (x min, x max, y min, y max).
-// One workgroup per group; a NaN position makes the group's box unbounded.
-__global__ __launch_bounds__(kBlock) void vort_target_box_kernel(int64_t nt,
-                                                                 const double* __restrict__ tx,
-                                                                 const double* __restrict__ ty,
-                                                                 const uint32_t* __restrict__ torder,
-                                                                 double* __restrict__ gbox) {
-  __shared__ double sm[4][kBlock];
-  const int t = threadIdx.x;
-  const int64_t p = (int64_t)blockIdx.x * kBlock + t;
-  double x0 = DBL_MAX, x1 = -DBL_MAX, y0 = DBL_MAX, y1 = -DBL_MAX;
-  if (p < nt) {
-    const int64_t i = torder[p];
-    x0 = x1 = tx[i];
-    y0 = y1 = ty[i];
-    if (!(x0 == x0) || !(y0 == y0)) {
-      x0 = y0 = -INFINITY;
-      x1 = y1 = INFINITY;
-    }
+// true unless every pair of source box b and target box (x0, x1, y0, y1) lies beyond the underflow
+// bound, by a relative margin of 2^-40, far above the rounding of this test and of a pair's own
+__device__ __forceinline__ bool box_near(const VBox& b, double x0, double x1, double y0, double y1) {
+  const double dx = fmax(0.0, fmax(b.x0 - x1, x0 - b.x1));
+  const double dy = fmax(0.0, fmax(b.y0 - y1, y0 - b.y1));
+  return !((dx * dx + dy * dy) * b.rr * (1.0 - 0x1p-40) > kUnderflow);
+}
+
+// Targets and sources in Morton order. Bound by the fp64 vector units: an exponential is 20 of a
+// pair's 26 operations, and the boxes decide how many pairs that add exactly 0 are met. A workgroup
+// takes 32 targets; wave w holds group w % 2 of 16 of them, each in four lanes that take every fourth
+// source, and the two waves of a group take the even and the odd boxes. The source tiles that the
+// workgroup's box reaches are listed 256 at a time (in order), and a wave takes the boxes of 32 sources
+// in them that its own 16 targets reach, without waiting for the others. For 200,000 wake particles
+// (radius 0.005, 1.65e8 pairs within the bound) that is 4.0e8 pairs; 64 targets against tiles of 256 were
+// 9.7e8. 735 us and 40 for the sum over chunks -> 319 us and 8. Staging whole tiles between
+// barriers took 548 us, exponentials without the branch around them 60% longer.
+//
+// blockIdx.y takes the listed tiles y, y + gridDim.y, ...; out: tw by torder when gridDim.y is 1, else
+// the partial sums part[y nt + p] of the target at position p.
+__global__ __launch_bounds__(kNearT) void vort_near_kernel(int64_t nt, const double* __restrict__ tx,
+                                                           const double* __restrict__ ty,
+                                                           const uint32_t* __restrict__ torder,
+                                                           int64_t ntiles, const VSrc* __restrict__ vs,
+                                                           const VBox* __restrict__ sub,
+                                                           const VBox* __restrict__ tbox,
+                                                           double* __restrict__ tw,
+                                                           double* __restrict__ part) {
+  constexpr int kWaves = kNearT / 64, kGroups = kNearTargets / kGroup, kLanes = 64 / kGroup;
+  static_assert(kWaves == 2 * kGroups && kLanes == 4, "two waves a group, four lanes a target");
+  static_assert(sizeof(VSrc) * kSub == 64 * sizeof(double2), "a box's sources are one load a lane");
+  __shared__ VSrc staged[kWaves][kSub];
+  __shared__ double e2t[64];  // kExp2Tab
+  __shared__ double gb[kWaves][4];
+  __shared__ uint32_t list[kNearT], found[kWaves];
+  __shared__ double sum[kGroups][kGroup];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, group = wave % kGroups;
+  const int half = wave / kGroups, q4 = lane / kGroup;
+  VSrc* mine = staged[wave];
+  if (t < 64) e2t[t] = kExp2Tab[t];
+  const int64_t p = (int64_t)blockIdx.x * kNearTargets + group * kGroup + (lane & (kGroup - 1));
+  const uint32_t o = torder[p < nt ? p : nt - 1];
+  const double px = tx[o], py = ty[o];
+  // the group's box, and the workgroup's (a NaN position: unbounded)
+  const bool bad = !(px == px) || !(py == py);
+  double x0 = bad ? -INFINITY : px, x1 = bad ? INFINITY : px;
+  double y0 = bad ? -INFINITY : py, y1 = bad ? INFINITY : py;
+#pragma unroll
+  for (int s = kGroup / 2; s > 0; s >>= 1) {
+    x0 = fmin(x0, __shfl_xor(x0, s, 64));
+    x1 = fmax(x1, __shfl_xor(x1, s, 64));
+    y0 = fmin(y0, __shfl_xor(y0, s, 64));
+    y1 = fmax(y1, __shfl_xor(y1, s, 64));
   }
-  sm[0][t] = x0;
-  sm[1][t] = x1;
-  sm[2][t] = y0;
-  sm[3][t] = y1;
+  if (lane == 0) {
+    gb[wave][0] = x0;
+    gb[wave][1] = x1;
+    gb[wave][2] = y0;
+    gb[wave][3] = y1;
+  }
   __syncthreads();
-  for (int w = kBlock / 2; w > 0; w >>= 1) {
-    if (t < w) {
-      sm[0][t] = fmin(sm[0][t], sm[0][t + w]);
-      sm[1][t] = fmax(sm[1][t], sm[1][t + w]);
-      sm[2][t] = fmin(sm[2][t], sm[2][t + w]);
-      sm[3][t] = fmax(sm[3][t], sm[3][t + w]);
-    }
+  double wx0 = gb[0][0], wx1 = gb[0][1], wy0 = gb[0][2], wy1 = gb[0][3];
+  for (int k = 1; k < kGroups; ++k) {
+    wx0 = fmin(wx0, gb[k][0]);
+    wx1 = fmax(wx1, gb[k][1]);
+    wy0 = fmin(wy0, gb[k][2]);
+    wy1 = fmax(wy1, gb[k][3]);
+  }
+  double acc = 0.0;
+  for (int64_t base = 0; base < ntiles; base += (int64_t)kNearT * gridDim.y) {
+    // the next kNearT of this row's tiles
+    const int64_t it = base + (int64_t)t * gridDim.y + blockIdx.y;
+    bool near = it < ntiles;
+    if (near) near = box_near(tbox[it], wx0, wx1, wy0, wy1);
+    const unsigned long long m = __ballot(near);
+    if (lane == 0) found[wave] = __popcll(m);
     __syncthreads();
-  }
-  if (t < 4) gbox[4 * blockIdx.x + t] = sm[t][0];
-}
-
-// true unless every pair of source tile box b (with its smallest 1/r^2) and target group box g
-// lies beyond the underflow bound, by a relative margin of 2^-40
-__device__ __forceinline__ bool tile_near(const double* b, const double* g) {
-  const double dx = fmax(0.0, fmax(b[0] - g[1], g[0] - b[1]));
-  const double dy = fmax(0.0, fmax(b[2] - g[3], g[2] - b[3]));
-  return !((dx * dx + dy * dy) * b[4] * (1.0 - 0x1p-40) > kUnderflow);
-}
-
-// vs/tbox null: the sources in input order from sx..sr; else the staged records in Morton
-// order with their tile boxes, gbox the boxes of the target groups of kBlock (a workgroup holds
-// two: its lanes' first and second targets) and torder the targets' order: the target at
-// position p is torder[p] and chunk partials are kept by position (vort_reduce_kernel maps
-// them). A tile is skipped for a group it cannot reach, for both groups at once when neither,
-// and, after staging, by each wave for its own 64 first or second targets that it cannot reach;
-// a workgroup whose chunk reaches neither group writes no partials and ends. The grid is one
-// dimensional: block b takes (target workgroup, chunk) number (b * perm) % (twgs * nchunk), row
-// major by chunk, so that the few (workgroup, chunk) pairs near the Morton diagonal that hold
-// work are spread over the whole dispatch. flag[workgroup * nchunk8 + chunk] says whether its
-// partials were written (nchunk8: the chunk count rounded up to 8; the padding is never read).
-__global__ __launch_bounds__(kBlock) void vort_kernel(int64_t ns, const double* __restrict__ sx,
-                                                      const double* __restrict__ sy,
-                                                      const double* __restrict__ ss,
-                                                      const double* __restrict__ sr, int64_t nt,
-                                                      const double* __restrict__ tx,
-                                                      const double* __restrict__ ty,
-                                                      int64_t chunk, double* __restrict__ out,
-                                                      uint8_t* __restrict__ flag, int64_t twgs,
-                                                      int64_t nchunk8,
-                                                      int64_t perm, int direct,
-                                                      const VSrc* __restrict__ vs,
-                                                      const double* __restrict__ tbox,
-                                                      const double* __restrict__ gbox,
-                                                      const uint32_t* __restrict__ torder) {
-  static_assert(kTpl == 2, "a workgroup holds two target groups");
-  __shared__ VSrc tile[kTile];
-  __shared__ double e2t[64];  // kExp2Tab, visible after the first tile's barrier
-  if (threadIdx.x < 64) e2t[threadIdx.x] = kExp2Tab[threadIdx.x];
-  const int64_t cell = ((int64_t)blockIdx.x * perm) % ((int64_t)gridDim.x);
-  const int64_t bx = cell % twgs, by = cell / twgs;
-  const int64_t j0 = by * chunk;
-  const int64_t j1 = (j0 + chunk < ns) ? j0 + chunk : ns;
-  double px[kTpl], py[kTpl], acc[kTpl];
-  int64_t ti[kTpl];
-#pragma unroll
-  for (int t = 0; t < kTpl; ++t) ti[t] = (bx * kTpl + t) * kBlock + threadIdx.x;
-  // the workgroup's two target groups (the second may hold no target)
-  const double* g0 = gbox ? gbox + 4 * (2 * bx) : nullptr;
-  const double* g1 = (gbox && (2 * bx + 1) * kBlock < nt) ? g0 + 4 : nullptr;
-  if (tbox) {  // uniform over the workgroup: chunks are whole tiles
-    bool any = false;
-    for (int64_t base = j0; base < j1 && !any; base += kTile) {
-      const double* b = tbox + 5 * (base / kTile);
-      any = tile_near(b, g0) || (g1 && tile_near(b, g1));
+    uint32_t at = 0, total = 0;
+    for (int w = 0; w < kWaves; ++w) {
+      at += w < wave ? found[w] : 0u;
+      total += found[w];
     }
-    if (!any) {
-      if (!direct && threadIdx.x == 0) flag[bx * nchunk8 + by] = 0;
-      return;
-    }
-  }
-  if (!direct && threadIdx.x == 0) flag[bx * nchunk8 + by] = 1;
-#pragma unroll
-  for (int t = 0; t < kTpl; ++t) {
-    const bool ok = ti[t] < nt;
-    const int64_t i = ok ? (torder ? (int64_t)torder[ti[t]] : ti[t]) : 0;
-    px[t] = ok ? tx[i] : 0.0;
-    py[t] = ok ? ty[i] : 0.0;
-    acc[t] = 0.0;
-  }
-  // each wave's box of its 64 first and 64 second targets (a NaN position: unbounded)
-  double wb[kTpl][4];
-#pragma unroll
-  for (int t = 0; t < kTpl; ++t) {
-    const bool ok = ti[t] < nt;
-    const bool bad = ok && (!(px[t] == px[t]) || !(py[t] == py[t]));
-    double x0 = ok ? px[t] : DBL_MAX, x1 = ok ? px[t] : -DBL_MAX;
-    double y0 = ok ? py[t] : DBL_MAX, y1 = ok ? py[t] : -DBL_MAX;
-    if (bad) {
-      x0 = y0 = -INFINITY;
-      x1 = y1 = INFINITY;
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-      x0 = fmin(x0, __shfl_xor(x0, o));
-      x1 = fmax(x1, __shfl_xor(x1, o));
-      y0 = fmin(y0, __shfl_xor(y0, o));
-      y1 = fmax(y1, __shfl_xor(y1, o));
-    }
-    wb[t][0] = x0;
-    wb[t][1] = x1;
-    wb[t][2] = y0;
-    wb[t][3] = y1;
-  }
-  for (int64_t base = j0; base < j1; base += kTile) {
-    const int n = (int)((j1 - base) < kTile ? (j1 - base) : kTile);
-    bool k0 = true, k1 = true;
-    if (tbox) {
-      const double* b = tbox + 5 * (base / kTile);
-      k0 = tile_near(b, g0);
-      k1 = g1 && tile_near(b, g1);
-      if (!k0 && !k1) continue;
-    }
+    if (near) list[at + __popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)it;
     __syncthreads();
-    if ((int)threadIdx.x < n) {
-      const int64_t j = base + threadIdx.x;
-      tile[threadIdx.x] = vs ? vs[j] : vsrc_of(sx[j], sy[j], ss[j], sr[j]);
-    }
-    __syncthreads();
-    // the same test for this wave's targets: uniform over the wave, no barrier below
-    if (tbox) {
-      const double* b = tbox + 5 * (base / kTile);
-      k0 = k0 && tile_near(b, wb[0]);
-      k1 = k1 && tile_near(b, wb[1]);
-    }
-    if (k0 && k1) {
-      for (int k = 0; k < n; ++k) {
-        const VSrc q = tile[k];
+    // 64 boxes of eight listed tiles at a time; the two waves of a group take the even and the odd
+    // ones. A box's sources pass through this wave's piece of LDS, the next box's loads under way.
+    for (uint32_t l0 = 0; l0 < total; l0 += 64 / kSubs) {
+      const uint32_t l = l0 + lane / kSubs;
+      uint32_t e = 0;
+      bool reach = false;
+      if (l < total && (lane & 1) == half) {
+        e = list[l] * kSubs + lane % kSubs;
+        reach = box_near(sub[e], x0, x1, y0, y1);
+      }
+      unsigned long long todo = __ballot(reach);
+      double2 next = make_double2(0.0, 0.0);
+      if (todo) {
+        const uint32_t f = __builtin_amdgcn_readlane(e, __builtin_ctzll(todo));
+        next = reinterpret_cast<const double2*>(vs + (int64_t)f * kSub)[lane];
+      }
+      while (todo) {
+        todo &= todo - 1;
+        wave_sync();
+        reinterpret_cast<double2*>(mine)[lane] = next;
+        wave_sync();
+        if (todo) {
+          const uint32_t f = __builtin_amdgcn_readlane(e, __builtin_ctzll(todo));
+          next = reinterpret_cast<const double2*>(vs + (int64_t)f * kSub)[lane];
+        }
 #pragma unroll
-        for (int t = 0; t < kTpl; ++t) {
-          const double dx = px[t] - q.x, dy = py[t] - q.y;
-          const double x = (dx * dx + dy * dy) * q.rr;
-          if (!(x >= kUnderflow)) acc[t] += q.c * exp_neg(x, e2t);  // a NaN exponent adds NaN
+        for (int k = 0; k < kSub / kLanes; ++k) {
+          const VSrc c = mine[k * kLanes + q4];
+          const double dx = px - c.x, dy = py - c.y;
+          const double x = (dx * dx + dy * dy) * c.rr;
+          if (!(x >= kUnderflow)) acc += c.c * exp_neg(x, e2t);  // a NaN exponent adds NaN
         }
       }
-    } else if (k0 || k1) {  // one group: the other's pairs with this tile all add nothing
-      const double qx = k0 ? px[0] : px[1], qy = k0 ? py[0] : py[1];
-      double a = k0 ? acc[0] : acc[1];
-      for (int k = 0; k < n; ++k) {
-        const VSrc q = tile[k];
-        const double dx = qx - q.x, dy = qy - q.y;
-        const double x = (dx * dx + dy * dy) * q.rr;
-        if (!(x >= kUnderflow)) a += q.c * exp_neg(x, e2t);
-      }
-      if (k0)
-        acc[0] = a;
-      else
-        acc[1] = a;
     }
+    __syncthreads();  // before the list changes
   }
-#pragma unroll
-  for (int t = 0; t < kTpl; ++t) {
-    if (ti[t] >= nt) continue;
-    if (direct)
-      out[torder ? (int64_t)torder[ti[t]] : ti[t]] += acc[t];
+  // a target's four lanes, then its two waves
+  acc += __shfl_xor(acc, kGroup, 64);
+  acc += __shfl_xor(acc, 2 * kGroup, 64);
+  if (half == 1 && lane < kGroup) sum[group][lane] = acc;
+  __syncthreads();
+  if (half == 0 && lane < kGroup && p < nt) {
+    acc += sum[group][lane];
+    if (part)
+      part[(int64_t)blockIdx.y * nt + p] = acc;
     else
-      out[by * nt + ti[t]] = acc[t];
+      tw[o] += acc;
   }
 }
 
-__global__ __launch_bounds__(kBlock) void vort_reduce_kernel(int64_t nchunk, int64_t nt,
+// tw[torder[p]] += the sum over rows of part[row nt + p], in row order
+__global__ __launch_bounds__(kBlock) void vort_reduce_kernel(int64_t rows, int64_t nt,
                                                              const double* __restrict__ part,
-                                                             const uint8_t* __restrict__ flag,
-                                                             int64_t nchunk8,
                                                              const uint32_t* __restrict__ torder,
                                                              double* __restrict__ tw) {
   const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (p >= nt) return;
-  const int64_t wg = p / (kBlock * kTpl);
-  // the workgroup's flags eight at a time (the row starts 8-byte aligned)
-  const uint64_t* fw = reinterpret_cast<const uint64_t*>(flag + wg * nchunk8);
   double s = 0.0;
-  for (int64_t w = 0; w < nchunk8 / 8; ++w) {
-    const uint64_t f = fw[w];
-    if (!f) continue;
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const int64_t c = 8 * w + b;
-      if (c < nchunk && ((f >> (8 * b)) & 0xff)) s += part[c * nt + p];
-    }
-  }
-  tw[torder ? (int64_t)torder[p] : p] += s;
+#pragma unroll 4
+  for (int64_t r = 0; r < rows; ++r) s += part[r * nt + p];
+  tw[torder[p]] += s;
 }
 
 }  // namespace
@@ -356,81 +309,34 @@ int vorticity_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const 
                   const double* ss, const double* sr, int64_t nt, const double* tx,
                   const double* ty, double* tw) {
   if (ns == 0 || nt == 0) return 0;
-  const int64_t twgs = (nt + kBlock * kTpl - 1) / (kBlock * kTpl);
   const int64_t ntiles = (ns + kTile - 1) / kTile;
-  // with many sources and targets, both in Morton order and source tiles skipped whole
-  const bool prune = ns >= kPruneSources && nt >= kPruneTargets;
-  int64_t nchunk;
-  if (prune) {  // short chunks: the work sits in few (workgroup, chunk) pairs
-    nchunk = (ntiles + O2D_VORT_PRUNED_TILES - 1) / O2D_VORT_PRUNED_TILES;
-    const int64_t cap = kPartialBytes / ((int64_t)sizeof(double) * nt);
-    if (nchunk > cap) nchunk = cap > 1 ? cap : 1;
-  } else {  // enough workgroups to keep every CU busy
-    const int64_t want = O2D_WANT_VORT * (int64_t)d->num_cu;
-    nchunk = twgs >= want ? 1 : (want + twgs - 1) / twgs;
-    if (nchunk > ntiles) nchunk = ntiles;
-  }
-  int64_t per = (ntiles + nchunk - 1) / nchunk;
-  while (per < ntiles && twgs * ((ntiles + per - 1) / per) > INT32_MAX) per *= 2;  // 1-D grid
-  nchunk = (ntiles + per - 1) / per;
-  const int64_t chunk = per * kTile;
-  const int64_t cells = twgs * nchunk;
-  // a multiplier coprime to the cell count spreads the cells over the dispatch order
-  int64_t perm = 1;
-  if (prune && cells > 1) {
-    perm = (int64_t)(0.6180339887 * (double)cells) | 1;
-    auto gcd = [](int64_t a, int64_t b) {
-      while (b) {
-        const int64_t t = a % b;
-        a = b;
-        b = t;
-      }
-      return a;
-    };
-    while (gcd(perm, cells) != 1) perm += 2;
-    perm %= cells;
-  }
-  double* out = tw;
-  uint8_t* flag = nullptr;
-  const int direct = nchunk == 1;
-  const int64_t nchunk8 = (nchunk + 7) & ~int64_t(7);
-  if (!direct) {
-    void* p;
-    O2D_TRY(slot(d, kPartials, sizeof(double) * nchunk * nt + twgs * nchunk8, s, &p));
-    out = static_cast<double*>(p);
-    flag = reinterpret_cast<uint8_t*>(out + nchunk * nt);
-  }
-  VSrc* vs = nullptr;
-  double* tbox = nullptr;
-  double* gbox = nullptr;
-  const uint32_t* torder = nullptr;
-  if (prune) {
-    const uint32_t* sorder = nullptr;
-    O2D_TRY(morton_order16(d, s, ns, sx, sy, &sorder));
-    void* vp;
-    const int64_t ngrp = (nt + kBlock - 1) / kBlock;
-    O2D_TRY(slot(d, kVortSrc, sizeof(VSrc) * ns + sizeof(double) * (5 * ntiles + 4 * ngrp), s,
-                 &vp));
-    vs = static_cast<VSrc*>(vp);
-    tbox = reinterpret_cast<double*>(vs + ns);
-    gbox = tbox + 5 * ntiles;
-    vort_gather_kernel<<<(unsigned)ntiles, kBlock, 0, s>>>(ns, sx, sy, ss, sr, sorder, vs, tbox);
-    O2D_LAUNCH_CHECK();
-    O2D_TRY(morton_order16(d, s, nt, tx, ty, &torder));  // reuses the order slot: vs holds the sources
-    vort_target_box_kernel<<<(unsigned)ngrp, kBlock, 0, s>>>(nt, tx, ty, torder, gbox);
-    O2D_LAUNCH_CHECK();
-  }
-  {
-    KernelTimer kt(O2D_KT_VORT, s);
-    vort_kernel<<<(unsigned)cells, kBlock, 0, s>>>(ns, sx, sy, ss, sr, nt, tx, ty, chunk, out,
-                                                   flag, twgs, nchunk8, perm, direct, vs, tbox,
-                                                   gbox, torder);
-    kt.stop();
-    O2D_LAUNCH_CHECK();
-  }
-  if (!direct) {
+  const uint32_t *sorder = nullptr, *torder = nullptr;
+  O2D_TRY(morton_order16(d, s, ns, sx, sy, &sorder));
+  void* vp;
+  O2D_TRY(slot(d, kVortSrc, (sizeof(VSrc) * kTile + sizeof(VBox) * (kSubs + 1)) * (size_t)ntiles, s,
+               &vp));
+  VSrc* vs = static_cast<VSrc*>(vp);
+  VBox* sub = reinterpret_cast<VBox*>(vs + kTile * ntiles);
+  VBox* tbox = sub + kSubs * ntiles;
+  vort_gather_kernel<<<(unsigned)ntiles, kBlock, 0, s>>>(ns, sx, sy, ss, sr, sorder, vs, sub, tbox);
+  O2D_LAUNCH_CHECK();
+  torder = sorder;  // the sources themselves, or another order in the same slot: vs holds the sources
+  if (!(tx == sx && ty == sy && nt == ns)) O2D_TRY(morton_order16(d, s, nt, tx, ty, &torder));
+  const int64_t twgs = (nt + kNearTargets - 1) / kNearTargets;
+  const int64_t want = kNearWgs * (int64_t)d->num_cu;
+  int64_t rows = std::max((want + twgs - 1) / twgs, kNearRows);
+  rows = std::min({rows, ntiles, kPartialBytes / ((int64_t)sizeof(double) * nt)});
+  rows = std::max<int64_t>(rows, 1);
+  void* part = nullptr;
+  if (rows > 1) O2D_TRY(slot(d, kPartials, sizeof(double) * rows * nt, s, &part));
+  KernelTimer kt(O2D_KT_VORT, s);
+  vort_near_kernel<<<dim3((unsigned)twgs, (unsigned)rows), kNearT, 0, s>>>(
+      nt, tx, ty, torder, ntiles, vs, sub, tbox, tw, static_cast<double*>(part));
+  kt.stop();
+  O2D_LAUNCH_CHECK();
+  if (rows > 1) {
     vort_reduce_kernel<<<(unsigned)((nt + kBlock - 1) / kBlock), kBlock, 0, s>>>(
-        nchunk, nt, out, flag, nchunk8, torder, tw);
+        rows, nt, static_cast<const double*>(part), torder, tw);
     O2D_LAUNCH_CHECK();
   }
   return 0;
