@@ -56,6 +56,11 @@ int lu_solve_dev(Device* d, hipStream_t s, int n, const double* lu, const int* p
 int matvec_dev(Device* d, hipStream_t s, int n, const double* a, const double* b, double* x);
 int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* x);
 
+// ou[order[i]] += sum over chunks c of pu[c*nt + i], and ov, ow alike (pw, ow may be null; order null: the
+// identity); nbody.hip
+int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* order, const double* pu,
+                  const double* pv, const double* pw, double* ou, double* ov, double* ow);
+
 int rk_move_dev(hipStream_t s, int64_t n, double dt, int nstage, const double* w,
                 const double* const* u, const double* const* v, const double* x0,
                 const double* y0, double* x, double* y, double* uc, double* vc);

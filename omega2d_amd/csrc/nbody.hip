@@ -716,6 +716,14 @@ int gather_targets(hipStream_t s, int core, int64_t n, const uint32_t* order, co
 
 }  // namespace
 
+int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* order, const double* pu,
+                  const double* pv, const double* pw, double* ou, double* ov, double* ow) {
+  reduce_chunks_kernel<<<(unsigned)((nt + 63) / 64), kBlock, 0, s>>>(nchunk, nt, order, pu, pv, pw,
+                                                                     ou, ov, ow);
+  O2D_LAUNCH_CHECK();
+  return 0;
+}
+
 // The most source chunks whose fp64 partials (nf per target) fit what is left of *ws; no limit
 // when the temporaries come from the buffer pool.
 int64_t max_chunks(const Workspace* ws, int nf, int64_t nt) {
@@ -837,9 +845,7 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
     kt.stop();
     O2D_LAUNCH_CHECK();
     if (!direct) {
-      reduce_chunks_kernel<<<(unsigned)((nt + 63) / 64), kBlock, 0, s>>>(cp.nchunk, nt, torder, ou,
-                                                                         ov, ow, tu, tv, tw);
-      O2D_LAUNCH_CHECK();
+      O2D_TRY(reduce_chunks(s, cp.nchunk, nt, torder, ou, ov, ow, tu, tv, tw));
     }
     return 0;
   }
@@ -897,9 +903,7 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
   kt.stop();
   O2D_LAUNCH_CHECK();
   if (!direct) {
-    reduce_chunks_kernel<<<(unsigned)((nt + 63) / 64), kBlock, 0, s>>>(cp.nchunk, nt, torder, ou,
-                                                                       ov, ow, tu, tv, tw);
-    O2D_LAUNCH_CHECK();
+    O2D_TRY(reduce_chunks(s, cp.nchunk, nt, torder, ou, ov, ow, tu, tv, tw));
   }
   return 0;
 }

@@ -23,18 +23,18 @@
 #include "o2d_runtime.h"
 #include "panel_math.h"
 
-// workgroups per CU the particle chunks of points_on_panels aim for (32: 0.990 -> 0.975 ms on
-// 200k particles x 2,048 panels; 128 took 1.073 ms)
-#ifndef O2D_WANT_RHS
-#define O2D_WANT_RHS 32
-#endif
-
 namespace o2d {
 
 namespace {
 
 constexpr int kBlock = 256;
 constexpr int kPTile = 256;  // panels per LDS stage (panels on points)
+// workgroups per CU the particle chunks of points_on_panels aim for: 200k particles and 2,048 panels
+// (both panel sums) take 323 us with 16, 329 with 32 and 339 with 8; 20k 152, 177 and 142; 100k and 500
+// panels 198, 226 and 193
+constexpr int64_t kRhsWgs = 16;
+// and those of its far clusters: 330 us with 8 or 4, 332 with 16 and 344 with 32
+constexpr int64_t kRhsFarWgs = 8;
 #ifndef O2D_PANTILE
 #define O2D_PANTILE 4
 #endif
@@ -192,52 +192,94 @@ __global__ __launch_bounds__(64) void cluster_kernel(int64_t np, const double* _
   }
 }
 
+// LDS writes of this wave visible to its own later reads, and no compiler reordering across
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // panels on points with the clustered far field: one lane per target (targets taken in the
 // order torder, so that a wave is compact and its lanes agree on near and far), the clusters
-// [blockIdx.y cchunk, (blockIdx.y + 1) cchunk); with several chunks, chunk y's sums go to
-// pu/pv[y nt + position in torder] for reduce_sorted_kernel, else they are added to ou/ov
+// blockIdx.y, blockIdx.y + gridDim.y, ...; with several such rows, row y's sums go to
+// pu/pv[y nt + position in torder] for reduce_chunks, else they are added to ou/ov.
+//
+// Bound by the fp64 units: 88 multiply-adds a far cluster, 32 logarithms (mostly short series) a near
+// one. Near clusters are neighbours along the body, so rows of consecutive clusters gave one
+// wave at the wall up to eleven of them, and the launch waited for it: 195 us for 200,000 points and 2,048
+// panels, 93 with the clusters dealt out to the rows. Heads and moments pass through LDS (scalar
+// loads stalled the wave: 206 us), and a wave's lanes prepare a near cluster's panels together. Two
+// targets a lane halve the broadcasts but not the time (they double the near work of a wave), and the
+// full unrolling of the series spilled.
+constexpr int kClusStage = 16;  // clusters brought into LDS at a time
 template <bool SRC>
-__global__ __launch_bounds__(kBlock, 5) void panels_clustered_kernel(
+__global__ __launch_bounds__(kBlock, 4) void panels_clustered_kernel(
     int64_t np, const double* __restrict__ nx, const double* __restrict__ ny,
     const uint32_t* __restrict__ idx, const double* __restrict__ vs, const double* __restrict__ ss,
     int64_t nclus, const double* __restrict__ head, const double* __restrict__ mom, int64_t nt,
     const double* __restrict__ tx, const double* __restrict__ ty,
-    const uint32_t* __restrict__ torder, int64_t cchunk, double* __restrict__ ou,
-    double* __restrict__ ov, int direct) {
-  const int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t* __restrict__ torder, double* __restrict__ ou, double* __restrict__ ov,
+    int direct) {
+  __shared__ double lhead[kClusStage][kHead];
+  __shared__ double2 lmom[kClusStage][kTerms];
+  __shared__ PanelPre lpan[kBlock / 64][kClus];
+  const int tid = threadIdx.x, lane = tid & 63;
+  PanelPre* mine = lpan[tid >> 6];
+  const int64_t g = (int64_t)blockIdx.x * kBlock + tid;
   const int64_t gg = g < nt ? g : nt - 1;
   const int64_t i = torder ? (int64_t)torder[gg] : gg;
   const double px = tx[i], py = ty[i];
   double au = 0.0, av = 0.0;
-  const int64_t cb = (int64_t)blockIdx.y * cchunk;
-  const int64_t ce = cb + cchunk < nclus ? cb + cchunk : nclus;
-  for (int64_t c = cb; c < ce; ++c) {
-    const double* h = head + kHead * c;
-    const double zx = px - h[0], zy = py - h[1];
-    const double z2 = __builtin_fma(zx, zx, zy * zy);
-    if (z2 >= h[2] && z2 > 0.0) {  // far (a point at the centre of a cluster of no extent is near)
-      // w = 1 / (z - c); sum_n A_n w^n = w (A_1 + w (A_2 + ... + w A_kTerms))
-      const double iz = rcp64(z2);
-      const double wx = zx * iz, wy = -zy * iz;
-      const double* A = mom + 2 * kTerms * c;
-      double sx = A[2 * (kTerms - 1)], sy = A[2 * (kTerms - 1) + 1];
-#pragma unroll
-      for (int n = kTerms - 2; n >= 0; --n) {
-        const double nx_ = __builtin_fma(sx, wx, __builtin_fma(-sy, wy, A[2 * n]));
-        sy = __builtin_fma(sx, wy, __builtin_fma(sy, wx, A[2 * n + 1]));
-        sx = nx_;
+  const int64_t step = gridDim.y;
+  for (int64_t c0 = blockIdx.y; c0 < nclus; c0 += step * kClusStage) {
+    const int64_t left = (nclus - c0 + step - 1) / step;
+    const int nc = (int)(left < kClusStage ? left : kClusStage);
+    __syncthreads();
+    for (int e = tid; e < nc * kHead; e += kBlock)
+      lhead[e / kHead][e % kHead] = head[kHead * (c0 + e / kHead * step) + e % kHead];
+    for (int e = tid; e < nc * kTerms; e += kBlock)
+      lmom[e / kTerms][e % kTerms] =
+          reinterpret_cast<const double2*>(mom)[kTerms * (c0 + e / kTerms * step) + e % kTerms];
+    __syncthreads();
+    for (int c = 0; c < nc; ++c) {
+      const double* h = lhead[c];
+      const double zx = px - h[0], zy = py - h[1];
+      const double z2 = __builtin_fma(zx, zx, zy * zy);
+      const bool far = z2 >= h[2] && z2 > 0.0;  // (a point at the centre of a cluster of no extent is near)
+      if (far) {
+        // w = 1 / (z - c); sum_n A_n w^n = w (A_1 + w (A_2 + ... + w A_kTerms))
+        const double iz = rcp64(z2);
+        const double wx = zx * iz, wy = -zy * iz;
+        double sx = lmom[c][kTerms - 1].x, sy = lmom[c][kTerms - 1].y;
+        static_assert((kTerms - 1) % 3 == 0, "three terms at a time");
+#pragma unroll 3
+        for (int n = kTerms - 2; n >= 0; --n) {
+          const double2 A = lmom[c][n];
+          const double x = __builtin_fma(sx, wx, __builtin_fma(-sy, wy, A.x));
+          sy = __builtin_fma(sx, wy, __builtin_fma(sy, wx, A.y));
+          sx = x;
+        }
+        av += __builtin_fma(sx, wx, -sy * wy);  // v + i u = W L
+        au += __builtin_fma(sx, wy, sy * wx);
       }
-      av += __builtin_fma(sx, wx, -sy * wy);  // v + i u = W L
-      au += __builtin_fma(sx, wy, sy * wx);
-    } else {
-      const int64_t k1 = (c + 1) * kClus < np ? (c + 1) * kClus : np;
-      for (int64_t k = c * kClus; k < k1; ++k) {
-        const uint32_t a = idx[2 * k], b = idx[2 * k + 1];
-        const PanelPre q = panel_pre(nx[a], ny[a], nx[b], ny[b], vs[k], SRC ? ss[k] : 0.0);
-        double lr, li;
-        panel_log(q, px, py, lr, li);
-        au += __builtin_fma(q.wr, li, q.wi * lr);
-        av += __builtin_fma(q.wr, lr, -q.wi * li);
+      if (!__all(far)) {
+        const int64_t k0 = (c0 + c * step) * kClus;
+        const int nk = (int)(np - k0 < kClus ? np - k0 : kClus);
+        wave_sync();  // the last near cluster's reads are done
+        if (lane < nk) {
+          const int64_t k = k0 + lane;
+          const uint32_t a = idx[2 * k], b = idx[2 * k + 1];
+          mine[lane] = panel_pre(nx[a], ny[a], nx[b], ny[b], vs[k], SRC ? ss[k] : 0.0);
+        }
+        wave_sync();
+        if (far) continue;
+        for (int k = 0; k < nk; ++k) {
+          const PanelPre& q = mine[k];
+          double lr, li;
+          panel_log(q, px, py, lr, li);
+          au += __builtin_fma(q.wr, li, q.wi * lr);
+          av += __builtin_fma(q.wr, lr, -q.wi * li);
+        }
       }
     }
   }
@@ -249,41 +291,6 @@ __global__ __launch_bounds__(kBlock, 5) void panels_clustered_kernel(
     ou[(int64_t)blockIdx.y * nt + g] = au;
     ov[(int64_t)blockIdx.y * nt + g] = av;
   }
-}
-
-// ou[torder[g]] += sum over chunks of pu[c nt + g], in chunk order (the same for ov)
-__global__ __launch_bounds__(kBlock) void reduce_sorted_kernel(int64_t nchunk, int64_t nt,
-                                                               const uint32_t* __restrict__ torder,
-                                                               const double* __restrict__ pu,
-                                                               const double* __restrict__ pv,
-                                                               double* __restrict__ ou,
-                                                               double* __restrict__ ov) {
-  const int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (g >= nt) return;
-  double su = 0.0, sv = 0.0;
-  for (int64_t c = 0; c < nchunk; ++c) {
-    su += pu[c * nt + g];
-    sv += pv[c * nt + g];
-  }
-  const int64_t i = torder ? (int64_t)torder[g] : g;
-  ou[i] += su;
-  ov[i] += sv;
-}
-
-__global__ __launch_bounds__(kBlock) void reduce_chunks2_kernel(int64_t nchunk, int64_t n,
-                                                                const double* __restrict__ pu,
-                                                                const double* __restrict__ pv,
-                                                                double* __restrict__ ou,
-                                                                double* __restrict__ ov) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  double su = 0.0, sv = 0.0;
-  for (int64_t c = 0; c < nchunk; ++c) {
-    su += pu[c * n + i];
-    sv += pv[c * n + i];
-  }
-  ou[i] += su;
-  ov[i] += sv;
 }
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -448,6 +455,10 @@ __global__ __launch_bounds__(kBlock) void gather_groups_kernel(int64_t ns,
 // to gpart[((c nchunk + y) kTerms + n - 1) 2 + {0, 1}]. A panel's sum over those particles is
 // then sum_j s_j L_p(z_j) = sum_n G_n (b_p^n - a_p^n) / n (rhs_combine_kernel), the expansion of
 // the panels-on-points moments read the other way, with the same remainder bound.
+//
+// Bound by the fp64 units, six operations a term, where a lane has many particles; with few by its own
+// end: a wave sum for each of the 44 values was most of the launch (20,000 particles and 2,048 panels:
+// 100 us, 16 with the exchanges below and half the chunks).
 __global__ __launch_bounds__(kBlock) void rhs_far_kernel(int64_t ns, const double* __restrict__ sx,
                                                          const double* __restrict__ sy,
                                                          const double* __restrict__ ss,
@@ -458,9 +469,9 @@ __global__ __launch_bounds__(kBlock) void rhs_far_kernel(int64_t ns, const doubl
   const int tid = threadIdx.x;
   const int64_t c = blockIdx.x;
   const double hx = head[kHead * c], hy = head[kHead * c + 1], hr2 = head[kHead * c + 2];
-  double gr[kTerms], gi[kTerms];
+  double g[2 * kTerms];
 #pragma unroll
-  for (int n = 0; n < kTerms; ++n) gr[n] = gi[n] = 0.0;
+  for (int n = 0; n < 2 * kTerms; ++n) g[n] = 0.0;
   const int64_t jb = (int64_t)blockIdx.y * chunk;
   const int64_t je = jb + chunk < ns ? jb + chunk : ns;
   for (int64_t j = jb + tid; j < je; j += kBlock) {
@@ -472,23 +483,38 @@ __global__ __launch_bounds__(kBlock) void rhs_far_kernel(int64_t ns, const doubl
       double pr = ss[j] * wx, pi = ss[j] * wy;   // s w^n
 #pragma unroll
       for (int n = 0; n < kTerms; ++n) {
-        gr[n] += pr;
-        gi[n] += pi;
+        g[2 * n] += pr;
+        g[2 * n + 1] += pi;
         const double npr = __builtin_fma(pr, wx, -pi * wy);
         pi = __builtin_fma(pr, wy, pi * wx);
         pr = npr;
       }
     }
   }
-  const int wv = tid / 64, ln = tid % 64;
-#pragma unroll
-  for (int n = 0; n < kTerms; ++n) {
-    const double a = wave_sum(gr[n]), b = wave_sum(gi[n]);
-    if (ln == 0) {
-      red[wv][2 * n] = a;
-      red[wv][2 * n + 1] = b;
-    }
+  // the wave's sums, halving the values a lane holds at each step (45 exchanges, not 6 for each of 44)
+  const int wv = tid / 64;
+  int at = 0, count = 2 * kTerms;  // the first value this lane holds, and how many (the rest is padding)
+#define O2D_HALVE(N, O)                                                      \
+  {                                                                          \
+    constexpr int kHalf = ((N) + 1) / 2;                                     \
+    const bool up = (tid & (O)) != 0;                                        \
+    _Pragma("unroll") for (int k = 0; k < kHalf; ++k) {                      \
+      const double hi = k + kHalf < (N) ? g[k + kHalf] : 0.0;                \
+      const double keep = up ? hi : g[k], send = up ? g[k] : hi;             \
+      g[k] = keep + __shfl_xor(send, (O), 64);                               \
+    }                                                                        \
+    if (up) at += kHalf;                                                     \
+    count = up ? count - kHalf : (count < kHalf ? count : kHalf);            \
   }
+  static_assert(2 * kTerms == 44, "the halvings below");
+  O2D_HALVE(44, 32)
+  O2D_HALVE(22, 16)
+  O2D_HALVE(11, 8)
+  O2D_HALVE(6, 4)
+  O2D_HALVE(3, 2)
+  O2D_HALVE(2, 1)
+#undef O2D_HALVE
+  if (count > 0) red[wv][at] = g[0];
   __syncthreads();
   if (tid < 2 * kTerms) {
     double acc = 0.0;
@@ -497,15 +523,29 @@ __global__ __launch_bounds__(kBlock) void rhs_far_kernel(int64_t ns, const doubl
   }
 }
 
-// gsum[(c kTerms + n) 2 + {0, 1}] = sum over the chunks of gpart, in chunk order
+// gsum[(c kTerms + n) 2 + {0, 1}] = sum over the chunks of gpart. A workgroup takes 64 entries, its
+// waves a quarter of the chunks each, in order, added in wave order (64 clusters, 64 chunks: 20 us with
+// a thread per entry, 5 so)
 __global__ __launch_bounds__(kBlock) void rhs_gsum_kernel(int64_t nclus, int64_t nchunk,
                                                           const double* __restrict__ gpart,
                                                           double* __restrict__ gsum) {
-  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;  // (c kTerms + n) 2 + part
-  if (e >= nclus * kTerms * 2) return;
+  constexpr int kWaves = kBlock / 64;
+  __shared__ double sm[kWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t e = (int64_t)blockIdx.x * 64 + lane;  // (c kTerms + n) 2 + part
   const int64_t c = e / (2 * kTerms), r = e % (2 * kTerms);
+  const int64_t share = (nchunk + kWaves - 1) / kWaves;
+  const int64_t y1 = (wave + 1) * share < nchunk ? (wave + 1) * share : nchunk;
   double acc = 0.0;
-  for (int64_t y = 0; y < nchunk; ++y) acc += gpart[(c * nchunk + y) * kTerms * 2 + r];
+  if (e < nclus * kTerms * 2) {
+#pragma unroll 4
+    for (int64_t y = wave * share; y < y1; ++y) acc += gpart[(c * nchunk + y) * kTerms * 2 + r];
+  }
+  sm[wave][lane] = acc;
+  __syncthreads();
+  if (wave != 0 || e >= nclus * kTerms * 2) return;
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) acc += sm[w][lane];
   gsum[e] = acc;
 }
 
@@ -588,12 +628,11 @@ int panels_on_points_dev(Device* d, hipStream_t s, int64_t nnodes, const double*
     O2D_LAUNCH_CHECK();
     const uint32_t* torder = nullptr;
     if (nt > kBlock) O2D_TRY(morton_order16(d, s, nt, tx, ty, &torder));
-    // chunks of clusters for 16 workgroups per CU (C3: 782 target tiles, 6 chunks)
+    // rows of clusters for 16 workgroups per CU (200,000 targets and 2,048 panels: 6 rows, 358 us for
+    // both panel sums; 375 with 8 per CU, 366 with 64)
     const int64_t twgs = (nt + kBlock - 1) / kBlock;
     const int64_t want = 16 * (int64_t)d->num_cu;
-    int64_t nchunk = twgs >= want ? 1 : std::min<int64_t>((want + twgs - 1) / twgs, nclus);
-    const int64_t cchunk = (nclus + nchunk - 1) / nchunk;
-    nchunk = (nclus + cchunk - 1) / cchunk;
+    const int64_t nchunk = twgs >= want ? 1 : std::min<int64_t>((want + twgs - 1) / twgs, nclus);
     double *ou = tu, *ov = tv;
     const int direct = nchunk == 1;
     if (!direct) {
@@ -606,15 +645,14 @@ int panels_on_points_dev(Device* d, hipStream_t s, int64_t nnodes, const double*
     KernelTimer kt(O2D_KT_PANELS, s);
     if (ss)
       panels_clustered_kernel<true><<<grid, kBlock, 0, s>>>(
-          np, nx, ny, idx, vs, ss, nclus, head, mom, nt, tx, ty, torder, cchunk, ou, ov, direct);
+          np, nx, ny, idx, vs, ss, nclus, head, mom, nt, tx, ty, torder, ou, ov, direct);
     else
       panels_clustered_kernel<false><<<grid, kBlock, 0, s>>>(
-          np, nx, ny, idx, vs, ss, nclus, head, mom, nt, tx, ty, torder, cchunk, ou, ov, direct);
+          np, nx, ny, idx, vs, ss, nclus, head, mom, nt, tx, ty, torder, ou, ov, direct);
     kt.stop();
     O2D_LAUNCH_CHECK();
     if (!direct) {
-      reduce_sorted_kernel<<<grid1(nt), kBlock, 0, s>>>(nchunk, nt, torder, ou, ov, tu, tv);
-      O2D_LAUNCH_CHECK();
+      O2D_TRY(reduce_chunks(s, nchunk, nt, torder, ou, ov, nullptr, tu, tv, nullptr));
     }
     return 0;
   }
@@ -644,8 +682,7 @@ int panels_on_points_dev(Device* d, hipStream_t s, int64_t nnodes, const double*
   kt.stop();
   O2D_LAUNCH_CHECK();
   if (!direct) {
-    reduce_chunks2_kernel<<<grid1(nt), kBlock, 0, s>>>(nchunk, nt, ou, ov, tu, tv);
-    O2D_LAUNCH_CHECK();
+    O2D_TRY(reduce_chunks(s, nchunk, nt, nullptr, ou, ov, nullptr, tu, tv, nullptr));
   }
   return 0;
 }
@@ -656,7 +693,7 @@ int points_on_panels_dev(Device* d, hipStream_t s, int64_t ns, const double* sx,
   (void)nnodes;
   if (np == 0 || ns == 0) return 0;
   const int64_t pwgs = (np + kPanTile - 1) / kPanTile;
-  const int64_t want = O2D_WANT_RHS * (int64_t)d->num_cu;
+  const int64_t want = kRhsWgs * d->num_cu;
   int64_t nchunk = pwgs >= want ? 1 : (want + pwgs - 1) / pwgs;
   const int64_t maxchunk = (ns + kBlock - 1) / kBlock;  // at least one particle per lane
   if (nchunk > maxchunk) nchunk = maxchunk;
@@ -696,11 +733,10 @@ int points_on_panels_dev(Device* d, hipStream_t s, int64_t ns, const double* sx,
   void* p;
   O2D_TRY(slot(d, kPartials, sizeof(double) * 2 * rows * np, s, &p));
   double* part = static_cast<double*>(p);
-  // far chunks for 16 workgroups per CU
   int64_t fchunk = 0, nfchunk = 0;
   double* gpart = nullptr;
   if (clus) {
-    const int64_t fwant = 16 * (int64_t)d->num_cu;
+    const int64_t fwant = kRhsFarWgs * d->num_cu;
     nfchunk = nclus >= fwant ? 1 : (fwant + nclus - 1) / nclus;
     if (nfchunk > maxchunk) nfchunk = maxchunk;
     fchunk = (ns + nfchunk - 1) / nfchunk;
@@ -718,7 +754,7 @@ int points_on_panels_dev(Device* d, hipStream_t s, int64_t ns, const double* sx,
         ns, sx, sy, ss, head, fchunk, nfchunk, gpart);
     O2D_LAUNCH_CHECK();
     double* gsum = gpart + 2 * kTerms * nclus * nfchunk;
-    rhs_gsum_kernel<<<grid1(2 * kTerms * nclus), kBlock, 0, s>>>(nclus, nfchunk, gpart, gsum);
+    rhs_gsum_kernel<<<(unsigned)((2 * kTerms * nclus + 63) / 64), kBlock, 0, s>>>(nclus, nfchunk, gpart, gsum);
     O2D_LAUNCH_CHECK();
     rhs_combine_kernel<<<grid1(np), kBlock, 0, s>>>(np, nx, ny, idx, head, gsum,
                                                     part + 2 * nchunk * np);
