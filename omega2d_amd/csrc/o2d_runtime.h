@@ -45,6 +45,8 @@ struct Device {
   hipStream_t stream = nullptr;
   void* buf[kNumSlots] = {};
   size_t cap[kNumSlots] = {};
+  void* pin = nullptr;  // page-locked host memory of the packed host-array calls
+  size_t pin_cap = 0;
   // LU factors of the last matrix given to o2d_hip_bem_factor_*
   int64_t lu_n = 0;
   bool lu_ready = false;
@@ -74,6 +76,9 @@ inline hipStream_t stream_of(const o2d_env* env, Device* d) {
 inline hipStream_t dev_stream(const o2d_env* env) { return static_cast<hipStream_t>(env->stream); }
 // Device buffer for `slot` with at least `bytes`; grows (after draining `s`) when too small.
 int slot(Device* d, Slot which, size_t bytes, hipStream_t s, void** out);
+
+// Page-locked host memory of at least `bytes`; grows (after draining the device) when too small.
+int pinned(Device* d, size_t bytes, void** out);
 
 // A fixed device buffer handed out in consecutive 256-byte-aligned pieces, for calls that
 // must not allocate.

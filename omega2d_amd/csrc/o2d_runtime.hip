@@ -70,6 +70,22 @@ int slot(Device* d, Slot which, size_t bytes, hipStream_t s, void** out) {
   return 0;
 }
 
+int pinned(Device* d, size_t bytes, void** out) {
+  if (d->pin_cap < bytes) {
+    if (d->pin) {
+      O2D_HIP(hipDeviceSynchronize());
+      O2D_HIP(hipHostFree(d->pin));
+      d->pin = nullptr;
+      d->pin_cap = 0;
+    }
+    size_t want = (bytes + bytes / 4 + 4095) & ~size_t(4095);
+    O2D_HIP(hipHostMalloc(&d->pin, want, hipHostMallocDefault));
+    d->pin_cap = want;
+  }
+  *out = d->pin;
+  return 0;
+}
+
 int take(Device* d, Workspace* ws, Slot which, size_t bytes, hipStream_t s, void** out) {
   if (!ws) return slot(d, which, bytes, s, out);
   if (bytes == 0) bytes = 256;
@@ -187,6 +203,7 @@ int o2d_hip_release(void) {
       d->buf[s] = nullptr;
       d->cap[s] = 0;
     }
+    if (d->pin) O2D_HIP(hipHostFree(d->pin));
     O2D_HIP(hipStreamDestroy(d->stream));
     *d = Device();
   }
