@@ -242,6 +242,26 @@ int o2d_hip_rk_advance_dev_d(const o2d_env* env, int64_t n, double dt, int32_t n
 int o2d_hip_finalize_dev_d(const o2d_env* env, int64_t n, double fsx, double fsy, double factor,
                            double* u, double* v);
 
+/* ---- the vector work of a body in a step (device arrays, each operation rounded) --------------- */
+
+/* rhs of a body's boundary-element system (src/RHS.h:54-115, src/BEMHelper.h:116-137): with u = fsx +
+ * pu * factor, v = fsy + pv * factor at the np panels, rhs[nunk p] = -(u tx + v ty) and, for nunk 2,
+ * rhs[2 p + 1] = -(u nx + v ny); rhs[nunk np] = reabsorbed + vol2 * omega_error (device scalars). */
+int o2d_hip_body_rhs_dev_d(const o2d_env* env, int64_t np, int32_t nunk, double fsx, double fsy,
+                           double factor, const double* pu, const double* pv, const double* tx,
+                           const double* ty, const double* nx, const double* ny,
+                           const double* reabsorbed, double vol2, const double* omega_error,
+                           double* rhs);
+/* The solution of that system taken apart: vs[p], ss[p] (0 for nunk 1), and its last entry into
+ * omega and omega_error. */
+int o2d_hip_body_unpack_dev_d(const o2d_env* env, int64_t np, int32_t nunk, const double* sol,
+                              double* vs, double* ss, double* omega, double* omega_error);
+/* Panel strengths with a rotation's added (src/Surfaces.h:556-620): ovs = vs - (ui tx + vi ty), oss =
+ * ss - (ui ty - vi tx), (ui, vi) = omega (-ddy, ddx). */
+int o2d_hip_body_strengths_dev_d(const o2d_env* env, int64_t np, const double* vs, const double* ss,
+                                 const double* omega, const double* tx, const double* ty,
+                                 const double* ddx, const double* ddy, double* ovs, double* oss);
+
 /* ---- adjoint (no reference counterpart) -------------------------------------------------- */
 
 /* Vector-Jacobian product of the unscaled point-target velocity sum

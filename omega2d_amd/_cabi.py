@@ -91,6 +91,10 @@ SIGNATURES = {
     "o2d_hip_rk_move_dev_d": [_envp, _i64, _dbl, _i32, _vp, _vp, _vp, _vp, _vp],
     "o2d_hip_rk_advance_dev_d": [_envp, _i64, _dbl, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                  _vp],
+    "o2d_hip_body_rhs_dev_d": [_envp, _i64, _i32, _dbl, _dbl, _dbl, _vp, _vp, _vp, _vp, _vp, _vp,
+                               _vp, _dbl, _vp, _vp],
+    "o2d_hip_body_unpack_dev_d": [_envp, _i64, _i32, _vp, _vp, _vp, _vp, _vp],
+    "o2d_hip_body_strengths_dev_d": [_envp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "o2d_hip_finalize_dev_d": [_envp, _i64, _dbl, _dbl, _dbl, _vp, _vp],
     "o2d_hip_points_on_points_adjoint_d": [_envp, _i64, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp,
                                            _vp, _vp, _vp, _vp, _vp],

@@ -12,6 +12,7 @@ from ._cabi import VELANDSHEAR, VELANDVORT, VELONLY, TreeOpts, call, make_env
 
 __all__ = ["points_on_points", "panels_on_points", "points_on_panels", "bem_assemble",
            "bem_factor", "bem_solve", "rk_move", "rk_advance", "finalize",
+           "body_rhs", "body_unpack", "body_strengths",
            "points_on_points_adjoint", "morton_order", "points_on_points_tree",
            "points_vorticity", "nearest_distances", "reflect", "clear_inner", "env_for"]
 
@@ -147,6 +148,39 @@ def finalize(u, v, fs, factor):
     call("o2d_hip_finalize_dev_d", ctypes.byref(env), u.numel(), float(fs[0]), float(fs[1]),
          float(factor), _ptr(u), _ptr(v))
     return u, v
+
+
+def body_rhs(pu, pv, fs, factor, tx, ty, nx, ny, nunk, reabsorbed, vol2, omega_error):
+    """The right-hand side of a body's system from the unscaled sums pu, pv at its panels."""
+    dev = _check(pu, pv, tx, ty, nx, ny, reabsorbed, omega_error)
+    rhs = torch.empty(pu.numel() * nunk + 1, dtype=torch.float64, device=dev)
+    env = env_for(dev)
+    call("o2d_hip_body_rhs_dev_d", ctypes.byref(env), pu.numel(), int(nunk), float(fs[0]),
+         float(fs[1]), float(factor), _ptr(pu), _ptr(pv), _ptr(tx), _ptr(ty), _ptr(nx), _ptr(ny),
+         _ptr(reabsorbed), float(vol2), _ptr(omega_error), _ptr(rhs))
+    return rhs
+
+
+def body_unpack(sol, nunk):
+    """The solution's vortex and source strengths, rotation and rotation error, as new tensors."""
+    dev = _check(sol)
+    npan = (sol.numel() - 1) // nunk
+    vs, ss = (torch.empty(npan, dtype=torch.float64, device=dev) for _ in range(2))
+    omega, error = (torch.empty((), dtype=torch.float64, device=dev) for _ in range(2))
+    env = env_for(dev)
+    call("o2d_hip_body_unpack_dev_d", ctypes.byref(env), npan, int(nunk), _ptr(sol), _ptr(vs),
+         _ptr(ss), _ptr(omega), _ptr(error))
+    return vs, ss, omega, error
+
+
+def body_strengths(vs, ss, omega, tx, ty, ddx, ddy):
+    """Panel strengths vs, ss with those of the rotation omega added, as new tensors."""
+    dev = _check(vs, ss, omega, tx, ty, ddx, ddy)
+    ovs, oss = torch.empty_like(vs), torch.empty_like(ss)
+    env = env_for(dev)
+    call("o2d_hip_body_strengths_dev_d", ctypes.byref(env), vs.numel(), _ptr(vs), _ptr(ss),
+         _ptr(omega), _ptr(tx), _ptr(ty), _ptr(ddx), _ptr(ddy), _ptr(ovs), _ptr(oss))
+    return ovs, oss
 
 
 def points_on_points_adjoint(sx, sy, ss, sr, tx, ty, gu, gv, *, core="gauss", out=None):

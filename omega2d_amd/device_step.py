@@ -126,36 +126,24 @@ class Body:
         vi = rotvel * self.ddx
         return (-1.0 * (ui * self.tx + vi * self.ty), -1.0 * (ui * self.ty - vi * self.tx))
 
+    def _scalar(self, v):
+        return torch.as_tensor(v, dtype=torch.float64, device=self.tx.device).reshape(())
+
     def solve(self, x, y, s, fs):
         """The boundary-element solve for particles (x, y, s) and freestream fs."""
-        pu = torch.zeros(self.np_, dtype=torch.float64, device=x.device)
-        pv = torch.zeros_like(pu)
+        pu, pv = torch.zeros((2, self.np_), dtype=torch.float64, device=x.device)
         dv.points_on_panels(x, y, s, self.nx, self.ny, self.idx, pu=pu, pv=pv)
-        pu = fs[0] + pu * FACTOR
-        pv = fs[1] + pv * FACTOR
-        rt = -(pu * self.tx + pv * self.ty)
-        if self.nunk == 1:
-            rhs = rt
-        else:
-            rn = -(pu * self.pnx + pv * self.pny)
-            rhs = torch.stack([rt, rn], 1).reshape(-1)
-        last = (0.0 + self.reabsorbed) + 2.0 * self.vol * self.omega_error
-        rhs = torch.cat([rhs, last.reshape(1)]).contiguous()
-        sol = dv.bem_solve(rhs)
-        self.omega = sol[-1].clone()
-        self.omega_error = self.omega.clone()
-        if self.nunk == 1:
-            self.vs = sol[:-1].clone()
-            self.ss = torch.zeros_like(self.vs)
-        else:
-            self.vs = sol[0:-1:2].clone()
-            self.ss = sol[1:-1:2].clone()
+        rhs = dv.body_rhs(pu, pv, fs, FACTOR, self.tx, self.ty, self.pnx, self.pny, self.nunk,
+                          self._scalar(self.reabsorbed), 2.0 * self.vol,
+                          self._scalar(self.omega_error))
+        sol = dv.bem_solve(rhs, torch.empty_like(rhs))
+        self.vs, self.ss, self.omega, self.omega_error = dv.body_unpack(sol, self.nunk)
 
     def add_vels(self, x, y, u, v):
         """Panels (with the solved rotation's strengths) on points, added into u, v."""
-        rv, rs = self.rot_strengths(1.0 * self.omega)
-        dv.panels_on_points(self.nx, self.ny, self.idx, (self.vs + rv).contiguous(),
-                            (self.ss + rs).contiguous(), x, y, tu=u, tv=v)
+        vs, ss = dv.body_strengths(self.vs.contiguous(), self.ss.contiguous(),
+                                   self._scalar(self.omega), self.tx, self.ty, self.ddx, self.ddy)
+        dv.panels_on_points(self.nx, self.ny, self.idx, vs, ss, x, y, tu=u, tv=v)
 
     def clear(self, x, y, s, r, ips):
         """Push particles out of the inner layer (method 1), in place."""

@@ -130,3 +130,24 @@ def test_advance_and_finalize_round_as_separate_operations(n, w):
     u, v = us[0].clone(), vs[0].clone()
     ds.dv.finalize(u, v, (1.5, -0.25), ds.FACTOR)
     assert torch.equal(u, 1.5 + us[0] * ds.FACTOR) and torch.equal(v, -0.25 + vs[0] * ds.FACTOR)
+
+
+@pytest.mark.parametrize("npan", [3, 255, 256, 257])
+@pytest.mark.parametrize("nunk", [1, 2])
+def test_body_vectors_round_as_separate_operations(npan, nunk):
+    # the same IEEE operations as torch's separate ones, so equal bit for bit
+    rng = np.random.default_rng(npan)
+    pu, pv, tx, ty, nx, ny, vs, ss, ddx, ddy = [T(rng.normal(size=npan)) for _ in range(10)]
+    a, e, w = [T(rng.normal(size=1)).reshape(()) for _ in range(3)]
+    rhs = ds.dv.body_rhs(pu, pv, (1.5, -0.25), ds.FACTOR, tx, ty, nx, ny, nunk, a, 0.7, e)
+    u, v = 1.5 + pu * ds.FACTOR, -0.25 + pv * ds.FACTOR
+    rows = [-(u * tx + v * ty), -(u * nx + v * ny)][:nunk]
+    ref = torch.cat([torch.stack(rows, 1).reshape(-1), ((0.0 + a) + 0.7 * e).reshape(1)])
+    assert torch.equal(rhs, ref)
+    pvs, pss, om, er = ds.dv.body_unpack(rhs, nunk)
+    assert torch.equal(pvs, rows[0]) and torch.equal(pss, rows[1] if nunk == 2 else 0 * rows[0])
+    assert torch.equal(om, rhs[-1]) and torch.equal(er, rhs[-1])
+    ovs, oss = ds.dv.body_strengths(vs, ss, w, tx, ty, ddx, ddy)
+    ui, vi = -w * ddy, w * ddx
+    assert torch.equal(ovs, vs + -1.0 * (ui * tx + vi * ty))
+    assert torch.equal(oss, ss + -1.0 * (ui * ty - vi * tx))
