@@ -9,7 +9,8 @@
 // The interaction is recomputed pair by pair and never stored. One lane per source, the point
 // targets (with their upstream gradients) staged through LDS; fp64 throughout. When there are
 // too few sources to fill the GPU the target range is split into chunks whose partials are
-// summed in a fixed order.
+// summed in a fixed order. From kTreePairsAdjoint pairs the Gaussian's adjoint takes the pairs beyond
+// the compact cutoff by clusters of targets instead, to rounding (treecode.hip).
 #include <algorithm>
 
 #include "nbody.h"

@@ -11,7 +11,8 @@
 //
 // Plain form (fp64): every lane owns TPL targets and runs an unrolled loop over a 256-source
 // tile staged in LDS with coalesced loads; all lanes of a wave read the same source (an LDS
-// broadcast). Sums are fp64 per target.
+// broadcast). Sums are fp64 per target. From kTreePairs pairs the Gaussian's velocity sum takes the
+// sources beyond its compact cutoff by clusters instead, to rounding (treecode.hip).
 //
 // Split form (fp32 pair arithmetic): the sorted sources are cut into groups of kGroup
 // sources, and stored as fp32 offsets from their group's fp64 centroid.
