@@ -163,28 +163,6 @@ void adjoint_kernel(
   }
 }
 
-__global__ __launch_bounds__(kBlock) void reduce4_kernel(int64_t nchunk, int64_t n,
-                                                         const double* __restrict__ part,
-                                                         double* __restrict__ ox,
-                                                         double* __restrict__ oy,
-                                                         double* __restrict__ os,
-                                                         double* __restrict__ orr) {
-  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (j >= n) return;
-  double a = 0.0, b = 0.0, c = 0.0, e = 0.0;
-  const int64_t stride = nchunk * n;
-  for (int64_t k = 0; k < nchunk; ++k) {
-    a += part[k * n + j];
-    b += part[stride + k * n + j];
-    c += part[2 * stride + k * n + j];
-    e += part[3 * stride + k * n + j];
-  }
-  ox[j] += a;
-  oy[j] += b;
-  os[j] += c;
-  orr[j] += e;
-}
-
 template <int CORE>
 void launch_adj(dim3 grid, hipStream_t s, int64_t ns, const double* sx, const double* sy,
                 const double* ss, const double* sr, int64_t nt, const double* tx,
@@ -234,9 +212,7 @@ int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx
   kt.stop();
   O2D_LAUNCH_CHECK();
   if (!direct) {
-    reduce4_kernel<<<(unsigned)((ns + kBlock - 1) / kBlock), kBlock, 0, s>>>(nchunk, ns, ox, gx, gy,
-                                                                             gs, gr);
-    O2D_LAUNCH_CHECK();
+    O2D_TRY(reduce_chunks(s, nchunk, ns, nullptr, 4, ox, gx, gy, gs, gr));
   }
   return 0;
 }

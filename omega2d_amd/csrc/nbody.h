@@ -56,10 +56,10 @@ int lu_solve_dev(Device* d, hipStream_t s, int n, const double* lu, const int* p
 int matvec_dev(Device* d, hipStream_t s, int n, const double* a, const double* b, double* x);
 int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* x);
 
-// ou[order[i]] += sum over chunks c of pu[c*nt + i], and ov, ow alike (pw, ow may be null; order null: the
-// identity); nbody.hip
-int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* order, const double* pu,
-                  const double* pv, const double* pw, double* ou, double* ov, double* ow);
+// o_f[order[i]] += sum over chunks c of part[(f nchunk + c) nt + i], for the nf (2 to 4) components f
+// (order null: the identity); nbody.hip
+int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* order, int nf,
+                  const double* part, double* o0, double* o1, double* o2, double* o3);
 
 int rk_move_dev(hipStream_t s, int64_t n, double dt, int nstage, const double* w,
                 const double* const* u, const double* const* v, const double* x0,

@@ -448,45 +448,56 @@ void nbody32_kernel(
   }
 }
 
-// out[order[i]] += sum over chunks c of part[c*nt + i] (order null: the identity). A workgroup takes
-// 64 targets, its four waves a quarter of the chunks each, in order, and their sums are added in
-// wave order. Bound by the latency of its loads: with a thread per target, 10,000 targets kept 157
-// waves busy with a loop over 40 chunks each (7.8 us, 4.9 us so).
+struct Outputs {
+  double* f[4];
+};
+
+// out.f[f][order[i]] += sum over chunks c of part[(f nchunk + c) nt + i] for the nf components (order
+// null: the identity). SPLIT: a workgroup takes 64 targets, its four waves a quarter of the chunks each,
+// in order, and their sums are added in wave order, a component by each wave; else a thread per
+// target. Bound by the latency of its loads where targets are few (10,000 targets, 40 chunks: 7.8 us
+// with a thread per target, 4.9 split), by bandwidth where they are many and chunks few (250,000
+// targets, 2 chunks of 4 components: 30 us with a thread per target, 39 split).
+template <int NF, bool SPLIT>
 __global__ __launch_bounds__(kBlock) void reduce_chunks_kernel(int64_t nchunk, int64_t nt,
                                                                const uint32_t* __restrict__ order,
-                                                               const double* __restrict__ pu,
-                                                               const double* __restrict__ pv,
-                                                               const double* __restrict__ pw,
-                                                               double* __restrict__ ou,
-                                                               double* __restrict__ ov,
-                                                               double* __restrict__ ow) {
-  constexpr int kWaves = kBlock / 64;
-  __shared__ double sm[3][kWaves][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t i = (int64_t)blockIdx.x * 64 + lane;
+                                                               const double* __restrict__ part,
+                                                               Outputs out) {
+  constexpr int kWaves = SPLIT ? kBlock / 64 : 1;
+  static_assert(!SPLIT || NF <= kWaves, "a component per wave");
+  const int lane = threadIdx.x & 63, wave = SPLIT ? threadIdx.x >> 6 : 0;
+  const int64_t i = SPLIT ? (int64_t)blockIdx.x * 64 + lane : (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const int64_t share = (nchunk + kWaves - 1) / kWaves;
   const int64_t c0 = wave * share, c1 = c0 + share < nchunk ? c0 + share : nchunk;
-  double su = 0.0, sv = 0.0, sw = 0.0;
+  double s[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) s[f] = 0.0;
   if (i < nt) {
 #pragma unroll 4
-    for (int64_t c = c0; c < c1; ++c) {
-      su += pu[c * nt + i];
-      sv += pv[c * nt + i];
-      if (pw) sw += pw[c * nt + i];
-    }
-  }
-  sm[0][wave][lane] = su;
-  sm[1][wave][lane] = sv;
-  sm[2][wave][lane] = sw;
-  __syncthreads();
-  const int f = wave;  // a component per wave
-  if (f > (pw ? 2 : 1) || i >= nt) return;
-  double s = sm[f][0][lane];
+    for (int64_t c = c0; c < c1; ++c)
 #pragma unroll
-  for (int w = 1; w < kWaves; ++w) s += sm[f][w][lane];
-  const int64_t o = order ? (int64_t)order[i] : i;
-  double* out = f == 0 ? ou : (f == 1 ? ov : ow);
-  out[o] += s;
+      for (int f = 0; f < NF; ++f) s[f] += part[(f * nchunk + c) * nt + i];
+  }
+  if constexpr (!SPLIT) {
+    if (i >= nt) return;
+    const int64_t o = order ? (int64_t)order[i] : i;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) out.f[f][o] += s[f];
+  } else {
+    __shared__ double sm[NF][kWaves][64];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) sm[f][wave][lane] = s[f];
+    __syncthreads();
+    if (wave >= NF || i >= nt) return;
+    double t = sm[wave][0][lane];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) t += sm[wave][w][lane];
+    const int64_t o = order ? (int64_t)order[i] : i;
+    double* to = out.f[0];  // by wave, without indexing the argument
+#pragma unroll
+    for (int f = 1; f < NF; ++f) to = wave == f ? out.f[f] : to;
+    to[o] += t;
+  }
 }
 
 // ---------------------------------------------------------------------------- staging
@@ -717,10 +728,18 @@ int gather_targets(hipStream_t s, int core, int64_t n, const uint32_t* order, co
 
 }  // namespace
 
-int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* order, const double* pu,
-                  const double* pv, const double* pw, double* ou, double* ov, double* ow) {
-  reduce_chunks_kernel<<<(unsigned)((nt + 63) / 64), kBlock, 0, s>>>(nchunk, nt, order, pu, pv, pw,
-                                                                     ou, ov, ow);
+int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* order, int nf,
+                  const double* part, double* o0, double* o1, double* o2, double* o3) {
+  const bool split = nchunk >= 8;
+  const unsigned grid = split ? (unsigned)((nt + 63) / 64) : grid1(nt).x;
+  const Outputs out{{o0, o1, o2, o3}};
+#define O2D_REDUCE(NF)                                                                            \
+  split ? reduce_chunks_kernel<NF, true><<<grid, kBlock, 0, s>>>(nchunk, nt, order, part, out)    \
+        : reduce_chunks_kernel<NF, false><<<grid, kBlock, 0, s>>>(nchunk, nt, order, part, out)
+  if (nf == 2) O2D_REDUCE(2);
+  else if (nf == 3) O2D_REDUCE(3);
+  else O2D_REDUCE(4);
+#undef O2D_REDUCE
   O2D_LAUNCH_CHECK();
   return 0;
 }
@@ -846,7 +865,7 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
     kt.stop();
     O2D_LAUNCH_CHECK();
     if (!direct) {
-      O2D_TRY(reduce_chunks(s, cp.nchunk, nt, torder, ou, ov, ow, tu, tv, tw));
+      O2D_TRY(reduce_chunks(s, cp.nchunk, nt, torder, nf, ou, tu, tv, tw, nullptr));
     }
     return 0;
   }
@@ -904,7 +923,7 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
   kt.stop();
   O2D_LAUNCH_CHECK();
   if (!direct) {
-    O2D_TRY(reduce_chunks(s, cp.nchunk, nt, torder, ou, ov, ow, tu, tv, tw));
+    O2D_TRY(reduce_chunks(s, cp.nchunk, nt, torder, nf, ou, tu, tv, tw, nullptr));
   }
   return 0;
 }

@@ -652,7 +652,7 @@ int panels_on_points_dev(Device* d, hipStream_t s, int64_t nnodes, const double*
     kt.stop();
     O2D_LAUNCH_CHECK();
     if (!direct) {
-      O2D_TRY(reduce_chunks(s, nchunk, nt, torder, ou, ov, nullptr, tu, tv, nullptr));
+      O2D_TRY(reduce_chunks(s, nchunk, nt, torder, 2, ou, tu, tv, nullptr, nullptr));
     }
     return 0;
   }
@@ -682,7 +682,7 @@ int panels_on_points_dev(Device* d, hipStream_t s, int64_t nnodes, const double*
   kt.stop();
   O2D_LAUNCH_CHECK();
   if (!direct) {
-    O2D_TRY(reduce_chunks(s, nchunk, nt, nullptr, ou, ov, nullptr, tu, tv, nullptr));
+    O2D_TRY(reduce_chunks(s, nchunk, nt, nullptr, 2, ou, tu, tv, nullptr, nullptr));
   }
   return 0;
 }

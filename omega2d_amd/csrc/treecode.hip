@@ -967,27 +967,6 @@ __global__ __launch_bounds__(kGroupBlock, 4) void tree_group_kernel(
   }
 }
 
-// outputs[torder[i]] += the shares' partial sums, in order (nf components)
-__global__ __launch_bounds__(kBlock) void tree_reduce_kernel(int64_t nt, int ksplit, int nf,
-                                                             const double* __restrict__ part,
-                                                             const uint32_t* __restrict__ torder,
-                                                             double* __restrict__ o0,
-                                                             double* __restrict__ o1,
-                                                             double* __restrict__ o2,
-                                                             double* __restrict__ o3) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= nt) return;
-  const uint32_t o = torder[i];
-  double* const out[4] = {o0, o1, o2, o3};
-#pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    if (f >= nf) break;
-    double s = 0.0;
-    for (int k = 0; k < ksplit; ++k) s += part[((int64_t)f * ksplit + k) * nt + i];
-    out[f][o] += s;
-  }
-}
-
 inline unsigned blocks(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
 struct Problem {
@@ -1147,9 +1126,7 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
   kt.stop();
   O2D_LAUNCH_CHECK();
   if (part) {
-    tree_reduce_kernel<<<blocks(nt), kBlock, 0, s>>>(nt, ga.ksplit, nf, part, torder, q.o0, q.o1,
-                                                     q.o2, q.o3);
-    O2D_LAUNCH_CHECK();
+    O2D_TRY(reduce_chunks(s, ga.ksplit, nt, torder, nf, part, q.o0, q.o1, q.o2, q.o3));
   }
   return 0;
 }
