@@ -448,22 +448,23 @@ void nbody32_kernel(
   }
 }
 
+constexpr int kReduceT = 1024;  // threads of the split sum over chunks
+
 struct Outputs {
   double* f[4];
 };
 
 // out.f[f][order[i]] += sum over chunks c of part[(f nchunk + c) nt + i] for the nf components (order
-// null: the identity). SPLIT: a workgroup takes 64 targets, its four waves a quarter of the chunks each,
-// in order, and their sums are added in wave order, a component by each wave; else a thread per
-// target. Bound by the latency of its loads where targets are few (10,000 targets, 40 chunks: 7.8 us
-// with a thread per target, 4.9 split), by bandwidth where they are many and chunks few (250,000
+// null: the identity). SPLIT: a workgroup takes 64 targets, its 16 waves a share of the chunks each, in
+// order, and their sums are added in wave order, a component by each wave; else a thread per target.
+// Bound by the latency of its loads where targets are few (10,000 targets, 40 chunks: 7.8 us with a
+// thread per target, 4.5 split; 100 targets, 938 chunks: 24 with four waves, 15 with 16), by bandwidth where they are many and chunks few (250,000
 // targets, 2 chunks of 4 components: 30 us with a thread per target, 39 split).
 template <int NF, bool SPLIT>
-__global__ __launch_bounds__(kBlock) void reduce_chunks_kernel(int64_t nchunk, int64_t nt,
-                                                               const uint32_t* __restrict__ order,
-                                                               const double* __restrict__ part,
-                                                               Outputs out) {
-  constexpr int kWaves = SPLIT ? kBlock / 64 : 1;
+__global__ __launch_bounds__(SPLIT ? kReduceT : kBlock) void reduce_chunks_kernel(
+    int64_t nchunk, int64_t nt, const uint32_t* __restrict__ order, const double* __restrict__ part,
+    Outputs out) {
+  constexpr int kWaves = SPLIT ? kReduceT / 64 : 1;
   static_assert(!SPLIT || NF <= kWaves, "a component per wave");
   const int lane = threadIdx.x & 63, wave = SPLIT ? threadIdx.x >> 6 : 0;
   const int64_t i = SPLIT ? (int64_t)blockIdx.x * 64 + lane : (int64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -473,7 +474,7 @@ __global__ __launch_bounds__(kBlock) void reduce_chunks_kernel(int64_t nchunk, i
 #pragma unroll
   for (int f = 0; f < NF; ++f) s[f] = 0.0;
   if (i < nt) {
-#pragma unroll 4
+#pragma unroll 8
     for (int64_t c = c0; c < c1; ++c)
 #pragma unroll
       for (int f = 0; f < NF; ++f) s[f] += part[(f * nchunk + c) * nt + i];
@@ -734,7 +735,7 @@ int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* ord
   const unsigned grid = split ? (unsigned)((nt + 63) / 64) : grid1(nt).x;
   const Outputs out{{o0, o1, o2, o3}};
 #define O2D_REDUCE(NF)                                                                            \
-  split ? reduce_chunks_kernel<NF, true><<<grid, kBlock, 0, s>>>(nchunk, nt, order, part, out)    \
+  split ? reduce_chunks_kernel<NF, true><<<grid, kReduceT, 0, s>>>(nchunk, nt, order, part, out)  \
         : reduce_chunks_kernel<NF, false><<<grid, kBlock, 0, s>>>(nchunk, nt, order, part, out)
   if (nf == 2) O2D_REDUCE(2);
   else if (nf == 3) O2D_REDUCE(3);

@@ -1,4 +1,4 @@
-"""The sum over source or target chunks, with a thread per target (below 8 chunks) and with four waves
+"""The sum over source or target chunks, with a thread per target (below 8 chunks) and with 16 waves
 per 64 targets, for two, three and four components: adding to what is there, at the edges of 64 targets
 and of the waves' shares, against the oracle at the fp64 form's 1e-12 relative L2."""
 import numpy as np
