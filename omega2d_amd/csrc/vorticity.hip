@@ -87,7 +87,7 @@ __device__ __forceinline__ double exp_neg(double x, const double* tab) {
   return ldexp(fma(t, q, t), m);
 }
 
-// the staged record of a source (as vort_kernel stages it)
+// the staged record of a source
 __device__ __forceinline__ VSrc vsrc_of(double x, double y, double s, double r) {
   const double r2 = r * r;
   const double rr = 1.0 / r2;
