@@ -765,7 +765,9 @@ __global__ __launch_bounds__(kGroupBlock, 4) void tree_group_kernel(
     // nearer the limit keep all p and the others stay well below its truncation
     int terms = p;
     if (far && b2d >= rfar) {
-      const float ratio = __builtin_amdgcn_logf((float)(c.z * c.z) / (float)b2d);
+      // the quotient in fp64: either square alone can leave the range of a float
+      const float ratio =
+          __builtin_amdgcn_logf((float)(c.z * c.z * __builtin_amdgcn_rcp(b2d)));
       const float need = __builtin_ceilf(logtail / ratio);
       terms = need < (float)p ? (need > 2.0f ? (int)need : 2) : p;
       terms = terms < p ? terms : p;
