@@ -67,11 +67,17 @@ constexpr int kStackSpare = 3 * kMaxLevels;  // what opening one cell at a time 
 // on themselves and 9,973 tracers, 0.36, whose remainder is 6e-15, 1.59 ms; the error against 64
 // bits did not move, 5e-16, a quarter of the pair by pair sum's.)
 constexpr double kExactTheta = 1.0 / 3.0;
-// local expansions add a truncation of their own: they take cells from a little further away
-constexpr double kLocalShare = 0.85;
-// and groups take cells from a little further than theta says, so that the sum over many more
-// cells than the coarser groups of an earlier form used keeps its error
-constexpr double kThetaShare = 0.955;
+// The remainder of a cell at distance d is (r / d)^p of its contribution, at most theta^p. A sum takes
+// many cells near the limit, and truncates some in more than one way, so each way keeps to a share of
+// theta^p: the moments of cells at the limit of groups of 64 targets and of 16 (smaller, so that more of
+// their targets are near it), the orders left out of cells further away, and local expansions. From
+// kShareOrder on a share is kept by taking cells from a little further than theta says; below, where
+// that little is much, cells near the limit use up to kSpareOrders more than p.
+constexpr double kShare64 = 0.275, kShare16 = 0.08, kShareTail = 0.02, kShareLocal = 0.0105;
+constexpr int kShareOrder = 28, kSpareOrders = 6;
+inline int kept_orders(int p) {
+  return p + std::max(0, std::min(kSpareOrders, kShareOrder - p));
+}
 // waves per CU the group kernel aims for by sharing a group's cells and leaves out: every share
 // opens the same cells, so more of them cost more (1M particles: 32 and 64 equal; 10,000 tracers
 // in groups of 16: 264 us at 16, 369 at 32)
@@ -612,7 +618,9 @@ struct GroupArgs {
   int ksplit;      // waves per group: wave k takes every ksplit-th far cell and leaf
   uint32_t start;  // starting cells when there are no super groups (or one gave up): start ..
   uint32_t nstart; // start + nstart - 1, all of one level
-  double theta, tol;
+  double theta;    // cells are far from radius / theta on
+  float logtail;   // twice the logarithm (base 2) of the remainder that cells further away keep to
+  double tol;
 };
 
 // One wave per G targets and share (blockIdx.y) of their far cells and leaves; every share opens
@@ -649,9 +657,8 @@ __global__ __launch_bounds__(kGroupBlock, 4) void tree_group_kernel(
   const double x0 = lanes_min<G>(x), x1 = lanes_max<G>(x);
   const double y0 = lanes_min<G>(y), y1 = lanes_max<G>(y);
   const double wt = __any(!(wmine < INFINITY)) ? INFINITY : lanes_max<G>(wmine);
-  const double itheta = 1.0 / (kThetaShare * a.theta);
+  const double itheta = 1.0 / a.theta;
   const int p = a.p;
-  const float logtail = 2.0f * (float)p * __builtin_amdgcn_logf((float)(0.9 * a.theta));
   // pairs: velocity u, v; adjoint dJ/ds, dJ/dx, dJ/dy, dJ/dr (the last three over the strength)
   double n0 = 0.0, n1 = 0.0, n2 = 0.0, n3 = 0.0;
   double2 S = make_double2(0.0, 0.0), S2 = S;  // far cells: S, and for the adjoint S2
@@ -761,14 +768,14 @@ __global__ __launch_bounds__(kGroupBlock, 4) void tree_group_kernel(
       }
     }
     const bool far = (fbits >> lane) & 1ull;
-    // orders that this cell needs at its distance: (r / d)^terms <= (0.9 theta)^p, so that cells
+    // orders that this cell needs at its distance: (r / d)^terms <= kShareTail theta^p, so that cells
     // nearer the limit keep all p and the others stay well below its truncation
     int terms = p;
     if (far && b2d >= rfar) {
       // the quotient in fp64: either square alone can leave the range of a float
       const float ratio =
           __builtin_amdgcn_logf((float)(c.z * c.z * __builtin_amdgcn_rcp(b2d)));
-      const float need = __builtin_ceilf(logtail / ratio);
+      const float need = __builtin_ceilf(a.logtail / ratio);
       terms = need < (float)p ? (need > 2.0f ? (int)need : 2) : p;
       terms = terms < p ? terms : p;
     }
@@ -973,9 +980,9 @@ inline unsigned blocks(int64_t n) { return (unsigned)((n + kBlock - 1) / kBlock)
 
 struct Problem {
   int core;
-  int p;
+  int order;  // the remainder of a far cell stays below theta^order
+  int p;      // orders kept of a cell and of a local expansion
   double theta, tol;
-  double theta_local;  // for local expansions, whose truncation adds to the moments'
   // sources, and their charges: strength and radius (velocity) or gv and gu (adjoint)
   int64_t ns;
   const double *sx, *sy, *sa, *sb;
@@ -986,6 +993,15 @@ struct Problem {
   int timed;  // kernel class of the evaluation
 };
 
+// log2 of the given share of theta^order
+inline double remainder(const Problem& q, double share) {
+  return q.order * std::log2(q.theta) + std::log2(share) * std::max(1.0, (double)q.order / kShareOrder);
+}
+// the r / d at which q.p orders leave that, at most theta
+inline double limit(const Problem& q, double share) {
+  return std::min(q.theta, std::exp2(remainder(q, share) / q.p));
+}
+
 template <int CORE, bool ADJ>
 void launch_eval(const Problem& q, hipStream_t s, int64_t nsuper, const GroupArgs& ga,
                  const Trg* trg, const uint32_t* torder, const double4* head, const uint2* kids,
@@ -993,7 +1009,7 @@ void launch_eval(const Problem& q, hipStream_t s, int64_t nsuper, const GroupArg
                  double* part) {
   if (nsuper)
     tree_super_kernel<CORE, ADJ><<<(unsigned)nsuper, kSuperBlock, 0, s>>>(
-        q.nt, trg, head, kids, mom, root, q.theta_local, q.tol, super, local, front);
+        q.nt, trg, head, kids, mom, root, limit(q, kShareLocal), q.tol, super, local, front);
   const int64_t groups = (q.nt + ga.g - 1) / ga.g;
   const dim3 grid((unsigned)((groups + kGroupWaves - 1) / kGroupWaves), (unsigned)ga.ksplit);
   auto* sup = nsuper ? super : nullptr;
@@ -1074,7 +1090,6 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
   GroupArgs ga{};
   ga.nt = nt;
   ga.p = q.p;
-  ga.theta = q.theta;
   ga.tol = q.tol;
   const int64_t nsup = (nt + kSuper - 1) / kSuper;
   const int64_t nsuper = nsup >= kMinSupers ? nsup : 0;
@@ -1083,6 +1098,8 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
   // targets are near (65,536 tracers among 1M particles: 0.47 ms in groups of 16, 0.51 of 32,
   // 0.72 of 64; the particles on themselves 3.2, 2.4 and 2.0 ms)
   ga.g = nt < ns / 4 ? 16 : 64;
+  ga.theta = limit(q, ga.g == 64 ? kShare64 : kShare16);
+  ga.logtail = (float)(2.0 * remainder(q, kShareTail));
   const int64_t groups = (nt + ga.g - 1) / ga.g, want = (int64_t)(ga.g == 64 ? kWaves64 : kWaves16) * d->num_cu;
   ga.ksplit = groups >= want ? 1 : (int)std::min<int64_t>(32, (want + groups - 1) / groups);
   // starting cells without a frontier: the lowest level that is tested in one go
@@ -1139,7 +1156,7 @@ int tree_dev(Device* d, hipStream_t s, int core, double theta, int p, double tol
              const double* sx, const double* sy, const double* ss, const double* sr, int64_t nt,
              const double* tx, const double* ty, const double* tr, double* tu, double* tv) {
   if (ns == 0 || nt == 0) return 0;
-  const Problem q{core, p, theta, tol, kLocalShare * theta, ns, sx, sy, ss, sr, nt, tx, ty, tr, nullptr,
+  const Problem q{core, p, kept_orders(p), theta, tol, ns, sx, sy, ss, sr, nt, tx, ty, tr, nullptr,
                   tu, tv, nullptr, nullptr, O2D_KT_TREE_EVAL};
   return tree_run<false>(d, s, q);
 }
@@ -1147,7 +1164,7 @@ int tree_dev(Device* d, hipStream_t s, int core, double theta, int p, double tol
 int gauss_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const double* sy,
                    const double* ss, const double* sr, int64_t nt, const double* tx,
                    const double* ty, const double* tr, double* tu, double* tv) {
-  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kExactTheta, 0.0, kLocalShare * kExactTheta, ns, sx, sy, ss, sr, nt,
+  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kMaxP, kExactTheta, 0.0, ns, sx, sy, ss, sr, nt,
                   tx, ty, tr, nullptr, tu, tv, nullptr, nullptr,
                   tr ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT};
   return tree_run<false>(d, s, q);
@@ -1157,7 +1174,7 @@ int gauss_adjoint_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* s
                            const double* sy, const double* ss, const double* sr, int64_t nt,
                            const double* tx, const double* ty, const double* gu,
                            const double* gv, double* gx, double* gy, double* gs, double* gr) {
-  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kExactTheta, 0.0, kLocalShare * kExactTheta, nt, tx, ty, gv, gu, ns,
+  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kMaxP, kExactTheta, 0.0, nt, tx, ty, gv, gu, ns,
                   sx, sy, sr, ss, gs, gx, gy, gr, O2D_KT_ADJOINT};
   return tree_run<true>(d, s, q);
 }
