@@ -276,6 +276,8 @@ int bem_factor_dev(Device* d, hipStream_t s, int64_t n, const double* A, int64_t
   O2D_TRY(slot(d, kLU, sizeof(double) * n * n, s, &lu));
   O2D_TRY(slot(d, kPivots, sizeof(rocblas_int) * n, s, &piv));
   O2D_TRY(slot(d, kInfo, sizeof(rocblas_int), s, &info));
+  void* scratch;  // all that any solve with these factors takes, so that none of them moves it
+  O2D_TRY(slot(d, kSolveTmp, solve_scratch(n), s, &scratch));
   O2D_HIP(hipMemcpy2DAsync(lu, sizeof(double) * n, A, sizeof(double) * lda, sizeof(double) * n, n,
                            hipMemcpyDeviceToDevice, s));
   rocblas_handle h;
@@ -315,14 +317,25 @@ __global__ __launch_bounds__(kBlock) void identity_kernel(int64_t n, double* __r
 // is one matrix-vector product (0.013 ms at 2049, against 0.27 by two triangular solves). A body that
 // does not move keeps its inverse for the whole run; a body in relative motion, refactored every
 // step and solved once per Runge-Kutta stage, never builds it: its two or three solves cost less.
-constexpr int kSolvesBeforeInverse = 3;
+// Beyond lu_max_order, where the library's triangular solves cost as much as the inverse, the second
+// solve builds it. A solve under stream capture allocates nothing and calls no library routine up to
+// lu_max_order: it goes by the factors unless the inverse is there.
+constexpr int kSolvesBeforeInverse = 3, kLibrarySolvesBeforeInverse = 1;
+
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
+  return st == hipStreamCaptureStatusActive;
+}
 
 int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* x) {
   if (!d->lu_ready || d->lu_n != n)
     return fail(O2D_ERR_STATE, "no LU factors of size %lld (factor first)", (long long)n);
-  rocblas_handle h;
-  O2D_TRY(blas_of(d, s, &h));
-  if (!d->inv_ready && d->lu_solves >= kSolvesBeforeInverse) {
+  const bool own = n <= lu_max_order();
+  if (!d->inv_ready && d->lu_solves >= (own ? kSolvesBeforeInverse : kLibrarySolvesBeforeInverse) &&
+      !(own && capturing(s))) {
+    rocblas_handle h;
+    O2D_TRY(blas_of(d, s, &h));
     void* inv;
     O2D_TRY(slot(d, kInv, sizeof(double) * n * n, s, &inv));
     const int64_t nn = n * n;
@@ -339,9 +352,11 @@ int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* 
   ++d->lu_solves;
   if (d->inv_ready)
     return matvec_dev(d, s, (int)n, static_cast<const double*>(d->buf[kInv]), b, x);
-  if (n <= lu_max_order())
+  if (own)
     return lu_solve_dev(d, s, (int)n, static_cast<const double*>(d->buf[kLU]),
                         static_cast<const int*>(d->buf[kLuPerm]), b, x);
+  rocblas_handle h;
+  O2D_TRY(blas_of(d, s, &h));
   if (x != b) O2D_HIP(hipMemcpyAsync(x, b, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   if (rocsolver_dgetrs(h, rocblas_operation_none, (rocblas_int)n, 1, static_cast<double*>(d->buf[kLU]),
                        (rocblas_int)n, static_cast<const rocblas_int*>(d->buf[kPivots]), x,

@@ -167,6 +167,12 @@ inline int blocks_of(int64_t n) { return (int)((n + kSB - 1) / kSB); }
 
 }  // namespace
 
+// two vectors for the block substitution, one per chunk of columns for the product; the same for both,
+// so that the slot stays where it is from one solve to the next (a captured solve keeps its address)
+size_t solve_scratch(int64_t n) {
+  return sizeof(double) * std::max<int64_t>(2, (n + kChunk - 1) / kChunk) * n;
+}
+
 // the diagonal inverses of the factors lu (n x n, leading dimension n), into the kLuDinv slot
 int lu_prepare_solve(Device* d, hipStream_t s, int n, const double* lu) {
   const int nblk = blocks_of(n);
@@ -182,7 +188,7 @@ int lu_solve_dev(Device* d, hipStream_t s, int n, const double* lu, const int* p
                  const double* b, double* x) {
   const int nblk = blocks_of(n);
   void* p;
-  O2D_TRY(slot(d, kSolveTmp, sizeof(double) * 2 * n, s, &p));
+  O2D_TRY(slot(d, kSolveTmp, solve_scratch(n), s, &p));
   double *r = static_cast<double*>(p), *y = r + n;
   const double* dl = static_cast<const double*>(d->buf[kLuDinv]);
   const double* du = dl + (int64_t)nblk * kSB * kSB;
@@ -207,7 +213,7 @@ int lu_solve_dev(Device* d, hipStream_t s, int n, const double* lu, const int* p
 int matvec_dev(Device* d, hipStream_t s, int n, const double* a, const double* b, double* x) {
   const int nchunk = (n + kChunk - 1) / kChunk;
   void* p;
-  O2D_TRY(slot(d, kSolveTmp, sizeof(double) * (int64_t)nchunk * n, s, &p));
+  O2D_TRY(slot(d, kSolveTmp, solve_scratch(n), s, &p));
   double* part = static_cast<double*>(p);
   matvec_kernel<<<dim3((n + kBlock - 1) / kBlock, nchunk), kBlock, 0, s>>>(n, a, b, part);
   O2D_LAUNCH_CHECK();

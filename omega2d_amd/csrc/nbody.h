@@ -52,6 +52,8 @@ int lu_factor_dev(Device* d, hipStream_t s, int n, double* A, int lda, int* ipiv
 int lu_prepare_solve(Device* d, hipStream_t s, int n, const double* lu);
 int lu_solve_dev(Device* d, hipStream_t s, int n, const double* lu, const int* perm,
                  const double* b, double* x);
+// bytes of the kSolveTmp slot that lu_solve_dev and matvec_dev take for order n
+size_t solve_scratch(int64_t n);
 // x = A b, A n x n column-major
 int matvec_dev(Device* d, hipStream_t s, int n, const double* a, const double* b, double* x);
 int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* x);

@@ -50,8 +50,8 @@ struct Device {
   // LU factors of the last matrix given to o2d_hip_bem_factor_*
   int64_t lu_n = 0;
   bool lu_ready = false;
-  // solves made with the current factors; from the second one on, the explicit inverse
-  // (built once from the factors) turns each solve into one matrix-vector product
+  // solves made with the current factors; after a few of them (bem.hip) the explicit inverse, built
+  // once from the factors, turns each solve into one matrix-vector product
   int64_t lu_solves = 0;
   bool inv_ready = false;
   void* blas = nullptr;  // rocblas_handle
