@@ -39,6 +39,16 @@ struct Packed {
   }
 };
 
+// Waits for the stream where a call that copies from or to the page-locked memory ends early: the next
+// call fills that memory again.
+struct Drain {
+  hipStream_t s;
+  bool pending = true;
+  ~Drain() {
+    if (pending) (void)hipStreamSynchronize(s);
+  }
+};
+
 // particles on points, packed: the inputs, then the outputs (which are inputs too: sums add to them)
 template <class T>
 int points_packed(Device* d, hipStream_t s, const o2d_env* env, int64_t ns, const T* sx, const T* sy,
@@ -69,6 +79,7 @@ int points_packed(Device* d, hipStream_t s, const o2d_env* env, int64_t ns, cons
   for (int k = 0; k < 3; ++k)
     if (out[k]) std::memcpy(p.host + ot[k], out[k], sizeof(T) * nt);
   float* f = nullptr;
+  Drain drain{s};
   if constexpr (sizeof(T) == sizeof(float)) {
     O2D_TRY(slot(d, kStageF0, sizeof(float) * p.n, s, &v));
     f = static_cast<float*>(v);
@@ -94,6 +105,7 @@ int points_packed(Device* d, hipStream_t s, const o2d_env* env, int64_t ns, cons
                            hipMemcpyDeviceToHost, s));
   }
   O2D_HIP(hipStreamSynchronize(s));
+  drain.pending = false;
   for (int k = 0; k < 3; ++k)
     if (out[k]) std::memcpy(out[k], p.host + ot[k], sizeof(T) * nt);
   return 0;
