@@ -4,15 +4,18 @@
 // of pairs ran as a merge sort at these sizes (a block sort and up to sixteen merge launches,
 // 110 us for 200k or 1M points, 45 us for 10k), after three or four launches that made the keys.
 //
-// Up to kRankMax keys one launch does everything, box included, by counting for each key the keys
-// that go before it (rank_kernel). Beyond, least significant digits first, 8 bits a pass: the box (one launch), the keys with the first digit's
-// tile histograms (one launch), then one launch per digit. A scatter launch sums the
-// histogram rows of the tiles before its own (every tile reads all rows from cache, which at
-// kMaxTiles rows is a fraction of the launch's own cost), ranks its keys within the tile by
-// wave-wide digit matches (stable: a wave's keys are consecutive), and counts the next digit of
-// each key it places into the row of the tile it places it in, so no launch only counts.
-// Counting uses integer atomics: sums do not depend on their order, and neither does the result.
-// Arrays past kMaxTiles tiles (4M keys) go to the library sort, whose cost is then bandwidth.
+// Up to kRankMax keys one launch does everything, box included, by counting for each key the keys that
+// go before it (rank_kernel). Beyond, least significant digits first, 8 bits a pass: the box (one
+// launch), the keys with the first digit's tile histograms (one launch), then one launch per digit. A
+// scatter launch sums the histogram rows of the tiles before its own (every tile reads all rows from
+// cache), ranks its keys within the tile by wave-wide digit matches (stable: a wave's keys are
+// consecutive), and, in small tiles, counts the next digit of each key it places into the row of the
+// tile it places it in, so no launch only counts. Counting uses integer atomics: sums do not depend on
+// their order, and neither does the result.
+// Arrays past kTiledMax keys go to the library sort, whose cost is then bandwidth: 2,000,000 keys take
+// 148 us tiled and 157 by the library, 1,048,577 114 and 144, but 3,000,000 224 and 171. (With the next
+// digit's count compiled into the large tiles' launches, where it is never taken, 16 keys a thread
+// spilled: 250 us at 2,000,000.)
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
@@ -31,7 +34,7 @@ constexpr int kBoxBlocks = 256;  // partial boxes
 constexpr int kST = 512;         // threads of a key or scatter workgroup
 constexpr int kSW = kST / 64;
 constexpr int kDigits = 256;
-constexpr int kMaxTiles = 512;
+constexpr int64_t kTiledMax = 1 << 21;
 constexpr int kCountItems = 2;   // keys per thread up to which a pass counts the next digit
 constexpr int kRankT = 1024;     // threads of a rank workgroup
 constexpr int kRankW = kRankT / 64;
@@ -224,7 +227,8 @@ __global__ __launch_bounds__(kST) void hist_kernel(int64_t n, int shift,
 
 // one digit pass of a tile: keys (and their values; FIRST: the value is the index) to their
 // places by digit (key >> shift) & 255; tab holds this digit's rows, next (unless null) takes
-// the next digit's counts. keys_out null: the keys are not needed any more.
+// the next digit's counts (up to kCountItems keys a thread). keys_out null: the keys are not needed any
+// more.
 template <int ITEMS, bool FIRST>
 __global__ __launch_bounds__(kST) void scatter_kernel(int64_t n, int ntiles, int shift,
                                                       const uint32_t* __restrict__ keys_in,
@@ -311,7 +315,7 @@ __global__ __launch_bounds__(kST) void scatter_kernel(int64_t n, int ntiles, int
       if (keys_out) keys_out[dst] = key[k];
       vals_out[dst] = val[k];
     }
-    if (next) {
+    if (ITEMS <= kCountItems && next) {
       // lanes with equal digits go to consecutive places; those that also share the next digit
       // and the destination tile count with one atomic (keys of clustered points share their
       // high digits)
@@ -336,12 +340,12 @@ __global__ __launch_bounds__(kST) void scatter_kernel(int64_t n, int ntiles, int
 // and the equal ones before it. Every workgroup makes all keys in LDS and places EACH of them, one to
 // a lane; its waves share the blocks of 64 keys to compare with, and the 64 / EACH lanes with the same
 // key share a block. Bound by latency up to 4,096 keys (7 us is the launch, two dependent passes over
-// the points and their box), beyond by the integer units and LDS together: 8.4 us at 1,531 keys,
-// 11.9 at 4,096, 18.3 at 8,192, 25.3 at 10,000 and 28.9 at 12,288. A one-workgroup radix sort in LDS took 15.4 us at
-// 1,531 (four digits, three barriers each), the six launches of the tiled passes 30 us and their gaps
-// at 10,000; here 16,384 keys take 37 us, and n^2 comparisons no longer pay. Comparing 64 keys with
-// one scalar key and counting the mask's bits took 40 us at 10,000 (scalar registers), two keys a lane
-// 28.
+// the points and their box), beyond by the integer units and LDS together: 8.4 us at 1,531 keys, 11.9
+// at 4,096, 18.3 at 8,192, 25.3 at 10,000 and 28.9 at 12,288. A one-workgroup radix sort in LDS took
+// 15.4 us at 1,531 (four digits, three barriers each), the six launches of the tiled passes 30 us and
+// their gaps at 10,000; here 16,384 keys take 37 us, and n^2 comparisons no longer pay. Comparing 64
+// keys with one scalar key and counting the mask's bits took 40 us at 10,000 (scalar registers), two
+// keys a lane 28.
 template <int KIND, int ITEMS, int EACH>
 __global__ __launch_bounds__(kRankT) void rank_kernel(KeyGen g, int n,
                                                       uint32_t* __restrict__ keys_out,
@@ -407,9 +411,26 @@ __global__ __launch_bounds__(kRankT) void rank_kernel(KeyGen g, int n,
   vals_out[c] = (uint32_t)i;
 }
 
-__global__ __launch_bounds__(kBoxBlock) void iota_kernel(int64_t n, uint32_t* __restrict__ v) {
-  const int64_t i = (int64_t)blockIdx.x * kBoxBlock + threadIdx.x;
-  if (i < n) v[i] = (uint32_t)i;
+// the keys and their indices, for the library sort
+template <int KIND>
+__global__ __launch_bounds__(kBoxBlock) void pair_kernel(KeyGen g, int64_t n,
+                                                         const Box* __restrict__ part, int npart,
+                                                         uint32_t* __restrict__ keys,
+                                                         uint32_t* __restrict__ vals) {
+  __shared__ Box sm[kBoxBlock / 64];
+  Box b = empty_box();
+  if (KIND != kNode && g.bbox) {
+    for (int p = threadIdx.x; p < npart; p += kBoxBlock)
+      grow(b, part[p].x0, part[p].y0, part[p].x1, part[p].y1);
+    b = block_box<kBoxBlock / 64>(b, sm);
+  }
+  double x0, y0, inv;
+  key_frame<KIND>(g, b, x0, y0, inv);
+  for (int64_t i = (int64_t)blockIdx.x * kBoxBlock + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * kBoxBlock) {
+    keys[i] = make_key<KIND>(g, b, x0, y0, inv, i);
+    vals[i] = (uint32_t)i;
+  }
 }
 
 // 16 keys a workgroup while that leaves no more than one for each of 256 compute units, then 32 or 64
@@ -493,11 +514,6 @@ int sort_order(Device* d, hipStream_t s, Workspace* ws, int64_t n, const KeyGen&
     O2D_LAUNCH_CHECK();
     return 0;
   }
-  // tiles of 1,024 to 8,192 keys: enough of them to spread a pass over the chip, few enough
-  // that every tile can sum the rows of all
-  const int items = n <= (1 << 16) ? 2 : (n <= (1 << 18) ? 4 : (n <= (1 << 20) ? 8 : 16));
-  const int64_t ntiles = (n + (int64_t)kST * items - 1) / ((int64_t)kST * items);
-  const bool lib = ntiles > kMaxTiles;
   void *kt, *vt, *tab = nullptr, *bp = nullptr;
   O2D_TRY(take(d, ws, kKeysA, n * sizeof(uint32_t), s, &kt));
   O2D_TRY(take(d, ws, kOrderA, n * sizeof(uint32_t), s, &vt));
@@ -511,17 +527,24 @@ int sort_order(Device* d, hipStream_t s, Workspace* ws, int64_t n, const KeyGen&
   const Box* part = static_cast<const Box*>(bp);
   uint32_t* k0 = static_cast<uint32_t*>(kt);
   uint32_t* v0 = static_cast<uint32_t*>(vt);
-  O2D_TRY(take(d, ws, kSortTab, sizeof(uint32_t) * kDigits * (size_t)ntiles * (size_t)npass, s,
-               &tab));
-  uint32_t* tb = static_cast<uint32_t*>(tab);
-  if (!lib) {
+  if (n <= kTiledMax) {
+    // tiles of 1,024 to 8,192 keys: enough of them to spread a pass over the chip, few enough (256)
+    // that every tile can sum the rows of all
+    const int items = n <= (1 << 16) ? 2 : (n <= (1 << 18) ? 4 : (n <= (1 << 20) ? 8 : 16));
+    const int64_t ntiles = (n + (int64_t)kST * items - 1) / ((int64_t)kST * items);
+    O2D_TRY(take(d, ws, kSortTab, sizeof(uint32_t) * kDigits * (size_t)ntiles * (size_t)npass, s, &tab));
+    uint32_t* tb = static_cast<uint32_t*>(tab);
     if (items == 2) return sort_tiles<2>(s, g, n, npass, part, npart, keys_out, order_out, k0, v0, tb, want_keys);
     if (items == 4) return sort_tiles<4>(s, g, n, npass, part, npart, keys_out, order_out, k0, v0, tb, want_keys);
     if (items == 8) return sort_tiles<8>(s, g, n, npass, part, npart, keys_out, order_out, k0, v0, tb, want_keys);
     return sort_tiles<16>(s, g, n, npass, part, npart, keys_out, order_out, k0, v0, tb, want_keys);
   }
-  launch_keys<16>(s, g, n, (int)ntiles, 1, part, npart, k0, tb);
-  iota_kernel<<<(unsigned)((n + kBoxBlock - 1) / kBoxBlock), kBoxBlock, 0, s>>>(n, v0);
+  const unsigned blocks = 4096;
+  switch (g.kind) {
+    case kMorton32: pair_kernel<kMorton32><<<blocks, kBoxBlock, 0, s>>>(g, n, part, npart, k0, v0); break;
+    case kMorton16: pair_kernel<kMorton16><<<blocks, kBoxBlock, 0, s>>>(g, n, part, npart, k0, v0); break;
+    default: pair_kernel<kNode><<<blocks, kBoxBlock, 0, s>>>(g, n, part, npart, k0, v0); break;
+  }
   O2D_LAUNCH_CHECK();
   size_t tbytes = 0;
   O2D_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tbytes, k0, keys_out, v0, order_out, (int)n,
