@@ -9,9 +9,10 @@
 // The interaction is recomputed pair by pair and never stored. One lane per source, the point
 // targets (with their upstream gradients) staged through LDS; fp64 throughout. When there are
 // too few sources to fill the GPU the target range is split into chunks whose partials are
-// summed in a fixed order. From kTreePairsAdjoint pairs the Gaussian's adjoint takes the pairs beyond
-// the compact cutoff by clusters of targets instead, to rounding (treecode.hip).
+// summed in a fixed order. Large sums of the Gaussian's adjoint take the pairs beyond the compact cutoff
+// by clusters of targets instead, to rounding (treecode.hip).
 #include <algorithm>
+#include <optional>
 
 #include "nbody.h"
 #include "o2d_math.h"
@@ -30,6 +31,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kTile = 256;
 constexpr int kTpl = 2;
+static_assert(kBlock * kTpl == kAdjointTileS && kTile == kAdjointTileT, "as nbody.h says");
 
 struct alignas(16) Probe {
   double x, y, gu, gv;
@@ -42,7 +44,8 @@ void adjoint_kernel(
     const double* __restrict__ ss, const double* __restrict__ sr, int64_t nt,
     const double* __restrict__ tx, const double* __restrict__ ty, const double* __restrict__ gu,
     const double* __restrict__ gv, int64_t chunk, double* __restrict__ ox, double* __restrict__ oy,
-    double* __restrict__ os, double* __restrict__ orr, int direct) {
+    double* __restrict__ os, double* __restrict__ orr, int direct, const int* __restrict__ gate) {
+  if (CORE == O2D_CORE_GAUSSIAN && gate && *gate == 0) return;
   __shared__ Probe tile[kTile];
   __shared__ double4 box[kBlock / 64];
   const int tid = threadIdx.x;
@@ -167,9 +170,9 @@ template <int CORE>
 void launch_adj(dim3 grid, hipStream_t s, int64_t ns, const double* sx, const double* sy,
                 const double* ss, const double* sr, int64_t nt, const double* tx,
                 const double* ty, const double* gu, const double* gv, int64_t chunk, double* ox,
-                double* oy, double* os, double* orr, int direct) {
+                double* oy, double* os, double* orr, int direct, const int* gate) {
   adjoint_kernel<CORE, kTpl><<<grid, kBlock, 0, s>>>(ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, chunk,
-                                                     ox, oy, os, orr, direct);
+                                                     ox, oy, os, orr, direct, gate);
 }
 
 }  // namespace
@@ -179,11 +182,19 @@ int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx
                 const double* tx, const double* ty, const double* gu, const double* gv,
                 double* gx, double* gy, double* gs, double* gr) {
   if (ns == 0 || nt == 0) return 0;
-  if (core == O2D_CORE_GAUSSIAN && (double)ns * (double)nt >= kTreePairsAdjoint)
+  if (core == O2D_CORE_GAUSSIAN && gauss_adjoint_clusters(ns, nt))
     return gauss_adjoint_tree_dev(d, s, ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, gx, gy, gs, gr);
+  return adjoint_pairs_dev(d, s, core, ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, gx, gy, gs, gr, nullptr);
+}
+
+int adjoint_pairs_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx,
+                      const double* sy, const double* ss, const double* sr, int64_t nt,
+                      const double* tx, const double* ty, const double* gu, const double* gv,
+                      double* gx, double* gy, double* gs, double* gr, const int* gate) {
   const int64_t swgs = (ns + kBlock * kTpl - 1) / (kBlock * kTpl);
   const int64_t ntiles = (nt + kTile - 1) / kTile;
-  const int64_t want = O2D_WANT_ADJ * (int64_t)d->num_cu;
+  // behind a gate, no more workgroups than fill the chip: most of these launches do nothing
+  const int64_t want = (gate ? 8 : O2D_WANT_ADJ) * (int64_t)d->num_cu;
   int64_t nchunk = swgs >= want ? 1 : std::min<int64_t>((want + swgs - 1) / swgs, ntiles);
   const int64_t per = (ntiles + nchunk - 1) / nchunk;
   nchunk = (ntiles + per - 1) / per;
@@ -199,8 +210,9 @@ int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx
     orr = os + nchunk * ns;
   }
   const dim3 grid((unsigned)swgs, (unsigned)nchunk);
-  KernelTimer kt(O2D_KT_ADJOINT, s);
-#define O2D_LADJ(C) launch_adj<C>(grid, s, ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, chunk, ox, oy, os, orr, direct)
+  std::optional<KernelTimer> kt;
+  if (!gate) kt.emplace(O2D_KT_ADJOINT, s);
+#define O2D_LADJ(C) launch_adj<C>(grid, s, ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, chunk, ox, oy, os, orr, direct, gate)
   switch (core) {
     case O2D_CORE_RM: O2D_LADJ(O2D_CORE_RM); break;
     case O2D_CORE_GAUSSIAN: O2D_LADJ(O2D_CORE_GAUSSIAN); break;
@@ -209,10 +221,10 @@ int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx
     default: O2D_LADJ(O2D_CORE_V3); break;
   }
 #undef O2D_LADJ
-  kt.stop();
+  if (kt) kt->stop();
   O2D_LAUNCH_CHECK();
   if (!direct) {
-    O2D_TRY(reduce_chunks(s, nchunk, ns, nullptr, 4, ox, gx, gy, gs, gr));
+    O2D_TRY(reduce_chunks(s, nchunk, ns, nullptr, 4, ox, gx, gy, gs, gr, gate));
   }
   return 0;
 }

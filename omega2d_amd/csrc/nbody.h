@@ -59,9 +59,11 @@ int matvec_dev(Device* d, hipStream_t s, int n, const double* a, const double* b
 int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* x);
 
 // o_f[order[i]] += sum over chunks c of part[(f nchunk + c) nt + i], for the nf (2 to 4) components f
-// (order null: the identity); nbody.hip
+// (order null: the identity). gate: a device flag (or null); unless it is set to `open`, nothing is done.
+// nbody.hip
 int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* order, int nf,
-                  const double* part, double* o0, double* o1, double* o2, double* o3);
+                  const double* part, double* o0, double* o1, double* o2, double* o3,
+                  const int* gate = nullptr, int open = 1);
 
 int rk_move_dev(hipStream_t s, int64_t n, double dt, int nstage, const double* w,
                 const double* const* u, const double* const* v, const double* x0,
@@ -73,19 +75,31 @@ int adjoint_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx
                 double* gx, double* gy, double* gs, double* gr);
 
 // the fp64 Gaussian velocity sum and its adjoint with the sources beyond the compact cutoff taken
-// by clusters, to rounding (treecode.hip), and the pairs from which they are faster than the pair
-// by pair sums. Clusters against pairs: particles on themselves 221 us against 203 at 16,000, 243
-// against 264 at 20,000, 299 against 590 at 32,000; 100,000 on 3,000 points 279 against 250, 30,000
-// on 16,000 286 against 334. With the adjoint: 50,000 on 4,096 374 against 381, 100,000 on 1,000 372
-// against 312, on 3,000 409 against 518.
-constexpr double kTreePairs = 3.5e8, kTreePairsAdjoint = 2e8;
+// by clusters, to rounding (treecode.hip), and the sizes from which they are faster than the pair by
+// pair sums. Where the cores hold so much of the set that they are not, which only the device knows, the
+// same calls sum pair by pair.
+int64_t sum64_targets(const Device* d, int64_t ns, int64_t nt);  // targets in a workgroup of the pairs
+constexpr int kAdjointTileS = 512, kAdjointTileT = 256;          // particles and probes in a tile of theirs
+bool gauss_clusters(const Device* d, int64_t ns, int64_t nt);
 int gauss_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const double* sy,
                    const double* ss, const double* sr, int64_t nt, const double* tx,
                    const double* ty, const double* tr, double* tu, double* tv);
+bool gauss_adjoint_clusters(int64_t ns, int64_t nt);
 int gauss_adjoint_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx,
                            const double* sy, const double* ss, const double* sr, int64_t nt,
                            const double* tx, const double* ty, const double* gu,
                            const double* gv, double* gx, double* gy, double* gs, double* gr);
+
+// The pair by pair forms of the two, launched behind a gate: they do nothing unless *gate (on the
+// device) is set when they run. src, trg: records (x, y, strength, radius term) in order, those of the
+// targets mapped to the outputs by torder (nbody.hip, adjoint.hip).
+int gauss_pairs_gated(Device* d, hipStream_t s, int64_t ns, const void* src, int64_t nt,
+                      const void* trg, bool radii, const uint32_t* torder, double* tu, double* tv,
+                      const int* gate);
+int adjoint_pairs_dev(Device* d, hipStream_t s, int core, int64_t ns, const double* sx,
+                      const double* sy, const double* ss, const double* sr, int64_t nt,
+                      const double* tx, const double* ty, const double* gu, const double* gv,
+                      double* gx, double* gy, double* gs, double* gr, const int* gate);
 
 // Gaussian vorticity of particles at targets (fp64, +=), device pointers
 int vorticity_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const double* sy,

@@ -11,8 +11,8 @@
 //
 // Plain form (fp64): every lane owns TPL targets and runs an unrolled loop over a 256-source
 // tile staged in LDS with coalesced loads; all lanes of a wave read the same source (an LDS
-// broadcast). Sums are fp64 per target. From kTreePairs pairs the Gaussian's velocity sum takes the
-// sources beyond its compact cutoff by clusters instead, to rounding (treecode.hip).
+// broadcast). Sums are fp64 per target. The Gaussian's large velocity sums take the sources beyond its
+// compact cutoff by clusters instead, to rounding (treecode.hip).
 //
 // Split form (fp32 pair arithmetic): the sorted sources are cut into groups of kGroup
 // sources, and stored as fp32 offsets from their group's fp64 centroid.
@@ -25,6 +25,7 @@
 // atomics, so results are reproducible run to run).
 #include <algorithm>
 #include <cstring>
+#include <optional>
 
 #include "nbody.h"
 #include "o2d_math.h"
@@ -107,9 +108,17 @@ __device__ __forceinline__ void tile_pairs64(const Src64* __restrict__ tile, int
   }
 }
 
-// src: the staged sources in Morton order; tq, tw: the targets' positions and radius terms in
-// Morton order (tw unused unless TR); torder[i]: the input index of sorted target i (torder
-// null: the targets are in input order).
+// The targets of the fp64 form, in Morton order: positions at pos[pstep i], radius terms (if any) at
+// w[wstep i], and order[i], the input index of sorted target i (null: they are in input order)
+struct Targets64 {
+  const double2* pos;
+  const double* w;
+  const uint32_t* order;
+  int pstep, wstep;
+};
+
+// src: the staged sources in Morton order. gate (the Gaussian's velocity only): a device flag, or null;
+// while it is 0 the kernel does nothing.
 //
 // Bound by the fp64 vector units (a Rosenhead-Moore or far Gaussian pair is 11 fp64 operations and
 // a reciprocal), by latency where the sum is small:
@@ -120,16 +129,19 @@ __device__ __forceinline__ void tile_pairs64(const Src64* __restrict__ tile, int
 // is inline: a call costs its whole latency, and the tile a wave's own targets lie in makes one for
 // most of its sources. Whole calls on themselves: 6,715 blob particles 209 us with two targets a
 // lane, whole tiles and calls, 132 with the inside inline, 84 in this form; 10,000 Rosenhead-Moore
-// particles 100 and 81. At kFewWgs (16,000 on themselves) 221 and 203 us; beyond it two targets
-// a lane halve the LDS reads per pair and win (a 262k blob sum is 4% slower inline).
+// particles 100 and 81. About kFewWgs (23,000 on themselves) the forms meet, two targets a lane and this
+// one: Rosenhead-Moore particles 253 and 262 us, 32,000 481 and 498; blob particles, pair by pair, 361 and
+// 313 and 590 and 556. Beyond it two targets a lane halve the LDS reads per pair (a 262k blob sum is 4%
+// slower inline).
 template <int CORE, int RES, bool TR, int TPL, bool FEW>
 __global__ __launch_bounds__(kBlock) void nbody64_kernel(
-    int64_t ns, const Src64* __restrict__ src, int64_t nt, const double2* __restrict__ tq,
-    const double* __restrict__ tw, const uint32_t* __restrict__ torder, int64_t chunk,
-    double* __restrict__ ou, double* __restrict__ ov, double* __restrict__ ow, int direct) {
+    int64_t ns, const Src64* __restrict__ src, int64_t nt, Targets64 tg, int64_t chunk,
+    double* __restrict__ ou, double* __restrict__ ov, double* __restrict__ ow, int direct,
+    const int* __restrict__ gate) {
   // the Gaussian's velocity sum takes a loop without the per-pair cutoff test for a tile that
   // lies beyond the compact cutoff of every target of the wave (d^2 > 16 w for all its pairs)
   constexpr bool kFar = CORE == O2D_CORE_GAUSSIAN && RES == O2D_VELONLY;
+  if (kFar && gate && *gate == 0) return;
   __shared__ Src64 tile[kTile];
   __shared__ double tbox[kBlock / 64][5];  // per wave: x min/max, y min/max, largest radius term
   const int tid = threadIdx.x;
@@ -140,10 +152,10 @@ __global__ __launch_bounds__(kBlock) void nbody64_kernel(
   for (int t = 0; t < TPL; ++t) {
     const int64_t i = tbase + (int64_t)t * kBlock;
     const int64_t ii = i < nt ? i : nt - 1;
-    const double2 p = tq[ii];
+    const double2 p = tg.pos[ii * tg.pstep];
     px[t] = p.x;
     py[t] = p.y;
-    pw[t] = TR ? tw[ii] : 0.0;
+    pw[t] = TR ? tg.w[ii * tg.wstep] : 0.0;
     au[t] = av[t] = aw[t] = 0.0;
   }
   // when every target of the block has the same radius term w0, it is added to each source's
@@ -153,7 +165,7 @@ __global__ __launch_bounds__(kBlock) void nbody64_kernel(
   bool uni = false;
   if constexpr (TR) {
     const int64_t i0 = (int64_t)blockIdx.x * (kBlock * TPL);
-    w0 = tw[i0 < nt ? i0 : nt - 1];
+    w0 = tg.w[(i0 < nt ? i0 : nt - 1) * tg.wstep];
     bool same = true;
 #pragma unroll
     for (int t = 0; t < TPL; ++t) same = same && pw[t] == w0;
@@ -237,7 +249,7 @@ __global__ __launch_bounds__(kBlock) void nbody64_kernel(
     const int64_t i = tbase + (int64_t)t * kBlock;
     if (i >= nt) continue;
     if (direct) {
-      const int64_t o = torder ? (int64_t)torder[i] : i;
+      const int64_t o = tg.order ? (int64_t)tg.order[i] : i;
       ou[o] += au[t];
       ov[o] += av[t];
       if (RES != O2D_VELONLY) ow[o] += aw[t];
@@ -458,12 +470,14 @@ struct Outputs {
 // null: the identity). SPLIT: a workgroup takes 64 targets, its 16 waves a share of the chunks each, in
 // order, and their sums are added in wave order, a component by each wave; else a thread per target.
 // Bound by the latency of its loads where targets are few (10,000 targets, 40 chunks: 7.8 us with a
-// thread per target, 4.5 split; 100 targets, 938 chunks: 24 with four waves, 15 with 16), by bandwidth where they are many and chunks few (250,000
-// targets, 2 chunks of 4 components: 30 us with a thread per target, 39 split).
+// thread per target, 4.5 split; 100 targets, 938 chunks: 24 with four waves, 15 with 16), by bandwidth
+// where they are many and chunks few (250,000 targets, 2 chunks of 4 components: 30 us with a thread per
+// target, 39 split).
 template <int NF, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? kReduceT : kBlock) void reduce_chunks_kernel(
     int64_t nchunk, int64_t nt, const uint32_t* __restrict__ order, const double* __restrict__ part,
-    Outputs out) {
+    Outputs out, const int* __restrict__ gate, int open) {
+  if (gate && (*gate != 0) != (open != 0)) return;
   constexpr int kWaves = SPLIT ? kReduceT / 64 : 1;
   static_assert(!SPLIT || NF <= kWaves, "a component per wave");
   const int lane = threadIdx.x & 63, wave = SPLIT ? threadIdx.x >> 6 : 0;
@@ -628,23 +642,21 @@ ChunkPlan plan_chunks(const Device* d, int64_t target_wgs, int64_t ntiles, int p
 
 template <int CORE, int RES, bool TR>
 void launch64(bool few, dim3 grid, hipStream_t s, int64_t ns, const Src64* src, int64_t nt,
-              const double2* tq, const double* tw, const uint32_t* torder, int64_t chunk,
-              double* ou, double* ov, double* ow, int direct) {
+              const Targets64& tg, int64_t chunk, double* ou, double* ov, double* ow, int direct,
+              const int* gate) {
   if (few)
-    nbody64_kernel<CORE, RES, TR, 1, true><<<grid, kBlock, 0, s>>>(ns, src, nt, tq, tw, torder,
-                                                                   chunk, ou, ov, ow, direct);
+    nbody64_kernel<CORE, RES, TR, 1, true><<<grid, kBlock, 0, s>>>(ns, src, nt, tg, chunk, ou, ov, ow,
+                                                                   direct, gate);
   else
-    nbody64_kernel<CORE, RES, TR, kTpl64, false><<<grid, kBlock, 0, s>>>(
-        ns, src, nt, tq, tw, torder, chunk, ou, ov, ow, direct);
+    nbody64_kernel<CORE, RES, TR, kTpl64, false><<<grid, kBlock, 0, s>>>(ns, src, nt, tg, chunk, ou,
+                                                                         ov, ow, direct, gate);
 }
 
 template <int CORE>
 void dispatch64(int res, bool tr_present, bool few, dim3 grid, hipStream_t s, int64_t ns,
-                const Src64* src, int64_t nt, const double2* tq, const double* tw,
-                const uint32_t* torder, int64_t chunk, double* ou, double* ov, double* ow,
-                int direct) {
-#define O2D_L64(R, T) \
-  launch64<CORE, R, T>(few, grid, s, ns, src, nt, tq, tw, torder, chunk, ou, ov, ow, direct)
+                const Src64* src, int64_t nt, const Targets64& tg, int64_t chunk, double* ou,
+                double* ov, double* ow, int direct, const int* gate) {
+#define O2D_L64(R, T) launch64<CORE, R, T>(few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate)
   if (res == O2D_VELONLY) {
     if (tr_present) O2D_L64(O2D_VELONLY, true);
     else O2D_L64(O2D_VELONLY, false);
@@ -730,13 +742,16 @@ int gather_targets(hipStream_t s, int core, int64_t n, const uint32_t* order, co
 }  // namespace
 
 int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* order, int nf,
-                  const double* part, double* o0, double* o1, double* o2, double* o3) {
+                  const double* part, double* o0, double* o1, double* o2, double* o3,
+                  const int* gate, int open) {
   const bool split = nchunk >= 8;
   const unsigned grid = split ? (unsigned)((nt + 63) / 64) : grid1(nt).x;
   const Outputs out{{o0, o1, o2, o3}};
-#define O2D_REDUCE(NF)                                                                            \
-  split ? reduce_chunks_kernel<NF, true><<<grid, kReduceT, 0, s>>>(nchunk, nt, order, part, out)  \
-        : reduce_chunks_kernel<NF, false><<<grid, kBlock, 0, s>>>(nchunk, nt, order, part, out)
+#define O2D_REDUCE(NF)                                                                      \
+  split ? reduce_chunks_kernel<NF, true><<<grid, kReduceT, 0, s>>>(nchunk, nt, order, part, \
+                                                                   out, gate, open)         \
+        : reduce_chunks_kernel<NF, false><<<grid, kBlock, 0, s>>>(nchunk, nt, order, part,  \
+                                                                  out, gate, open)
   if (nf == 2) O2D_REDUCE(2);
   else if (nf == 3) O2D_REDUCE(3);
   else O2D_REDUCE(4);
@@ -781,6 +796,81 @@ int prep_targets(Device* d, hipStream_t s, Workspace* ws, int core, int64_t nt, 
   return 0;
 }
 
+namespace {
+// too few pairs of a set of targets and a tile of sources for whole tiles to fill the chip
+bool sum64_few(const Device* d, int64_t ns, int64_t nt) {
+  const int64_t sets = (nt + kBlock * kTpl64 - 1) / (kBlock * kTpl64), tiles = (ns + kTile - 1) / kTile;
+  return sets * tiles < kFewWgs * d->num_cu;
+}
+}  // namespace
+
+int64_t sum64_targets(const Device* d, int64_t ns, int64_t nt) {
+  return sum64_few(d, ns, nt) ? kBlock : kBlock * kTpl64;
+}
+
+namespace {
+
+// The fp64 form on staged sources and targets. Behind a gate, no more workgroups than fill the chip: most
+// of these launches do nothing.
+int sum64(Device* d, hipStream_t s, Workspace* ws, int core, int res, bool trp, int64_t ns,
+          const Src64* src, int64_t nt, const Targets64& tg, double* tu, double* tv, double* tw,
+          const int* gate) {
+  int64_t twgs = (nt + kBlock * kTpl64 - 1) / (kBlock * kTpl64);
+  const int64_t ntiles = (ns + kTile - 1) / kTile;
+  const int nf = res == O2D_VELONLY ? 2 : 3;
+  const bool few = sum64_few(d, ns, nt);
+  ChunkPlan cp;
+  int64_t chunk;
+  if (few) {
+    twgs = (nt + kBlock - 1) / kBlock;
+    const int64_t units = (ns + kUnit - 1) / kUnit;
+    int64_t n = std::min((kFewWgs * d->num_cu + twgs - 1) / twgs, units);
+    n = std::max<int64_t>(1, std::min(n, max_chunks(ws, nf, nt)));
+    const int64_t per = (units + n - 1) / n;
+    cp = ChunkPlan{(units + per - 1) / per, per};
+    chunk = per * kUnit;
+  } else {
+    cp = plan_chunks(d, twgs, ntiles, gate ? 8 : O2D_WANT64, max_chunks(ws, nf, nt));
+    chunk = cp.per_chunk * kTile;
+  }
+  const dim3 grid((unsigned)twgs, (unsigned)cp.nchunk);
+  double *ou = tu, *ov = tv, *ow = tw;
+  const int direct = cp.nchunk == 1;
+  if (!direct) {
+    void* p;
+    O2D_TRY(take(d, ws, kPartials, sizeof(double) * nf * cp.nchunk * nt, s, &p));
+    ou = static_cast<double*>(p);
+    ov = ou + cp.nchunk * nt;
+    ow = res == O2D_VELONLY ? nullptr : ov + cp.nchunk * nt;
+  }
+  std::optional<KernelTimer> kt;
+  if (!gate) kt.emplace(trp ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT, s);
+  switch (core) {
+    case O2D_CORE_RM: dispatch64<O2D_CORE_RM>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
+    case O2D_CORE_GAUSSIAN: dispatch64<O2D_CORE_GAUSSIAN>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
+    case O2D_CORE_WL: dispatch64<O2D_CORE_WL>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
+    case O2D_CORE_V2: dispatch64<O2D_CORE_V2>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
+    default: dispatch64<O2D_CORE_V3>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
+  }
+  if (kt) kt->stop();
+  O2D_LAUNCH_CHECK();
+  if (!direct) {
+    O2D_TRY(reduce_chunks(s, cp.nchunk, nt, tg.order, nf, ou, tu, tv, tw, nullptr, gate));
+  }
+  return 0;
+}
+
+}  // namespace
+
+int gauss_pairs_gated(Device* d, hipStream_t s, int64_t ns, const void* src, int64_t nt,
+                      const void* trg, bool radii, const uint32_t* torder, double* tu, double* tv,
+                      const int* gate) {
+  const double* t = static_cast<const double*>(trg);
+  return sum64(d, s, nullptr, O2D_CORE_GAUSSIAN, O2D_VELONLY, radii, ns,
+               static_cast<const Src64*>(src), nt,
+               Targets64{reinterpret_cast<const double2*>(t), t + 3, torder, 2, 4}, tu, tv, nullptr, gate);
+}
+
 int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns, const double* sx,
               const double* sy, const double* ss, const double* sr, int64_t nt, const double* tx,
               const double* ty, const double* tr, double* tu, double* tv, double* tw,
@@ -790,7 +880,7 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
   if (ns > 0x7fffffffLL || nt > 0x7fffffffLL)
     return fail(O2D_ERR_SIZE, "more than 2^31 - 1 sources or targets");
   if (prec == O2D_PLAIN_FP64 && core == O2D_CORE_GAUSSIAN && res == O2D_VELONLY && !ws &&
-      (double)ns * (double)nt >= kTreePairs)
+      gauss_clusters(d, ns, nt))
     return gauss_tree_dev(d, s, ns, sx, sy, ss, sr, nt, tx, ty, tr, tu, tv);
   const bool trp = tr != nullptr;
   // targets that are the sources themselves (a collection acting on itself) share their order
@@ -827,48 +917,8 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
     O2D_TRY(prep_targets<double>(d, s, ws, core, nt, tx, ty, tr, sort, self ? order : nullptr,
                                  &torder, &tq, &twv));
 
-    int64_t twgs = (nt + kBlock * kTpl64 - 1) / (kBlock * kTpl64);
-    const int64_t ntiles = (ns + kTile - 1) / kTile;
-    const int nf = res == O2D_VELONLY ? 2 : 3;
-    const bool few = twgs * ntiles < kFewWgs * d->num_cu;
-    ChunkPlan cp;
-    int64_t chunk;
-    if (few) {
-      twgs = (nt + kBlock - 1) / kBlock;
-      const int64_t units = (ns + kUnit - 1) / kUnit;
-      int64_t n = std::min((kFewWgs * d->num_cu + twgs - 1) / twgs, units);
-      n = std::max<int64_t>(1, std::min(n, max_chunks(ws, nf, nt)));
-      const int64_t per = (units + n - 1) / n;
-      cp = ChunkPlan{(units + per - 1) / per, per};
-      chunk = per * kUnit;
-    } else {
-      cp = plan_chunks(d, twgs, ntiles, O2D_WANT64, max_chunks(ws, nf, nt));
-      chunk = cp.per_chunk * kTile;
-    }
-    const dim3 grid((unsigned)twgs, (unsigned)cp.nchunk);
-    double *ou = tu, *ov = tv, *ow = tw;
-    const int direct = cp.nchunk == 1;
-    if (!direct) {
-      void* p;
-      O2D_TRY(take(d, ws, kPartials, sizeof(double) * nf * cp.nchunk * nt, s, &p));
-      ou = static_cast<double*>(p);
-      ov = ou + cp.nchunk * nt;
-      ow = res == O2D_VELONLY ? nullptr : ov + cp.nchunk * nt;
-    }
-    KernelTimer kt(trp ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT, s);
-    switch (core) {
-      case O2D_CORE_RM: dispatch64<O2D_CORE_RM>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
-      case O2D_CORE_GAUSSIAN: dispatch64<O2D_CORE_GAUSSIAN>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
-      case O2D_CORE_WL: dispatch64<O2D_CORE_WL>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
-      case O2D_CORE_V2: dispatch64<O2D_CORE_V2>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
-      default: dispatch64<O2D_CORE_V3>(res, trp, few, grid, s, ns, src, nt, tq, twv, torder, chunk, ou, ov, ow, direct); break;
-    }
-    kt.stop();
-    O2D_LAUNCH_CHECK();
-    if (!direct) {
-      O2D_TRY(reduce_chunks(s, cp.nchunk, nt, torder, nf, ou, tu, tv, tw, nullptr));
-    }
-    return 0;
+    return sum64(d, s, ws, core, res, trp, ns, src, nt, Targets64{tq, twv, torder, 1, 1}, tu, tv, tw,
+                 nullptr);
   }
 
   // split form

@@ -32,7 +32,7 @@ enum Slot : int {
   kNearPart, kNodeNorm, kPanRec, kCutTable, kNearCounts, kNearTiles,
   kInv, kSolveTmp,
   kTreeKeys, kTreeOrder, kTreeTOrder, kTreeSrc, kTreeCells, kTreeBox, kTreeMom,
-  kTreeTrg, kTreeSuper,
+  kTreeTrg, kTreeSuper, kTreeGate,
   kPan2X, kPan2Y, kPan2Idx, kPanGeom2,
   kLuPairs, kPanClus, kPanClusG, kPanClusS, kVortSrc,
   kNumSlots

@@ -78,12 +78,59 @@ constexpr int kShareOrder = 28, kSpareOrders = 6;
 inline int kept_orders(int p) {
   return p + std::max(0, std::min(kSpareOrders, kShareOrder - p));
 }
+// Groups of 16 targets where targets are much sparser than the sources, else of 64: a box of 64 would
+// hold many leaves that few of its targets are near. 1M sources, targets a 64th, 16th, 12th, 8th and 5th
+// as many: 564, 722, 822, 876 and 1,009 us in groups of 16, 714, 766, 804, 872 and 999 of 64; at theta
+// 1/3 804, 1,191, 1,410, 1,578 and 1,964 against 1,003, 1,142, 1,233, 1,417 and 1,727. In the adjoint,
+// whose targets are the particles: 50,000 among 200,000 probes 887 and 756, 10,000 among 100,000 486 and
+// 457, 781 among 50,000 219 and 244, 1,000 among 1M 788 and 1,094.
+constexpr int64_t kSparse = 12, kSparseAdjoint = 64;
 // waves per CU the group kernel aims for by sharing a group's cells and leaves out: every share
-// opens the same cells, so more of them cost more (1M particles: 32 and 64 equal; 10,000 tracers
-// in groups of 16: 264 us at 16, 369 at 32)
-constexpr int kWaves64 = 32, kWaves16 = 16;
-// fewer super groups than this leave most of the chip idle for longer than they save
-constexpr int64_t kMinSupers = 16;
+// opens the same cells, so more of them cost more (1M particles: 32 and 64 equal), unless they no
+// longer fit the chip at once (16 per CU do): 20,000 particles take 163 us at 16 or just below and 175
+// at 32, 100,000 and 8,000 targets in groups of 16 214 at or just below 16 and 222 just above. From
+// kEvenGroups groups on a second round of waves costs less than groups of unequal work (40,000
+// targets 635 and 660 us, 262,144 1,437 and 1,698).
+constexpr int kWaves64 = 32, kWavesOnce = 16;
+constexpr int64_t kEvenGroups = 512;
+// Fewer super groups than this leave most of the chip idle for longer than they save: us with and without,
+// 40,000 blob particles on themselves (40 of them) 237 and 225, 90,000 339 and 325, 110,000 382 and 373,
+// 130,000 412 and 417, 262,144 717 and 743, 524,288 1,220 and 1,325; the adjoint of 30,000 particles 301 and
+// 281, 64,000 317 and 313, 80,000 348 and 352, 200,000 422 and 475
+constexpr int64_t kMinSupers = 120, kMinSupersAdjoint = 72;
+
+// When the fp64 Gaussian sums go by clusters. In units of a pair of the pair by pair form, whose work is
+// sources times targets filled up to its tiles: what building and walking the tree costs besides, which
+// grows more slowly than the sources, and (up to a most) with targets that share few cells.
+// Velocity, us by clusters and pair by pair (blobs): 10,000 on themselves 137 and 101, 16,000 184 and 206,
+// 20,000 182 and 259; 50,000 on 6,000 points 243 and 225; 100,000 on 3,000 and 4,000 266 and 274 against 227
+// and 273; 262,144 on 2,000 and 3,000 382 and 383 against 345 and 492; 1M on 300, 700 and 1,000 618, 627
+// and 655 against 419, 653 and 656; 2M on 100 883 and 756; 4M on 100 1,155 and 1,362; 10,000 on 30,000
+// 203 and 230; 1,000 on 200,000 and 350,000 193 and 262 against 183 and 282.
+constexpr double kClusterPairs = 1.2e8, kClusterSources = 9e5, kClusterTarget = 300, kClusterTargets = 2e8;
+// The adjoint: 10,000 on themselves 182 and 203, 16,000 247 and 315; 60,000 particles and 4,000 probes 241
+// and 256; 100,000 and 2,200 and 3,000 254 and 279 against 231 and 316; 250,000 and 1,000 and 1,500 313 and
+// 352 against 259 and 375; 1M and 500 574 and 499; 4M and 100 and 700 1,258 and 2,633 against 902 and 2,915;
+// 10,000 and 25,000 265 and 257; 3,000 and 50,000 and 150,000 297 and 426 against 172 and 443; 2,000 and
+// 300,000 493 and 601; 1,000 and 500,000 and 1M 578 and 797 against 537 and 1,022; 100 and 4M 1,836 and
+// 1,951, but 2,677 with a pair in the cutoff sampled; 40 and 10M 3,324 and 4,528.
+constexpr double kAdjointPairs = 2e8, kAdjointParticle = 500, kAdjointProbe = 400, kAdjointFew = 1000,
+                 kAdjointFewMost = 2.5e8;
+
+// Clusters gain nothing on pairs nearer than the cutoff, and where few targets share the chip their walk is
+// far slower there than the pair by pair loops. A sample of kSampleS sources and kSampleT targets says
+// which part of the pairs that is; past a limit the call sums pair by pair (8 us more than pairs alone,
+// and the tree for nothing). The limit, the targets from which it is whole (with fewer: times the
+// square of their part) and those from which nothing is sampled, because clusters are about as fast as
+// pairs at any radius. us by clusters and pair by pair; velocity: 262,144 on 10,000 with 8% of the pairs
+// near 2,274 and 3,949, 28% 4,990 and 4,961, 74% 9,834 and 6,487; 20,000 on themselves 19% 471 and 471, 99%
+// 1,064 and 777; 100,000 on 4,000 0.5% 330 and 406, 8% 728 and 571; 1M on 1,000 0.5% 1,418 and 1,184, 75%
+// 17,020 and 2,729; 10,000 on 100,000 78% 2,003 and 2,482. Adjoint: 10,000 particles and 100,000 probes 0.5%
+// 557 and 1,018, 8% 1,282 and 1,373, 77% 4,786 and 3,025; 1,000 and 1M 0 792 and 1,022, 0.5% 1,381 and
+// 1,186, 77% 28,915 and 3,433; 30,000 and 12,000 100% 1,619 and 1,199; 100,000 and 8,000 75% 2,545 and 2,284.
+constexpr int kSampleS = 256, kSampleT = 64;
+constexpr double kNearLimit = 0.3, kNearTargets = 1e4, kNearMany = 5e4;
+constexpr double kNearLimitAdjoint = 0.4, kNearTargetsAdjoint = 2e4, kNearManyAdjoint = 7e4;
 
 // A cell: head = (centre x, y, radius, largest radius term), kids = (first child, children); a
 // leaf has no children, and its first child is its index among the leaves. (As one struct the
@@ -191,21 +238,67 @@ __device__ __forceinline__ double2 cinv(double x, double y) {
 
 // ---------------------------------------------------------------------------- the tree
 
+// What a call samples: its targets (tr null: no radii), and the part of the pairs within the Gaussian's
+// cutoff from which *gate is set
+struct Sample {
+  int64_t nt;
+  const double *tx, *ty, *tr;
+  double limit;
+  int* gate;
+};
+
+// *gate = more than the limit of kSampleS x kSampleT pairs, spread evenly over the arrays, are within the
+// cutoff (one workgroup; sr: the sources' radii, in the adjoint only the targets' count; lds: three
+// arrays of kSampleT and a count per wave). Pairs with a NaN are not.
+template <bool ADJ>
+__device__ void sample_near(int64_t ns, const double* x, const double* y, const double* sr,
+                            const Sample& m, double* lds) {
+  double *tx = lds, *ty = lds + kSampleT, *tw = lds + 2 * kSampleT;
+  int* near = reinterpret_cast<int*>(lds + 3 * kSampleT);
+  const int t = threadIdx.x;
+  static_assert(kSampleS == kBlock, "a source per thread");
+  if (t < kSampleT) {
+    const int64_t i = m.nt * t / kSampleT;
+    tx[t] = m.tx[i];
+    ty[t] = m.ty[i];
+    tw[t] = m.tr ? m.tr[i] * m.tr[i] : 0.0;
+  }
+  const int64_t j = ns * t / kSampleS;
+  const double px = x[j], py = y[j], w = ADJ ? 0.0 : sr[j] * sr[j];
+  __syncthreads();
+  int n = 0;
+  for (int i = 0; i < kSampleT; ++i) {
+    const double dx = px - tx[i], dy = py - ty[i];
+    n += dx * dx + dy * dy < kGaussFar * (w + tw[i]) ? 1 : 0;
+  }
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+  if ((t & 63) == 0) near[t >> 6] = n;
+  __syncthreads();
+  if (t != 0) return;
+  for (int w = 1; w < kWaves; ++w) n += near[w];
+  *m.gate = (double)n > m.limit * (kSampleS * kSampleT) ? 1 : 0;
+}
+
 // One wave per 64 sources in Morton order (kLeafs leaves): gathers their records (padding a
 // short last leaf with charges of 0 at its last source) and forms each leaf's cell, box and
 // moments. The powers of eight orders at a time pass through LDS, and each (leaf, order) sum is
 // taken by a few lanes: a wave sum per order through shuffles took 130 us for 1M sources.
-// ADJ: a is gv's and b gu's array, and radii play no part.
+// ADJ: a is gv's and b gu's array, and radii play no part. The last workgroup samples instead, where
+// there is a gate to set.
 template <bool ADJ>
 __global__ __launch_bounds__(kBlock) void tree_leaf_kernel(
     int64_t ns, int64_t nleaf, int p, const uint32_t* __restrict__ order,
     const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ a,
     const double* __restrict__ b, int core, Src* __restrict__ src, double4* __restrict__ head,
-    uint2* __restrict__ kids, double4* __restrict__ box, double2* __restrict__ mom) {
+    uint2* __restrict__ kids, double4* __restrict__ box, double2* __restrict__ mom, Sample sample) {
   constexpr int kLeafs = 64 / kLeaf, kChunk = 8;
   constexpr int kShare = 64 / (kLeafs * kChunk);  // lanes per (leaf, order)
   static_assert(kShare >= 1 && kLeaf % kShare == 0, "whole shares");
   __shared__ double2 buf[kWaves][kChunk][64 + 1];
+  if (sample.gate && blockIdx.x == gridDim.x - 1) {
+    sample_near<ADJ>(ns, x, y, b, sample, reinterpret_cast<double*>(buf));
+    return;
+  }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t first = ((int64_t)blockIdx.x * kWaves + wave) * 64;
   if (first >= nleaf * kLeaf) return;  // whole waves; no workgroup barrier below
@@ -430,7 +523,9 @@ template <int CORE, bool ADJ>
 __global__ __launch_bounds__(kSuperBlock) void tree_super_kernel(
     int64_t nt, const Trg* __restrict__ trg, const double4* __restrict__ head,
     const uint2* __restrict__ kids, const double2* __restrict__ mom, uint32_t root, double theta, double tol,
-    Super* __restrict__ super, double2* __restrict__ local, uint32_t* __restrict__ front) {
+    Super* __restrict__ super, double2* __restrict__ local, uint32_t* __restrict__ front,
+    const int* __restrict__ gate) {
+  if (gate && *gate != 0) return;
   __shared__ double binom[kMaxP * kMaxP];
   __shared__ uint32_t queue[2][kQueue], taken[kSuperBlock];
   __shared__ int counts[kSuperWaves][3];
@@ -621,6 +716,7 @@ struct GroupArgs {
   double theta;    // cells are far from radius / theta on
   float logtail;   // twice the logarithm (base 2) of the remainder that cells further away keep to
   double tol;
+  const int* gate;  // set (or null): nothing is done
 };
 
 // One wave per G targets and share (blockIdx.y) of their far cells and leaves; every share opens
@@ -648,6 +744,7 @@ __global__ __launch_bounds__(kGroupBlock, 4) void tree_group_kernel(
   const int slice = lane / G, mine = lane % G;
   const int64_t group = (int64_t)blockIdx.x * kGroupWaves + wave;
   if (group * G >= a.nt) return;  // whole waves; no workgroup barrier below
+  if (a.gate && *a.gate != 0) return;
   uint32_t* st = stacks[wave];
   double2* data = buffers[wave][slice];
   const int64_t i = group * G + mine;
@@ -991,6 +1088,8 @@ struct Problem {
   const double *tx, *ty, *tr, *ts;
   double *o0, *o1, *o2, *o3;
   int timed;  // kernel class of the evaluation
+  // part of the pairs within the cutoff, as sampled, past which the sum goes pair by pair (0: never)
+  double near_limit;
 };
 
 // log2 of the given share of theta^order
@@ -1009,7 +1108,7 @@ void launch_eval(const Problem& q, hipStream_t s, int64_t nsuper, const GroupArg
                  double* part) {
   if (nsuper)
     tree_super_kernel<CORE, ADJ><<<(unsigned)nsuper, kSuperBlock, 0, s>>>(
-        q.nt, trg, head, kids, mom, root, limit(q, kShareLocal), q.tol, super, local, front);
+        q.nt, trg, head, kids, mom, root, limit(q, kShareLocal), q.tol, super, local, front, ga.gate);
   const int64_t groups = (q.nt + ga.g - 1) / ga.g;
   const dim3 grid((unsigned)((groups + kGroupWaves - 1) / kGroupWaves), (unsigned)ga.ksplit);
   auto* sup = nsuper ? super : nullptr;
@@ -1053,13 +1152,20 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
   double2* mom = static_cast<double2*>(mb);
   const uint32_t* torder = sorder;
   const Trg* trg;
+  int* gate = nullptr;
+  if (q.near_limit > 0.0) {
+    void* gp;
+    O2D_TRY(slot(d, kTreeGate, sizeof(int), s, &gp));
+    gate = static_cast<int*>(gp);
+  }
   {
     KernelTimer kt(O2D_KT_TREE_BUILD, s);
     O2D_TRY(morton_order(d, s, ns, q.sx, q.sy, true, 0.0, 0.0, 0.0, static_cast<uint32_t*>(kb),
                          sorder, nullptr, false));
     const int64_t lwaves = (nsrc + 63) / 64;
-    tree_leaf_kernel<ADJ><<<(unsigned)((lwaves + kWaves - 1) / kWaves), kBlock, 0, s>>>(
-        ns, lv.cnt[0], q.p, sorder, q.sx, q.sy, q.sa, q.sb, q.core, src, head, kids, box, mom);
+    tree_leaf_kernel<ADJ><<<(unsigned)((lwaves + kWaves - 1) / kWaves + (gate ? 1 : 0)), kBlock, 0, s>>>(
+        ns, lv.cnt[0], q.p, sorder, q.sx, q.sy, q.sa, q.sb, q.core, src, head, kids, box, mom,
+        Sample{nt, q.tx, q.ty, q.tr, q.near_limit, gate});
     O2D_LAUNCH_CHECK();
     for (int l = 0; l + 1 < lv.n; l += 2) {
       const bool two = l + 2 < lv.n;
@@ -1092,16 +1198,16 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
   ga.p = q.p;
   ga.tol = q.tol;
   const int64_t nsup = (nt + kSuper - 1) / kSuper;
-  const int64_t nsuper = nsup >= kMinSupers ? nsup : 0;
-  // waves per group: enough for O2D_TREE_WAVES waves per CU
-  // targets much sparser than the sources: a box of 64 would hold many leaves that few of its
-  // targets are near (65,536 tracers among 1M particles: 0.47 ms in groups of 16, 0.51 of 32,
-  // 0.72 of 64; the particles on themselves 3.2, 2.4 and 2.0 ms)
-  ga.g = nt < ns / 4 ? 16 : 64;
+  const int64_t nsuper = nsup >= (ADJ ? kMinSupersAdjoint : kMinSupers) ? nsup : 0;
+  ga.gate = gate;
+  ga.g = nt < ns / (ADJ ? kSparseAdjoint : kSparse) ? 16 : 64;
   ga.theta = limit(q, ga.g == 64 ? kShare64 : kShare16);
   ga.logtail = (float)(2.0 * remainder(q, kShareTail));
-  const int64_t groups = (nt + ga.g - 1) / ga.g, want = (int64_t)(ga.g == 64 ? kWaves64 : kWaves16) * d->num_cu;
-  ga.ksplit = groups >= want ? 1 : (int)std::min<int64_t>(32, (want + groups - 1) / groups);
+  const int64_t groups = (nt + ga.g - 1) / ga.g;
+  const int64_t once = (int64_t)kWavesOnce * d->num_cu, most = (int64_t)kWaves64 * d->num_cu;
+  ga.ksplit = (int)std::min<int64_t>(32, ga.g == 64 && groups > kEvenGroups
+                                             ? (most + groups - 1) / groups
+                                             : std::max<int64_t>(1, once / groups));
   // starting cells without a frontier: the lowest level that is tested in one go
   int sl = lv.n - 1;
   while (sl > 0 && lv.cnt[sl - 1] <= 64) --sl;
@@ -1128,6 +1234,13 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
   }
   const uint32_t root = (uint32_t)lv.off[lv.n - 1];
   KernelTimer kt(q.timed, s);
+  if (gate) {
+    if constexpr (ADJ)
+      O2D_TRY(adjoint_pairs_dev(d, s, q.core, nt, q.tx, q.ty, q.ts, q.tr, ns, q.sx, q.sy, q.sb, q.sa,
+                                q.o1, q.o2, q.o0, q.o3, gate));
+    else
+      O2D_TRY(gauss_pairs_gated(d, s, ns, src, nt, trg, q.tr != nullptr, torder, q.o0, q.o1, gate));
+  }
 #define O2D_EVAL(C) \
   launch_eval<C, ADJ>(q, s, nsuper, ga, trg, torder, head, kids, mom, src, root, super, local, front, part)
   switch (q.core) {
@@ -1145,7 +1258,7 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
   kt.stop();
   O2D_LAUNCH_CHECK();
   if (part) {
-    O2D_TRY(reduce_chunks(s, ga.ksplit, nt, torder, nf, part, q.o0, q.o1, q.o2, q.o3));
+    O2D_TRY(reduce_chunks(s, ga.ksplit, nt, torder, nf, part, q.o0, q.o1, q.o2, q.o3, gate, 0));
   }
   return 0;
 }
@@ -1157,8 +1270,29 @@ int tree_dev(Device* d, hipStream_t s, int core, double theta, int p, double tol
              const double* tx, const double* ty, const double* tr, double* tu, double* tv) {
   if (ns == 0 || nt == 0) return 0;
   const Problem q{core, p, kept_orders(p), theta, tol, ns, sx, sy, ss, sr, nt, tx, ty, tr, nullptr,
-                  tu, tv, nullptr, nullptr, O2D_KT_TREE_EVAL};
+                  tu, tv, nullptr, nullptr, O2D_KT_TREE_EVAL, 0.0};
   return tree_run<false>(d, s, q);
+}
+
+namespace {
+// the sampled part of near pairs past which n targets are summed pair by pair (0: never)
+inline double near_limit(double n, double limit, double whole, double many) {
+  const double part = std::min(1.0, n / whole);
+  return n < many ? limit * part * part : 0.0;
+}
+inline double filled(int64_t n, int64_t tile) { return (double)((n + tile - 1) / tile * tile); }
+}  // namespace
+
+bool gauss_clusters(const Device* d, int64_t ns, int64_t nt) {
+  return (double)ns * filled(nt, sum64_targets(d, ns, nt)) >=
+         kClusterPairs + kClusterSources * std::sqrt((double)ns) +
+             std::min(kClusterTarget * nt, kClusterTargets);
+}
+
+bool gauss_adjoint_clusters(int64_t ns, int64_t nt) {
+  return filled(ns, kAdjointTileS) * filled(nt, kAdjointTileT) >=
+         kAdjointPairs + kAdjointParticle * ns + kAdjointProbe * nt +
+             std::min(kAdjointFew * nt, kAdjointFewMost);
 }
 
 int gauss_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const double* sy,
@@ -1166,7 +1300,8 @@ int gauss_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const
                    const double* ty, const double* tr, double* tu, double* tv) {
   const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kMaxP, kExactTheta, 0.0, ns, sx, sy, ss, sr, nt,
                   tx, ty, tr, nullptr, tu, tv, nullptr, nullptr,
-                  tr ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT};
+                  tr ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT,
+                  near_limit((double)nt, kNearLimit, kNearTargets, kNearMany)};
   return tree_run<false>(d, s, q);
 }
 
@@ -1175,7 +1310,8 @@ int gauss_adjoint_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* s
                            const double* tx, const double* ty, const double* gu,
                            const double* gv, double* gx, double* gy, double* gs, double* gr) {
   const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kMaxP, kExactTheta, 0.0, nt, tx, ty, gv, gu, ns,
-                  sx, sy, sr, ss, gs, gx, gy, gr, O2D_KT_ADJOINT};
+                  sx, sy, sr, ss, gs, gx, gy, gr, O2D_KT_ADJOINT,
+                  near_limit((double)ns, kNearLimitAdjoint, kNearTargetsAdjoint, kNearManyAdjoint)};
   return tree_run<true>(d, s, q);
 }
 
