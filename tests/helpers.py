@@ -28,3 +28,27 @@ def particles(rng, n, lo=-1.0, hi=1.0, rad=(0.01, 0.05), smean=0.0, sstd=1.0):
     s = rng.normal(smean, sstd, n)
     r = rng.uniform(rad[0], rad[1], n)
     return x, y, s, r
+
+
+def pair_sum(src, tgt, tr=None, core="gauss", most=262144):
+    """The fp64 velocity of device tensors src = (x, y, s, r) at tgt = (x, y), pair by pair: the
+    no-allocation entry never takes clusters, and adds `most` sources and targets at a time."""
+    import ctypes
+
+    import torch
+
+    from omega2d_amd import _cabi
+    from omega2d_amd.device import env_for
+    u, v = (torch.zeros(tgt[0].numel(), dtype=torch.float64, device="cuda") for _ in range(2))
+    env = env_for(u.device, core, "fp64", "vel")
+    p = lambda a: None if a is None else ctypes.c_void_p(a.data_ptr())  # noqa: E731
+    for i in range(0, u.numel(), most):
+        cut = slice(i, i + most)
+        t = [a[cut].contiguous() for a in (*tgt, *([] if tr is None else [tr]))]
+        for j in range(0, src[0].numel(), most):
+            s = [a[j:j + most].contiguous() for a in src]
+            _cabi.call("o2d_hip_points_on_points_noalloc_dev_d", ctypes.byref(env), s[0].numel(),
+                       *[p(a) for a in s], t[0].numel(), p(t[0]), p(t[1]),
+                       p(t[2]) if tr is not None else None, p(u[cut]), p(v[cut]), None, None)
+        torch.cuda.synchronize()
+    return u, v
