@@ -72,8 +72,10 @@ constexpr double kExactTheta = 1.0 / 3.0;
 // theta^p: the moments of cells at the limit of groups of 64 targets and of 16 (smaller, so that more of
 // their targets are near it), the orders left out of cells further away, and local expansions. From
 // kShareOrder on a share is kept by taking cells from a little further than theta says; below, where
-// that little is much, cells near the limit use up to kSpareOrders more than p.
+// that little is much, cells near the limit use up to kSpareOrders more than p. The exact sums, whose
+// remainders are below rounding, take the wider shares (their error is 4.6e-16 with either).
 constexpr double kShare64 = 0.275, kShare16 = 0.08, kShareTail = 0.02, kShareLocal = 0.0105;
+constexpr double kExactShare16 = 0.275, kExactShareTail = 0.05;
 constexpr int kShareOrder = 28, kSpareOrders = 6;
 inline int kept_orders(int p) {
   return p + std::max(0, std::min(kSpareOrders, kShareOrder - p));
@@ -1080,6 +1082,7 @@ struct Problem {
   int order;  // the remainder of a far cell stays below theta^order
   int p;      // orders kept of a cell and of a local expansion
   double theta, tol;
+  double share16, tail;  // of theta^order, for groups of 16 and for orders left out
   // sources, and their charges: strength and radius (velocity) or gv and gu (adjoint)
   int64_t ns;
   const double *sx, *sy, *sa, *sb;
@@ -1201,8 +1204,8 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
   const int64_t nsuper = nsup >= (ADJ ? kMinSupersAdjoint : kMinSupers) ? nsup : 0;
   ga.gate = gate;
   ga.g = nt < ns / (ADJ ? kSparseAdjoint : kSparse) ? 16 : 64;
-  ga.theta = limit(q, ga.g == 64 ? kShare64 : kShare16);
-  ga.logtail = (float)(2.0 * remainder(q, kShareTail));
+  ga.theta = limit(q, ga.g == 64 ? kShare64 : q.share16);
+  ga.logtail = (float)(2.0 * remainder(q, q.tail));
   const int64_t groups = (nt + ga.g - 1) / ga.g;
   const int64_t once = (int64_t)kWavesOnce * d->num_cu, most = (int64_t)kWaves64 * d->num_cu;
   ga.ksplit = (int)std::min<int64_t>(32, ga.g == 64 && groups > kEvenGroups
@@ -1269,7 +1272,7 @@ int tree_dev(Device* d, hipStream_t s, int core, double theta, int p, double tol
              const double* sx, const double* sy, const double* ss, const double* sr, int64_t nt,
              const double* tx, const double* ty, const double* tr, double* tu, double* tv) {
   if (ns == 0 || nt == 0) return 0;
-  const Problem q{core, p, kept_orders(p), theta, tol, ns, sx, sy, ss, sr, nt, tx, ty, tr, nullptr,
+  const Problem q{core, p, kept_orders(p), theta, tol, kShare16, kShareTail, ns, sx, sy, ss, sr, nt, tx, ty, tr, nullptr,
                   tu, tv, nullptr, nullptr, O2D_KT_TREE_EVAL, 0.0};
   return tree_run<false>(d, s, q);
 }
@@ -1298,7 +1301,7 @@ bool gauss_adjoint_clusters(int64_t ns, int64_t nt) {
 int gauss_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const double* sy,
                    const double* ss, const double* sr, int64_t nt, const double* tx,
                    const double* ty, const double* tr, double* tu, double* tv) {
-  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kMaxP, kExactTheta, 0.0, ns, sx, sy, ss, sr, nt,
+  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kMaxP, kExactTheta, 0.0, kExactShare16, kExactShareTail, ns, sx, sy, ss, sr, nt,
                   tx, ty, tr, nullptr, tu, tv, nullptr, nullptr,
                   tr ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT,
                   near_limit((double)nt, kNearLimit, kNearTargets, kNearMany)};
@@ -1309,7 +1312,7 @@ int gauss_adjoint_tree_dev(Device* d, hipStream_t s, int64_t ns, const double* s
                            const double* sy, const double* ss, const double* sr, int64_t nt,
                            const double* tx, const double* ty, const double* gu,
                            const double* gv, double* gx, double* gy, double* gs, double* gr) {
-  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kMaxP, kExactTheta, 0.0, nt, tx, ty, gv, gu, ns,
+  const Problem q{O2D_CORE_GAUSSIAN, kMaxP, kMaxP, kExactTheta, 0.0, kExactShare16, kExactShareTail, nt, tx, ty, gv, gu, ns,
                   sx, sy, sr, ss, gs, gx, gy, gr, O2D_KT_ADJOINT,
                   near_limit((double)ns, kNearLimitAdjoint, kNearTargetsAdjoint, kNearManyAdjoint)};
   return tree_run<true>(d, s, q);
