@@ -6,10 +6,12 @@
 // [0, 746).
 //
 // Sources and targets go in Morton order, and a group of 16 targets meets only the boxes of 32 sources
-// that its own box can reach. The order is fixed, so sums are reproducible. (A kernel without orders
-// or boxes, two targets a lane, took 58 us at 1,000 particles against 22, 59 at 4,000 against 32, 45 for
-// 200 on 50,000 points against 41; it was faster for 200,000 on 50, 108 against 115, and where the
-// radii reach across the whole domain, 3,000 on 200,000: 442 against 521, 129 at ordinary radii.)
+// that its own box can reach. The order is fixed, so sums are reproducible. (A kernel without boxes, two
+// targets a lane, in orders from 4,096 sources and 1,024 targets on, took 50 us at 1,000 particles against
+// 26, 64 at 4,000 against 47, 262 for 200,000 on 50 points against 111 and 322 for 3,000 on 200,000 against
+// 79. Where the radii reach across the whole domain the boxes leave nothing out, and a call that it did
+// not order pays for its orders: 3,000 on 200,000 461 against 516, 1,000 on 200,000 184 against 204;
+// 50,000 on themselves 1,957 against 1,994. Radii are known on the device only.)
 //
 // A NaN position or radius adds NaN, as in the reference (its tile and its targets' group are never
 // skipped); a non-finite strength or a zero radius beyond the bound adds nothing, where the
@@ -31,11 +33,15 @@ constexpr int kSubs = kTile / kSub;
 constexpr int kGroup = 16;                 // targets per wave of vort_near_kernel
 constexpr int kNearT = 256;                // its threads
 constexpr int kNearTargets = 32;           // its targets: two groups, two waves each
+constexpr int kPer = 2;                    // targets a lane holds
 // rows of tiles that its grid is cut into: kNearWgs workgroups per CU, and at least kNearRows (the
 // workgroups of dense regions last longest, and without rows the launch waits for them): 200,000 wake
 // particles take 394 us a call with one row, 347 with two, 330 with four; 100,000 209, 173 (two)
 // and 148 (three); 20,000 51 with 12 workgroups per CU and 65 with 48
 constexpr int64_t kNearWgs = 12, kNearRows = 3;
+// as long as a row keeps kRowTiles tiles: with fewer the rows' own work is most of it (3,000 particles on
+// 200,000 points 106 us with three rows, 76 with one; 12,000 152 and 141)
+constexpr int64_t kRowTiles = 32;
 constexpr int64_t kPartialBytes = int64_t(1) << 30;  // the cap on the rows' partial sums
 
 struct alignas(16) VSrc {
@@ -166,17 +172,20 @@ __device__ __forceinline__ bool box_near(const VBox& b, double x0, double x1, do
 
 // Targets and sources in Morton order. Bound by the fp64 vector units: an exponential is 20 of a
 // pair's 26 operations, and the boxes decide how many pairs that add exactly 0 are met. A workgroup
-// takes 32 targets; wave w holds group w % 2 of 16 of them, each in four lanes that take every fourth
-// source, and the two waves of a group take the even and the odd boxes. The source tiles that the
-// workgroup's box reaches are listed 256 at a time (in order), and a wave takes the boxes of 32 sources
-// in them that its own 16 targets reach, without waiting for the others. For 200,000 wake particles
-// (radius 0.005, 1.65e8 pairs within the bound) that is 4.0e8 pairs; 64 targets against tiles of 256 were
-// 9.7e8. 735 us and 40 for the sum over chunks -> 319 us and 8. Staging whole tiles between
-// barriers took 548 us, exponentials without the branch around them 60% longer.
+// takes 32 targets; wave w holds group w % 2 of 16 of them, two a lane, each in eight lanes that take every
+// eighth source, and the two waves of a group take the even and the odd boxes. The source tiles that
+// the workgroup's box reaches are listed 256 at a time (in order), and a wave takes the boxes of 32
+// sources in them that its own 16 targets reach, without waiting for the others. For 200,000 wake
+// particles (radius 0.005, 1.65e8 pairs within the bound) that is 4.0e8 pairs; 64 targets against tiles
+// of 256 were 9.7e8. 735 us and 40 for the sum over chunks -> 306 us and 8. Staging whole tiles between
+// barriers took 548 us, exponentials without the branch around them 60% longer. One target a lane reads
+// LDS twice as often for a pair, which shows where most pairs are near: 50,000 particles that all are
+// 2,050 us a call, two 1,990, 200,000 of radius 0.02 6,340 and 6,070, 200,000 wake particles 334 and 322; six
+// waves a SIMD, without spills, where registers alone would leave five.
 //
 // blockIdx.y takes the listed tiles y, y + gridDim.y, ...; out: tw by torder when gridDim.y is 1, else
 // the partial sums part[y nt + p] of the target at position p.
-__global__ __launch_bounds__(kNearT) void vort_near_kernel(int64_t nt, const double* __restrict__ tx,
+__global__ __launch_bounds__(kNearT, 6) void vort_near_kernel(int64_t nt, const double* __restrict__ tx,
                                                            const double* __restrict__ ty,
                                                            const uint32_t* __restrict__ torder,
                                                            int64_t ntiles, const VSrc* __restrict__ vs,
@@ -184,8 +193,9 @@ __global__ __launch_bounds__(kNearT) void vort_near_kernel(int64_t nt, const dou
                                                            const VBox* __restrict__ tbox,
                                                            double* __restrict__ tw,
                                                            double* __restrict__ part) {
-  constexpr int kWaves = kNearT / 64, kGroups = kNearTargets / kGroup, kLanes = 64 / kGroup;
-  static_assert(kWaves == 2 * kGroups && kLanes == 4, "two waves a group, four lanes a target");
+  constexpr int kWaves = kNearT / 64, kGroups = kNearTargets / kGroup;
+  constexpr int kSpan = kGroup / kPer, kLanes = 64 / kSpan;
+  static_assert(kWaves == 2 * kGroups && kSub % kLanes == 0, "two waves a group, whole shares");
   static_assert(sizeof(VSrc) * kSub == 64 * sizeof(double2), "a box's sources are one load a lane");
   __shared__ VSrc staged[kWaves][kSub];
   __shared__ double e2t[64];  // kExp2Tab
@@ -193,18 +203,29 @@ __global__ __launch_bounds__(kNearT) void vort_near_kernel(int64_t nt, const dou
   __shared__ uint32_t list[kNearT], found[kWaves];
   __shared__ double sum[kGroups][kGroup];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, group = wave % kGroups;
-  const int half = wave / kGroups, q4 = lane / kGroup;
+  const int half = wave / kGroups, share = lane / kSpan;
   VSrc* mine = staged[wave];
   if (t < 64) e2t[t] = kExp2Tab[t];
-  const int64_t p = (int64_t)blockIdx.x * kNearTargets + group * kGroup + (lane & (kGroup - 1));
-  const uint32_t o = torder[p < nt ? p : nt - 1];
-  const double px = tx[o], py = ty[o];
+  const int64_t p0 = (int64_t)blockIdx.x * kNearTargets + group * kGroup + lane % kSpan;
+  uint32_t o[kPer];
+  double px[kPer], py[kPer], acc[kPer];
   // the group's box, and the workgroup's (a NaN position: unbounded)
-  const bool bad = !(px == px) || !(py == py);
-  double x0 = bad ? -INFINITY : px, x1 = bad ? INFINITY : px;
-  double y0 = bad ? -INFINITY : py, y1 = bad ? INFINITY : py;
+  double x0 = INFINITY, x1 = -INFINITY, y0 = INFINITY, y1 = -INFINITY;
 #pragma unroll
-  for (int s = kGroup / 2; s > 0; s >>= 1) {
+  for (int e = 0; e < kPer; ++e) {
+    const int64_t p = p0 + e * kSpan;
+    o[e] = torder[p < nt ? p : nt - 1];
+    px[e] = tx[o[e]];
+    py[e] = ty[o[e]];
+    acc[e] = 0.0;
+    const bool bad = !(px[e] == px[e]) || !(py[e] == py[e]);
+    x0 = fmin(x0, bad ? -INFINITY : px[e]);
+    x1 = fmax(x1, bad ? INFINITY : px[e]);
+    y0 = fmin(y0, bad ? -INFINITY : py[e]);
+    y1 = fmax(y1, bad ? INFINITY : py[e]);
+  }
+#pragma unroll
+  for (int s = kSpan / 2; s > 0; s >>= 1) {
     x0 = fmin(x0, __shfl_xor(x0, s, 64));
     x1 = fmax(x1, __shfl_xor(x1, s, 64));
     y0 = fmin(y0, __shfl_xor(y0, s, 64));
@@ -224,7 +245,6 @@ __global__ __launch_bounds__(kNearT) void vort_near_kernel(int64_t nt, const dou
     wy0 = fmin(wy0, gb[k][2]);
     wy1 = fmax(wy1, gb[k][3]);
   }
-  double acc = 0.0;
   for (int64_t base = 0; base < ntiles; base += (int64_t)kNearT * gridDim.y) {
     // the next kNearT of this row's tiles
     const int64_t it = base + (int64_t)t * gridDim.y + blockIdx.y;
@@ -267,26 +287,36 @@ __global__ __launch_bounds__(kNearT) void vort_near_kernel(int64_t nt, const dou
         }
 #pragma unroll
         for (int k = 0; k < kSub / kLanes; ++k) {
-          const VSrc c = mine[k * kLanes + q4];
-          const double dx = px - c.x, dy = py - c.y;
-          const double x = (dx * dx + dy * dy) * c.rr;
-          if (!(x >= kUnderflow)) acc += c.c * exp_neg(x, e2t);  // a NaN exponent adds NaN
+          const VSrc c = mine[k * kLanes + share];
+#pragma unroll
+          for (int e = 0; e < kPer; ++e) {
+            const double dx = px[e] - c.x, dy = py[e] - c.y;
+            const double x = (dx * dx + dy * dy) * c.rr;
+            if (!(x >= kUnderflow)) acc[e] += c.c * exp_neg(x, e2t);  // a NaN exponent adds NaN
+          }
         }
       }
     }
     __syncthreads();  // before the list changes
   }
-  // a target's four lanes, then its two waves
-  acc += __shfl_xor(acc, kGroup, 64);
-  acc += __shfl_xor(acc, 2 * kGroup, 64);
-  if (half == 1 && lane < kGroup) sum[group][lane] = acc;
+  // a target's lanes, then its two waves
+#pragma unroll
+  for (int e = 0; e < kPer; ++e) {
+#pragma unroll
+    for (int s = kSpan; s < 64; s <<= 1) acc[e] += __shfl_xor(acc[e], s, 64);
+    if (half == 1 && share == 0) sum[group][e * kSpan + lane] = acc[e];
+  }
   __syncthreads();
-  if (half == 0 && lane < kGroup && p < nt) {
-    acc += sum[group][lane];
+  if (half != 0 || share != 0) return;
+#pragma unroll
+  for (int e = 0; e < kPer; ++e) {
+    const int64_t p = p0 + e * kSpan;
+    if (p >= nt) continue;
+    const double s = acc[e] + sum[group][e * kSpan + lane];
     if (part)
-      part[(int64_t)blockIdx.y * nt + p] = acc;
+      part[(int64_t)blockIdx.y * nt + p] = s;
     else
-      tw[o] += acc;
+      tw[o[e]] += s;
   }
 }
 
@@ -324,7 +354,7 @@ int vorticity_dev(Device* d, hipStream_t s, int64_t ns, const double* sx, const 
   if (!(tx == sx && ty == sy && nt == ns)) O2D_TRY(morton_order16(d, s, nt, tx, ty, &torder));
   const int64_t twgs = (nt + kNearTargets - 1) / kNearTargets;
   const int64_t want = kNearWgs * (int64_t)d->num_cu;
-  int64_t rows = std::max((want + twgs - 1) / twgs, kNearRows);
+  int64_t rows = std::max((want + twgs - 1) / twgs, std::min(kNearRows, ntiles / kRowTiles));
   rows = std::min({rows, ntiles, kPartialBytes / ((int64_t)sizeof(double) * nt)});
   rows = std::max<int64_t>(rows, 1);
   void* part = nullptr;
