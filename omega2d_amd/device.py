@@ -36,6 +36,13 @@ def _check(*ts, dtype=torch.float64):
     return dev
 
 
+def _sizes(n, *ts):
+    """The kernels take one count for all of a call's arrays."""
+    for t in ts:
+        if t.numel() != n:
+            raise ValueError(f"expected {n} entries, got {t.numel()}")
+
+
 def env_for(device, core="v2", precision="fp64", results="vel"):
     idx = device.index if device.index is not None else torch.cuda.current_device()
     stream = torch.cuda.current_stream(device).cuda_stream
@@ -132,6 +139,9 @@ def rk_advance(x0, y0, us, vs, w, dt, x=None, y=None, combined=False):
     y = torch.empty_like(y0) if y is None else y
     uc, vc = (torch.empty_like(x0), torch.empty_like(y0)) if combined else (None, None)
     dev = _check(x0, y0, x, y, *us, *vs)
+    _sizes(x.numel(), x0, y0, y, *us, *vs)
+    if not len(us) == len(vs) == len(w):
+        raise ValueError("a stage needs u, v and a weight")
     env = env_for(dev)
     wv = (ctypes.c_double * len(w))(*[float(a) for a in w])
     up = (ctypes.c_void_p * len(us))(*[u.data_ptr() for u in us])
@@ -144,6 +154,7 @@ def rk_advance(x0, y0, us, vs, w, dt, x=None, y=None, combined=False):
 def finalize(u, v, fs, factor):
     """In place u = fs[0] + u * factor, v = fs[1] + v * factor."""
     dev = _check(u, v)
+    _sizes(u.numel(), v)
     env = env_for(dev)
     call("o2d_hip_finalize_dev_d", ctypes.byref(env), u.numel(), float(fs[0]), float(fs[1]),
          float(factor), _ptr(u), _ptr(v))
@@ -153,6 +164,8 @@ def finalize(u, v, fs, factor):
 def body_rhs(pu, pv, fs, factor, tx, ty, nx, ny, nunk, reabsorbed, vol2, omega_error):
     """The right-hand side of a body's system from the unscaled sums pu, pv at its panels."""
     dev = _check(pu, pv, tx, ty, nx, ny, reabsorbed, omega_error)
+    _sizes(pu.numel(), pv, tx, ty, nx, ny)
+    _sizes(1, reabsorbed, omega_error)
     rhs = torch.empty(pu.numel() * nunk + 1, dtype=torch.float64, device=dev)
     env = env_for(dev)
     call("o2d_hip_body_rhs_dev_d", ctypes.byref(env), pu.numel(), int(nunk), float(fs[0]),
@@ -164,7 +177,8 @@ def body_rhs(pu, pv, fs, factor, tx, ty, nx, ny, nunk, reabsorbed, vol2, omega_e
 def body_unpack(sol, nunk):
     """The solution's vortex and source strengths, rotation and rotation error, as new tensors."""
     dev = _check(sol)
-    npan = (sol.numel() - 1) // nunk
+    npan = max(0, sol.numel() - 1) // nunk
+    _sizes(npan * nunk + 1, sol)
     vs, ss = (torch.empty(npan, dtype=torch.float64, device=dev) for _ in range(2))
     omega, error = (torch.empty((), dtype=torch.float64, device=dev) for _ in range(2))
     env = env_for(dev)
@@ -176,6 +190,8 @@ def body_unpack(sol, nunk):
 def body_strengths(vs, ss, omega, tx, ty, ddx, ddy):
     """Panel strengths vs, ss with those of the rotation omega added, as new tensors."""
     dev = _check(vs, ss, omega, tx, ty, ddx, ddy)
+    _sizes(vs.numel(), ss, tx, ty, ddx, ddy)
+    _sizes(1, omega)
     ovs, oss = torch.empty_like(vs), torch.empty_like(ss)
     env = env_for(dev)
     call("o2d_hip_body_strengths_dev_d", ctypes.byref(env), vs.numel(), _ptr(vs), _ptr(ss),
