@@ -472,7 +472,10 @@ struct Outputs {
 // Bound by the latency of its loads where targets are few (10,000 targets, 40 chunks: 7.8 us with a
 // thread per target, 4.5 split; 100 targets, 938 chunks: 24 with four waves, 15 with 16), by bandwidth
 // where they are many and chunks few (250,000 targets, 2 chunks of 4 components: 30 us with a thread per
-// target, 39 split).
+// target, 39 split) and where they fill the chip by themselves (whole calls, 100 panels on 15,000, 60,000,
+// 100,000 and 200,000 points: 28.5, 36.3, 45.4 and 69.1 with a thread per target, 24.9, 36.4, 47.8 and 74.0
+// split).
+constexpr int64_t kSplitChunks = 8, kSplitTargets = 65536;
 template <int NF, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? kReduceT : kBlock) void reduce_chunks_kernel(
     int64_t nchunk, int64_t nt, const uint32_t* __restrict__ order, const double* __restrict__ part,
@@ -744,7 +747,7 @@ int gather_targets(hipStream_t s, int core, int64_t n, const uint32_t* order, co
 int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* order, int nf,
                   const double* part, double* o0, double* o1, double* o2, double* o3,
                   const int* gate, int open) {
-  const bool split = nchunk >= 8;
+  const bool split = nchunk >= kSplitChunks && nt < kSplitTargets;
   const unsigned grid = split ? (unsigned)((nt + 63) / 64) : grid1(nt).x;
   const Outputs out{{o0, o1, o2, o3}};
 #define O2D_REDUCE(NF)                                                                      \
