@@ -23,8 +23,11 @@ __global__ void d2f_kernel(int64_t n, const double* __restrict__ a, float* __res
 // its outputs, at once through page-locked memory: an array by itself costs a copy of 3 us on the
 // device and about as much on the host, and in float a conversion launch. 1,531 float particles on
 // themselves: 160 us with nine uploads and two downloads, 77 packed; in double 119 and 68; 60,000
-// (1.9 and 3.8 MB) 1,052 and 935, 1,037 and 997; 300,000 on 300 points (9.6 MB in double) 532 and 514.
-constexpr size_t kPackBytes = size_t(16) << 20;
+// (1.9 and 3.8 MB) 1,052 and 935, 1,037 and 997; 500,000 on 100 points (15 MB in double) 1,271 and 749.
+// Outputs pass through that memory three times, and from kPackOut bytes of them array by array is the
+// faster: 100 on 150,000, 200,000 and 240,000 points in double 492, 554 and 601 us, packed 425, 552 and
+// 640; on 400,000 and 500,000 in float 649 and 716, packed 602 and 753.
+constexpr size_t kPackBytes = size_t(16) << 20, kPackOut = size_t(3) << 20;
 constexpr int64_t kPackAlign = 32;  // elements: each array starts on 128 bytes or more
 
 template <class T>
@@ -67,7 +70,7 @@ int points_packed(Device* d, hipStream_t s, const o2d_env* env, int64_t ns, cons
   for (int k = 0; k < 7; ++k) at[k] = in[k] ? p.add(k < 4 ? ns : nt) : -1;
   const int64_t first = p.n;  // of the outputs
   for (int k = 0; k < 3; ++k) ot[k] = out[k] ? p.add(nt) : -1;
-  if (sizeof(T) * (size_t)p.n > kPackBytes) return 0;
+  if (sizeof(T) * (size_t)p.n > kPackBytes || sizeof(T) * (size_t)(p.n - first) > kPackOut) return 0;
   *done = true;
   void *h, *v;
   O2D_TRY(pinned(d, sizeof(T) * p.n, &h));
