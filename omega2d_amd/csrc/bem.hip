@@ -13,6 +13,8 @@
 // src/Coefficients.h:464-537.
 #include <rocblas/rocblas.h>
 #include <algorithm>
+#include <memory>
+#include <new>
 #include <rocsolver/rocsolver.h>
 
 #include "nbody.h"
@@ -268,7 +270,25 @@ int bem_assemble_pair_dev(Device* d, hipStream_t s, const double* snx, const dou
   return 0;
 }
 
+// The row permutation that the row interchanges piv (1-based, on the device) compose to, into perm: row i
+// of the factors is row perm[i] of the matrix. On the host: the library's factorisation, which alone needs
+// it, takes 60 ms at the smallest order it is used for.
+static int compose_rows(hipStream_t s, int n, const int* piv, int* perm) {
+  const std::unique_ptr<int[]> p(new (std::nothrow) int[2 * (size_t)n]);
+  if (!p) return fail(O2D_ERR_STATE, "out of host memory");
+  int *rows = p.get(), *swaps = rows + n;
+  O2D_HIP(hipMemcpyAsync(swaps, piv, sizeof(int) * n, hipMemcpyDeviceToHost, s));
+  O2D_HIP(hipStreamSynchronize(s));
+  for (int i = 0; i < n; ++i) rows[i] = i;
+  for (int i = 0; i < n; ++i)
+    if (swaps[i] >= 1 && swaps[i] <= n) std::swap(rows[i], rows[swaps[i] - 1]);
+  O2D_HIP(hipMemcpyAsync(perm, rows, sizeof(int) * n, hipMemcpyHostToDevice, s));
+  O2D_HIP(hipStreamSynchronize(s));
+  return 0;
+}
+
 int bem_factor_dev(Device* d, hipStream_t s, int64_t n, const double* A, int64_t lda) {
+  static_assert(sizeof(rocblas_int) == sizeof(int), "pivots as int");
   d->lu_ready = false;
   d->inv_ready = false;
   d->lu_solves = 0;
@@ -280,23 +300,26 @@ int bem_factor_dev(Device* d, hipStream_t s, int64_t n, const double* A, int64_t
   O2D_TRY(slot(d, kSolveTmp, solve_scratch(n), s, &scratch));
   O2D_HIP(hipMemcpy2DAsync(lu, sizeof(double) * n, A, sizeof(double) * lda, sizeof(double) * n, n,
                            hipMemcpyDeviceToDevice, s));
-  rocblas_handle h;
-  O2D_TRY(blas_of(d, s, &h));
-  if (n <= lu_max_order()) {
-    void* perm;
-    O2D_TRY(slot(d, kLuPerm, sizeof(int) * n, s, &perm));
+  void* perm;
+  O2D_TRY(slot(d, kLuPerm, sizeof(int) * n, s, &perm));
+  const bool own = n <= lu_max_order();
+  if (own) {
     O2D_TRY(lu_factor_dev(d, s, (int)n, static_cast<double*>(lu), (int)n, static_cast<int*>(piv),
                           static_cast<int*>(perm), static_cast<int*>(info)));
-    O2D_TRY(lu_prepare_solve(d, s, (int)n, static_cast<const double*>(lu)));
-  } else if (rocsolver_dgetrf(h, (rocblas_int)n, (rocblas_int)n, static_cast<double*>(lu),
-                              (rocblas_int)n, static_cast<rocblas_int*>(piv),
-                              static_cast<rocblas_int*>(info)) != rocblas_status_success) {
-    return fail(O2D_ERR_HIP, "rocsolver_dgetrf failed");
+  } else {
+    rocblas_handle h;
+    O2D_TRY(blas_of(d, s, &h));
+    if (rocsolver_dgetrf(h, (rocblas_int)n, (rocblas_int)n, static_cast<double*>(lu), (rocblas_int)n,
+                         static_cast<rocblas_int*>(piv),
+                         static_cast<rocblas_int*>(info)) != rocblas_status_success)
+      return fail(O2D_ERR_HIP, "rocsolver_dgetrf failed");
   }
+  O2D_TRY(lu_prepare_solve(d, s, (int)n, static_cast<const double*>(lu)));
   rocblas_int hinfo = 0;
   O2D_HIP(hipMemcpyAsync(&hinfo, info, sizeof(hinfo), hipMemcpyDeviceToHost, s));
   O2D_HIP(hipStreamSynchronize(s));
   if (hinfo != 0) return fail(O2D_ERR_STATE, "BEM matrix is singular (getrf info=%d)", (int)hinfo);
+  if (!own) O2D_TRY(compose_rows(s, (int)n, static_cast<const int*>(piv), static_cast<int*>(perm)));
   d->lu_n = n;
   d->lu_ready = true;
   return 0;
@@ -317,10 +340,10 @@ __global__ __launch_bounds__(kBlock) void identity_kernel(int64_t n, double* __r
 // is one matrix-vector product (0.013 ms at 2049, against 0.27 by two triangular solves). A body that
 // does not move keeps its inverse for the whole run; a body in relative motion, refactored every
 // step and solved once per Runge-Kutta stage, never builds it: its two or three solves cost less.
-// Beyond lu_max_order, where the library's triangular solves cost as much as the inverse, the second
-// solve builds it. A solve under stream capture allocates nothing and calls no library routine up to
-// lu_max_order: it goes by the factors unless the inverse is there.
-constexpr int kSolvesBeforeInverse = 3, kLibrarySolvesBeforeInverse = 1;
+// A solve under stream capture allocates nothing and calls no library routine: it goes by the factors
+// unless the inverse is there. (Past lu_max_order the factors are the library's, in the same layout. Its
+// triangular solves of one column take 5 ms at order 6,145, where the inverse is built in 15.)
+constexpr int kSolvesBeforeInverse = 3;
 
 bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -331,9 +354,7 @@ bool capturing(hipStream_t s) {
 int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* x) {
   if (!d->lu_ready || d->lu_n != n)
     return fail(O2D_ERR_STATE, "no LU factors of size %lld (factor first)", (long long)n);
-  const bool own = n <= lu_max_order();
-  if (!d->inv_ready && d->lu_solves >= (own ? kSolvesBeforeInverse : kLibrarySolvesBeforeInverse) &&
-      !(own && capturing(s))) {
+  if (!d->inv_ready && d->lu_solves >= kSolvesBeforeInverse && !capturing(s)) {
     rocblas_handle h;
     O2D_TRY(blas_of(d, s, &h));
     void* inv;
@@ -352,17 +373,8 @@ int bem_solve_dev(Device* d, hipStream_t s, int64_t n, const double* b, double* 
   ++d->lu_solves;
   if (d->inv_ready)
     return matvec_dev(d, s, (int)n, static_cast<const double*>(d->buf[kInv]), b, x);
-  if (own)
-    return lu_solve_dev(d, s, (int)n, static_cast<const double*>(d->buf[kLU]),
-                        static_cast<const int*>(d->buf[kLuPerm]), b, x);
-  rocblas_handle h;
-  O2D_TRY(blas_of(d, s, &h));
-  if (x != b) O2D_HIP(hipMemcpyAsync(x, b, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-  if (rocsolver_dgetrs(h, rocblas_operation_none, (rocblas_int)n, 1, static_cast<double*>(d->buf[kLU]),
-                       (rocblas_int)n, static_cast<const rocblas_int*>(d->buf[kPivots]), x,
-                       (rocblas_int)n) != rocblas_status_success)
-    return fail(O2D_ERR_HIP, "rocsolver_dgetrs failed");
-  return 0;
+  return lu_solve_dev(d, s, (int)n, static_cast<const double*>(d->buf[kLU]),
+                      static_cast<const int*>(d->buf[kLuPerm]), b, x);
 }
 
 static int check_bem(const o2d_env* env, int64_t nnodes, const void* nx, const void* ny,

@@ -45,13 +45,30 @@ def test_captured_solves(n, before):
 
 
 def test_solves_past_the_blocked_factorisation():
-    """From order 6,145 the factors are the library's: the first solve by them, then by the inverse."""
+    """From order 6,145 the factors are the library's: three solves by them, the later ones by the
+    inverse, and a captured one."""
     n = 6145
     g = torch.Generator(device="cuda").manual_seed(1)
     A = torch.randn((n, n), dtype=torch.float64, device="cuda", generator=g) * (0.25 / np.sqrt(n))
     A += torch.eye(n, dtype=torch.float64, device="cuda")
+    A = A[torch.randperm(n, device="cuda", generator=g)]
     dv.bem_factor(A.T.contiguous())
-    for _ in range(3):
-        b = torch.randn(n, dtype=torch.float64, device="cuda", generator=g)
-        x = dv.bem_solve(b)
+    new = lambda: torch.randn(n, dtype=torch.float64, device="cuda", generator=g)  # noqa: E731
+
+    def check(x, b):
         assert float((A @ x - b).norm() / b.norm()) <= 1e-12
+
+    b = new()
+    check(dv.bem_solve(b), b)
+    held, x = new(), torch.empty_like(b)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        dv.bem_solve(held, x)
+    for _ in range(4):
+        held.copy_(new())
+        graph.replay()
+        torch.cuda.synchronize()
+        check(x, held)
+        b = new()
+        check(dv.bem_solve(b), b)
