@@ -25,17 +25,51 @@ constexpr int kSB = 64;     // rows per block of a triangular solve
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kChunk = 32;  // columns per workgroup of the matrix-vector product
+constexpr int kOnceT = 1024, kOnceMax = 256;  // threads and largest order of its form in one launch
 static_assert(kSB == 64, "a lane per row of a block");
 
 // The inverses of the diagonal blocks of L (unit lower; blockIdx.y = 0) and U (upper; 1), padded
-// with the identity past n: dinv[((y nblk) + block) kSB^2 + k kSB + i] = inverse(i, k), by
-// substitution. Four lanes of one wave share the sums of column k, so a column needs no workgroup
-// barrier. (One lane a column took 86 us at order 2049; with the column in registers and every
-// loop unrolled, 190: code that runs once comes in from memory.)
+// with the identity past n: dinv[((y nblk) + block) kSB^2 + k kSB + i] = inverse(i, k). Each wave inverts
+// one of the four diagonal kSub x kSub blocks by substitution, four lanes to a column; then, twice,
+// pairs of inverted blocks X11, X22 are joined over the block M21 between them: X21 = -X22 (M21 X11).
+// Bound by the latency of its chain: substitution over all 64 rows took 38 us at any order, this takes
+// 17 (the factorisation of order 50 with one solve 178 and 157).
+constexpr int kSub = 16;
+
+// x[h + i][k] = -sum_l X22[i][l] (M21 X11)[l][k] for the kH x kH block below and left of the middle of the
+// 2 kH rows from r on; the sum's first product stands in x's own place in between. PAIRS of them at a time.
+template <int kH, int PAIRS>
+__device__ void join_blocks(const double (*m)[kSB + 1], double (*x)[kSB + 1]) {
+  constexpr int kEach = PAIRS * kH * kH / kBlock;
+  static_assert(PAIRS * 2 * kH == kSB && kEach >= 1, "all rows, whole shares");
+  double v[kEach];
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) {
+      const int e = threadIdx.x + u * kBlock;
+      const int r = e / (kH * kH) * 2 * kH, i = e / kH % kH, k = e % kH;
+      double s = 0.0;
+#pragma unroll 8
+      for (int l = 0; l < kH; ++l)
+        s = pass == 0 ? __builtin_fma(m[r + kH + i][r + l], x[r + l][r + k], s)
+                      : __builtin_fma(-x[r + kH + i][r + kH + l], x[r + kH + l][r + k], s);
+      v[u] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) {
+      const int e = threadIdx.x + u * kBlock;
+      x[e / (kH * kH) * 2 * kH + kH + e / kH % kH][e / (kH * kH) * 2 * kH + e % kH] = v[u];
+    }
+    __syncthreads();
+  }
+}
+
 __global__ __launch_bounds__(kBlock) void lu_diag_inverse_kernel(int n, int nblk,
                                                                  const double* __restrict__ lu,
                                                                  double* __restrict__ dinv) {
-  static_assert(kBlock == 4 * kSB, "four lanes per column");
+  static_assert(kSB == kWaves * kSub && 64 == 4 * kSub, "a wave per block, four lanes per column");
   __shared__ double m[kSB][kSB + 1];  // m[r][c]: the block; of U, its mirror
   __shared__ double x[kSB][kSB + 1];  // x[i][k]
   const int t = threadIdx.x, b = blockIdx.x, r0 = b * kSB;
@@ -50,22 +84,31 @@ __global__ __launch_bounds__(kBlock) void lu_diag_inverse_kernel(int n, int nblk
     if (r == c && (!upper || !in)) v = 1.0;
     if (upper) m[kSB - 1 - r][kSB - 1 - c] = v;
     else m[r][c] = v;
+    x[r][c] = 0.0;
   }
   __syncthreads();
-  const int k = t / 4, q = t % 4;
-  for (int i = 0; i < kSB; ++i) {
-    double s = 0.0;
-#pragma unroll 4
-    for (int j = q; j < i; j += 4) s = __builtin_fma(-m[i][j], x[j][k], s);
-    s += __shfl_xor(s, 1, 64);
-    s += __shfl_xor(s, 2, 64);
-    s += k == i ? 1.0 : 0.0;
-    if (q == 0) x[i][k] = upper ? s / m[i][i] : s;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  {
+    const int o = t / 64 * kSub, k = t % 64 / 4, q = t % 4;  // rows of this wave's block, column, lane
+    double mine[kSub / 4];  // x[q + 4 l][k]
+#pragma unroll
+    for (int i = 0; i < kSub; ++i) {
+      double s = 0.0;
+#pragma unroll
+      for (int l = 0; 4 * l < i; ++l)
+        if (q + 4 * l < i) s = __builtin_fma(-m[o + i][o + q + 4 * l], mine[l], s);
+      s += __shfl_xor(s, 1, 64);
+      s += __shfl_xor(s, 2, 64);
+      s += k == i ? 1.0 : 0.0;
+      if (upper) s /= m[o + i][o + i];
+      if (q == i % 4) {
+        mine[i / 4] = s;
+        x[o + i][o + k] = s;
+      }
+    }
   }
   __syncthreads();
+  join_blocks<kSub, 2>(m, x);
+  join_blocks<2 * kSub, 1>(m, x);
   double* out = dinv + ((int64_t)blockIdx.y * nblk + b) * kSB * kSB;
 #pragma unroll 4
   for (int e = t; e < kSB * kSB; e += kBlock) {
@@ -163,6 +206,28 @@ __global__ __launch_bounds__(kBlock) void matvec_sum_kernel(int n, int nchunk,
   if (wave == 0 && row < n) x[row] = ((sm[0][lane] + sm[1][lane]) + sm[2][lane]) + sm[3][lane];
 }
 
+// x = a b in one launch, for small orders: a workgroup takes 64 rows, its 16 waves every 16th column, added
+// in wave order. Order 50 2.1 us, 3.3 in two launches, 200 4.2 and 4.3, 300 5.6 and 4.7 (in a graph; a call
+// by itself, which waits for its launches, 6.9 and 9.3)
+__global__ __launch_bounds__(kOnceT) void matvec_once_kernel(int n, const double* __restrict__ a,
+                                                             const double* b, double* x) {
+  constexpr int kW = kOnceT / 64;
+  __shared__ double sm[kW][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = blockIdx.x * 64 + lane;
+  double s = 0.0;
+  if (row < n) {
+#pragma unroll 8
+    for (int c = wave; c < n; c += kW) s = __builtin_fma(a[(int64_t)c * n + row], b[c], s);
+  }
+  sm[wave][lane] = s;
+  __syncthreads();
+  if (wave != 0 || row >= n) return;
+#pragma unroll
+  for (int w = 1; w < kW; ++w) s += sm[w][lane];
+  x[row] = s;
+}
+
 inline int blocks_of(int64_t n) { return (int)((n + kSB - 1) / kSB); }
 
 }  // namespace
@@ -211,6 +276,11 @@ int lu_solve_dev(Device* d, hipStream_t s, int n, const double* lu, const int* p
 
 // x = A b, A n x n column-major (x may alias b)
 int matvec_dev(Device* d, hipStream_t s, int n, const double* a, const double* b, double* x) {
+  if (n <= kOnceMax && (x != b || n <= 64)) {  // (in place, another workgroup could still read b)
+    matvec_once_kernel<<<blocks_of(n), kOnceT, 0, s>>>(n, a, b, x);
+    O2D_LAUNCH_CHECK();
+    return 0;
+  }
   const int nchunk = (n + kChunk - 1) / kChunk;
   void* p;
   O2D_TRY(slot(d, kSolveTmp, solve_scratch(n), s, &p));

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("before", [0, 1, 2, 3, 4, 5])
-@pytest.mark.parametrize("n", [1, 65, 513])
+@pytest.mark.parametrize("n", [1, 64, 65, 256, 257, 513])
 def test_captured_solves(n, before):
     rng = np.random.default_rng(n + before)
     A = (np.eye(n) + 0.25 * rng.normal(size=(n, n)) / np.sqrt(n))[rng.permutation(n)]
@@ -72,3 +72,17 @@ def test_solves_past_the_blocked_factorisation():
         check(x, held)
         b = new()
         check(dv.bem_solve(b), b)
+
+
+@pytest.mark.parametrize("n", [16, 17, 63, 64, 65, 255, 256, 257])
+def test_solves_in_place(n):
+    """Every solve of a run in place: by the factors, then by the inverse on both sides of the order up to
+    which its product is one launch."""
+    rng = np.random.default_rng(n)
+    A = (np.eye(n) + 0.25 * rng.normal(size=(n, n)) / np.sqrt(n))[rng.permutation(n)]
+    dv.bem_factor(torch.from_numpy(np.ascontiguousarray(A.T)).cuda())
+    for k in range(6):
+        b = rng.normal(size=n)
+        x = torch.from_numpy(b).cuda()
+        dv.bem_solve(x, x)
+        assert rel_l2(x.cpu().numpy(), np.linalg.solve(A, b)) <= 1e-12, k
