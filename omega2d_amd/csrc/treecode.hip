@@ -91,10 +91,13 @@ constexpr int64_t kSparse = 12, kSparseAdjoint = 64;
 // opens the same cells, so more of them cost more (1M particles: 32 and 64 equal), unless they no
 // longer fit the chip at once (16 per CU do): 20,000 particles take 163 us at 16 or just below and 175
 // at 32, 100,000 and 8,000 targets in groups of 16 214 at or just below 16 and 222 just above. From
-// kEvenGroups groups on a second round of waves costs less than groups of unequal work (40,000
-// targets 635 and 660 us, 262,144 1,437 and 1,698).
+// kEvenGroups groups on a second round of waves costs less than groups of unequal work (30,000 targets of
+// which many are within the cores 394 and 418 us, 40,000 635 and 660, 262,144 1,437 and 1,698). (Opening
+// the same cells in every share is also why small theta gains nothing over the earlier form, whose shares
+// began at different cells, where targets are few: 200,000 sources on 12,500 at theta 0.3 404 us against
+// 412, 0.2 555 and 474, 0.1 1,090 and 560.)
 constexpr int kWaves64 = 32, kWavesOnce = 16;
-constexpr int64_t kEvenGroups = 512;
+constexpr int64_t kEvenGroups = 400;
 // Fewer super groups than this leave most of the chip idle for longer than they save: us with and without,
 // 40,000 blob particles on themselves (40 of them) 237 and 225, 90,000 339 and 325, 110,000 382 and 373,
 // 130,000 412 and 417, 262,144 717 and 743, 524,288 1,220 and 1,325; the adjoint of 30,000 particles 301 and
