@@ -37,7 +37,7 @@ struct alignas(16) Probe {
   double x, y, gu, gv;
 };
 
-template <int CORE, int TPL>
+template <int CORE, int TPL, bool GATED>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void adjoint_kernel(
     int64_t ns, const double* __restrict__ sx, const double* __restrict__ sy,
@@ -45,7 +45,9 @@ void adjoint_kernel(
     const double* __restrict__ tx, const double* __restrict__ ty, const double* __restrict__ gu,
     const double* __restrict__ gv, int64_t chunk, double* __restrict__ ox, double* __restrict__ oy,
     double* __restrict__ os, double* __restrict__ orr, int direct, const int* __restrict__ gate) {
-  if (CORE == O2D_CORE_GAUSSIAN && gate && *gate == 0) return;
+  if constexpr (GATED) {
+    if (*gate == 0) return;
+  }
   __shared__ Probe tile[kTile];
   __shared__ double4 box[kBlock / 64];
   const int tid = threadIdx.x;
@@ -166,12 +168,12 @@ void adjoint_kernel(
   }
 }
 
-template <int CORE>
+template <int CORE, bool GATED = false>
 void launch_adj(dim3 grid, hipStream_t s, int64_t ns, const double* sx, const double* sy,
                 const double* ss, const double* sr, int64_t nt, const double* tx,
                 const double* ty, const double* gu, const double* gv, int64_t chunk, double* ox,
                 double* oy, double* os, double* orr, int direct, const int* gate) {
-  adjoint_kernel<CORE, kTpl><<<grid, kBlock, 0, s>>>(ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, chunk,
+  adjoint_kernel<CORE, kTpl, GATED><<<grid, kBlock, 0, s>>>(ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, chunk,
                                                      ox, oy, os, orr, direct, gate);
 }
 
@@ -215,7 +217,10 @@ int adjoint_pairs_dev(Device* d, hipStream_t s, int core, int64_t ns, const doub
 #define O2D_LADJ(C) launch_adj<C>(grid, s, ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, chunk, ox, oy, os, orr, direct, gate)
   switch (core) {
     case O2D_CORE_RM: O2D_LADJ(O2D_CORE_RM); break;
-    case O2D_CORE_GAUSSIAN: O2D_LADJ(O2D_CORE_GAUSSIAN); break;
+    case O2D_CORE_GAUSSIAN:
+      if (gate) launch_adj<O2D_CORE_GAUSSIAN, true>(grid, s, ns, sx, sy, ss, sr, nt, tx, ty, gu, gv, chunk, ox, oy, os, orr, direct, gate);
+      else O2D_LADJ(O2D_CORE_GAUSSIAN);
+      break;
     case O2D_CORE_WL: O2D_LADJ(O2D_CORE_WL); break;
     case O2D_CORE_V2: O2D_LADJ(O2D_CORE_V2); break;
     default: O2D_LADJ(O2D_CORE_V3); break;

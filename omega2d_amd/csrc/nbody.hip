@@ -25,7 +25,6 @@
 // atomics, so results are reproducible run to run).
 #include <algorithm>
 #include <cstring>
-#include <optional>
 
 #include "nbody.h"
 #include "o2d_math.h"
@@ -108,17 +107,10 @@ __device__ __forceinline__ void tile_pairs64(const Src64* __restrict__ tile, int
   }
 }
 
-// The targets of the fp64 form, in Morton order: positions at pos[pstep i], radius terms (if any) at
-// w[wstep i], and order[i], the input index of sorted target i (null: they are in input order)
-struct Targets64 {
-  const double2* pos;
-  const double* w;
-  const uint32_t* order;
-  int pstep, wstep;
-};
-
-// src: the staged sources in Morton order. gate (the Gaussian's velocity only): a device flag, or null;
-// while it is 0 the kernel does nothing.
+// src: the staged sources in Morton order; tq, tw: the targets' positions and radius terms in
+// Morton order (tw unused unless TR); torder[i]: the input index of sorted target i (torder
+// null: the targets are in input order). GATED: nothing is done while *gate is 0, and tq and tw point
+// into records of four (x, y, strength, radius term).
 //
 // Bound by the fp64 vector units (a Rosenhead-Moore or far Gaussian pair is 11 fp64 operations and
 // a reciprocal), by latency where the sum is small:
@@ -133,15 +125,19 @@ struct Targets64 {
 // one: Rosenhead-Moore particles 253 and 262 us, 32,000 481 and 498; blob particles, pair by pair, 361 and
 // 313 and 590 and 556. Beyond it two targets a lane halve the LDS reads per pair (a 262k blob sum is 4%
 // slower inline).
-template <int CORE, int RES, bool TR, int TPL, bool FEW>
+template <int CORE, int RES, bool TR, int TPL, bool FEW, bool GATED>
 __global__ __launch_bounds__(kBlock) void nbody64_kernel(
-    int64_t ns, const Src64* __restrict__ src, int64_t nt, Targets64 tg, int64_t chunk,
+    int64_t ns, const Src64* __restrict__ src, int64_t nt, const double2* __restrict__ tq,
+    const double* __restrict__ tw, const uint32_t* __restrict__ torder, int64_t chunk,
     double* __restrict__ ou, double* __restrict__ ov, double* __restrict__ ow, int direct,
     const int* __restrict__ gate) {
+  constexpr int kStepP = GATED ? 2 : 1, kStepW = GATED ? 4 : 1;
   // the Gaussian's velocity sum takes a loop without the per-pair cutoff test for a tile that
   // lies beyond the compact cutoff of every target of the wave (d^2 > 16 w for all its pairs)
   constexpr bool kFar = CORE == O2D_CORE_GAUSSIAN && RES == O2D_VELONLY;
-  if (kFar && gate && *gate == 0) return;
+  if constexpr (GATED) {
+    if (*gate == 0) return;
+  }
   __shared__ Src64 tile[kTile];
   __shared__ double tbox[kBlock / 64][5];  // per wave: x min/max, y min/max, largest radius term
   const int tid = threadIdx.x;
@@ -152,10 +148,10 @@ __global__ __launch_bounds__(kBlock) void nbody64_kernel(
   for (int t = 0; t < TPL; ++t) {
     const int64_t i = tbase + (int64_t)t * kBlock;
     const int64_t ii = i < nt ? i : nt - 1;
-    const double2 p = tg.pos[ii * tg.pstep];
+    const double2 p = tq[ii * kStepP];
     px[t] = p.x;
     py[t] = p.y;
-    pw[t] = TR ? tg.w[ii * tg.wstep] : 0.0;
+    pw[t] = TR ? tw[ii * kStepW] : 0.0;
     au[t] = av[t] = aw[t] = 0.0;
   }
   // when every target of the block has the same radius term w0, it is added to each source's
@@ -165,7 +161,7 @@ __global__ __launch_bounds__(kBlock) void nbody64_kernel(
   bool uni = false;
   if constexpr (TR) {
     const int64_t i0 = (int64_t)blockIdx.x * (kBlock * TPL);
-    w0 = tg.w[(i0 < nt ? i0 : nt - 1) * tg.wstep];
+    w0 = tw[(i0 < nt ? i0 : nt - 1) * kStepW];
     bool same = true;
 #pragma unroll
     for (int t = 0; t < TPL; ++t) same = same && pw[t] == w0;
@@ -249,7 +245,7 @@ __global__ __launch_bounds__(kBlock) void nbody64_kernel(
     const int64_t i = tbase + (int64_t)t * kBlock;
     if (i >= nt) continue;
     if (direct) {
-      const int64_t o = tg.order ? (int64_t)tg.order[i] : i;
+      const int64_t o = torder ? (int64_t)torder[i] : i;
       ou[o] += au[t];
       ov[o] += av[t];
       if (RES != O2D_VELONLY) ow[o] += aw[t];
@@ -476,11 +472,13 @@ struct Outputs {
 // 100,000 and 200,000 points: 28.5, 36.3, 45.4 and 69.1 with a thread per target, 24.9, 36.4, 47.8 and 74.0
 // split).
 constexpr int64_t kSplitChunks = 8, kSplitTargets = 65536;
-template <int NF, bool SPLIT>
+template <int NF, bool SPLIT, bool GATED>
 __global__ __launch_bounds__(SPLIT ? kReduceT : kBlock) void reduce_chunks_kernel(
     int64_t nchunk, int64_t nt, const uint32_t* __restrict__ order, const double* __restrict__ part,
     Outputs out, const int* __restrict__ gate, int open) {
-  if (gate && (*gate != 0) != (open != 0)) return;
+  if constexpr (GATED) {
+    if ((*gate != 0) != (open != 0)) return;
+  }
   constexpr int kWaves = SPLIT ? kReduceT / 64 : 1;
   static_assert(!SPLIT || NF <= kWaves, "a component per wave");
   const int lane = threadIdx.x & 63, wave = SPLIT ? threadIdx.x >> 6 : 0;
@@ -643,23 +641,30 @@ ChunkPlan plan_chunks(const Device* d, int64_t target_wgs, int64_t ntiles, int p
   return {nchunk, per};
 }
 
-template <int CORE, int RES, bool TR>
+// the targets of the fp64 form, as its kernel takes them
+struct Targets64 {
+  const double2* pos;
+  const double* w;
+  const uint32_t* order;
+};
+
+template <int CORE, int RES, bool TR, bool GATED = false>
 void launch64(bool few, dim3 grid, hipStream_t s, int64_t ns, const Src64* src, int64_t nt,
               const Targets64& tg, int64_t chunk, double* ou, double* ov, double* ow, int direct,
-              const int* gate) {
+              const int* gate = nullptr) {
   if (few)
-    nbody64_kernel<CORE, RES, TR, 1, true><<<grid, kBlock, 0, s>>>(ns, src, nt, tg, chunk, ou, ov, ow,
-                                                                   direct, gate);
+    nbody64_kernel<CORE, RES, TR, 1, true, GATED><<<grid, kBlock, 0, s>>>(
+        ns, src, nt, tg.pos, tg.w, tg.order, chunk, ou, ov, ow, direct, gate);
   else
-    nbody64_kernel<CORE, RES, TR, kTpl64, false><<<grid, kBlock, 0, s>>>(ns, src, nt, tg, chunk, ou,
-                                                                         ov, ow, direct, gate);
+    nbody64_kernel<CORE, RES, TR, kTpl64, false, GATED><<<grid, kBlock, 0, s>>>(
+        ns, src, nt, tg.pos, tg.w, tg.order, chunk, ou, ov, ow, direct, gate);
 }
 
 template <int CORE>
 void dispatch64(int res, bool tr_present, bool few, dim3 grid, hipStream_t s, int64_t ns,
                 const Src64* src, int64_t nt, const Targets64& tg, int64_t chunk, double* ou,
-                double* ov, double* ow, int direct, const int* gate) {
-#define O2D_L64(R, T) launch64<CORE, R, T>(few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate)
+                double* ov, double* ow, int direct) {
+#define O2D_L64(R, T) launch64<CORE, R, T>(few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct)
   if (res == O2D_VELONLY) {
     if (tr_present) O2D_L64(O2D_VELONLY, true);
     else O2D_L64(O2D_VELONLY, false);
@@ -750,15 +755,17 @@ int reduce_chunks(hipStream_t s, int64_t nchunk, int64_t nt, const uint32_t* ord
   const bool split = nchunk >= kSplitChunks && nt < kSplitTargets;
   const unsigned grid = split ? (unsigned)((nt + 63) / 64) : grid1(nt).x;
   const Outputs out{{o0, o1, o2, o3}};
-#define O2D_REDUCE(NF)                                                                      \
-  split ? reduce_chunks_kernel<NF, true><<<grid, kReduceT, 0, s>>>(nchunk, nt, order, part, \
-                                                                   out, gate, open)         \
-        : reduce_chunks_kernel<NF, false><<<grid, kBlock, 0, s>>>(nchunk, nt, order, part,  \
-                                                                  out, gate, open)
+#define O2D_REDUCE_G(NF, GATED)                                                             \
+  split ? reduce_chunks_kernel<NF, true, GATED>                                             \
+              <<<grid, kReduceT, 0, s>>>(nchunk, nt, order, part, out, gate, open)          \
+        : reduce_chunks_kernel<NF, false, GATED>                                            \
+              <<<grid, kBlock, 0, s>>>(nchunk, nt, order, part, out, gate, open)
+#define O2D_REDUCE(NF) gate ? O2D_REDUCE_G(NF, true) : O2D_REDUCE_G(NF, false)
   if (nf == 2) O2D_REDUCE(2);
   else if (nf == 3) O2D_REDUCE(3);
   else O2D_REDUCE(4);
 #undef O2D_REDUCE
+#undef O2D_REDUCE_G
   O2D_LAUNCH_CHECK();
   return 0;
 }
@@ -846,19 +853,26 @@ int sum64(Device* d, hipStream_t s, Workspace* ws, int core, int res, bool trp, 
     ov = ou + cp.nchunk * nt;
     ow = res == O2D_VELONLY ? nullptr : ov + cp.nchunk * nt;
   }
-  std::optional<KernelTimer> kt;
-  if (!gate) kt.emplace(trp ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT, s);
-  switch (core) {
-    case O2D_CORE_RM: dispatch64<O2D_CORE_RM>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
-    case O2D_CORE_GAUSSIAN: dispatch64<O2D_CORE_GAUSSIAN>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
-    case O2D_CORE_WL: dispatch64<O2D_CORE_WL>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
-    case O2D_CORE_V2: dispatch64<O2D_CORE_V2>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
-    default: dispatch64<O2D_CORE_V3>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate); break;
+  if (gate) {  // the Gaussian's velocity, timed with the clusters that it stands in for
+    constexpr int G = O2D_CORE_GAUSSIAN, V = O2D_VELONLY;
+    if (trp) launch64<G, V, true, true>(few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate);
+    else launch64<G, V, false, true>(few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct, gate);
+    O2D_LAUNCH_CHECK();
+    if (!direct) O2D_TRY(reduce_chunks(s, cp.nchunk, nt, tg.order, nf, ou, tu, tv, tw, nullptr, gate));
+    return 0;
   }
-  if (kt) kt->stop();
+  KernelTimer kt(trp ? O2D_KT_NBODY_PLAIN : O2D_KT_NBODY_PLAIN_PT, s);
+  switch (core) {
+    case O2D_CORE_RM: dispatch64<O2D_CORE_RM>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct); break;
+    case O2D_CORE_GAUSSIAN: dispatch64<O2D_CORE_GAUSSIAN>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct); break;
+    case O2D_CORE_WL: dispatch64<O2D_CORE_WL>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct); break;
+    case O2D_CORE_V2: dispatch64<O2D_CORE_V2>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct); break;
+    default: dispatch64<O2D_CORE_V3>(res, trp, few, grid, s, ns, src, nt, tg, chunk, ou, ov, ow, direct); break;
+  }
+  kt.stop();
   O2D_LAUNCH_CHECK();
   if (!direct) {
-    O2D_TRY(reduce_chunks(s, cp.nchunk, nt, tg.order, nf, ou, tu, tv, tw, nullptr, gate));
+    O2D_TRY(reduce_chunks(s, cp.nchunk, nt, tg.order, nf, ou, tu, tv, tw, nullptr));
   }
   return 0;
 }
@@ -871,7 +885,7 @@ int gauss_pairs_gated(Device* d, hipStream_t s, int64_t ns, const void* src, int
   const double* t = static_cast<const double*>(trg);
   return sum64(d, s, nullptr, O2D_CORE_GAUSSIAN, O2D_VELONLY, radii, ns,
                static_cast<const Src64*>(src), nt,
-               Targets64{reinterpret_cast<const double2*>(t), t + 3, torder, 2, 4}, tu, tv, nullptr, gate);
+               Targets64{reinterpret_cast<const double2*>(t), t + 3, torder}, tu, tv, nullptr, gate);
 }
 
 int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns, const double* sx,
@@ -920,7 +934,7 @@ int nbody_dev(Device* d, hipStream_t s, int core, int prec, int res, int64_t ns,
     O2D_TRY(prep_targets<double>(d, s, ws, core, nt, tx, ty, tr, sort, self ? order : nullptr,
                                  &torder, &tq, &twv));
 
-    return sum64(d, s, ws, core, res, trp, ns, src, nt, Targets64{tq, twv, torder, 1, 1}, tu, tv, tw,
+    return sum64(d, s, ws, core, res, trp, ns, src, nt, Targets64{tq, twv, torder}, tu, tv, tw,
                  nullptr);
   }
 
