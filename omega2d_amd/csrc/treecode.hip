@@ -1219,6 +1219,15 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
   while (sl > 0 && lv.cnt[sl - 1] <= 64) --sl;
   ga.start = (uint32_t)lv.off[sl];
   ga.nstart = (uint32_t)lv.cnt[sl];
+  KernelTimer kt(q.timed, s);
+  // before the shares' partial sums are taken: both are the kPartials slot, which may move when it grows
+  if (gate) {
+    if constexpr (ADJ)
+      O2D_TRY(adjoint_pairs_dev(d, s, q.core, nt, q.tx, q.ty, q.ts, q.tr, ns, q.sx, q.sy, q.sb, q.sa,
+                                q.o1, q.o2, q.o0, q.o3, gate));
+    else
+      O2D_TRY(gauss_pairs_gated(d, s, ns, src, nt, trg, q.tr != nullptr, torder, q.o0, q.o1, gate));
+  }
   const int nf = ADJ ? 4 : 2;
   double* part = nullptr;
   if (ga.ksplit > 1) {
@@ -1239,14 +1248,6 @@ int tree_run(Device* d, hipStream_t s, const Problem& q) {
     front = reinterpret_cast<uint32_t*>(super + nsuper);
   }
   const uint32_t root = (uint32_t)lv.off[lv.n - 1];
-  KernelTimer kt(q.timed, s);
-  if (gate) {
-    if constexpr (ADJ)
-      O2D_TRY(adjoint_pairs_dev(d, s, q.core, nt, q.tx, q.ty, q.ts, q.tr, ns, q.sx, q.sy, q.sb, q.sa,
-                                q.o1, q.o2, q.o0, q.o3, gate));
-    else
-      O2D_TRY(gauss_pairs_gated(d, s, ns, src, nt, trg, q.tr != nullptr, torder, q.o0, q.o1, gate));
-  }
 #define O2D_EVAL(C) \
   launch_eval<C, ADJ>(q, s, nsuper, ga, trg, torder, head, kids, mom, src, root, super, local, front, part)
   switch (q.core) {
