@@ -286,8 +286,9 @@ int o2d_hip_points_on_points_adjoint_dev_d(const o2d_env* env, int64_t ns, const
  * centre c) acts on a target z through its complex moments when r <= theta |z - c| and the
  * core equals 1/d^2 for every pair to within core_tol (exactly, for the Gaussian, beyond its
  * compact cutoff); otherwise it is opened, and leaves of 32 sources are summed directly with
- * the exact core in fp64. The truncation error of a used cell is about (theta)^order of its
- * contribution. order: 1..32; theta in (0, 1); core_tol >= 0 (ignored by the Gaussian). */
+ * the exact core in fp64. The truncation error of a used cell is at most about (theta)^order of its
+ * contribution (cells near theta's limit may use a few moments more than order, or be opened a
+ * little before it, and far ones fewer, to that end). order: 1..32; theta in (0, 1); core_tol >= 0 (ignored by the Gaussian). */
 typedef struct o2d_tree_opts {
   double theta;
   int32_t order;

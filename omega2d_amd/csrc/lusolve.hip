@@ -6,12 +6,13 @@
 // the inverse of its diagonal block (kSB x kSB, prepared once per factorisation) and takes it off
 // its own rows of what is left, so a launch spreads its column panel over the chip and the
 // launches' own latency (2 x 33 at order 2049, 4 us each) is what remains: 0.92 -> 0.27 ms a solve,
-// after 0.04 ms for the diagonal blocks.
+// after 0.017 ms for the diagonal blocks.
 // Row interchanges are applied to the right-hand side as a gather by the permutation that the
 // factorisation composed block by block.
 //
 // With the explicit inverse a solve is one matrix-vector product, split over columns so that the
-// read is spread over the chip, partial sums added in order: 83 -> 12.5 us at order 2049.
+// read is spread over the chip, partial sums added in order: 83 -> 12.5 us at order 2049; up to order
+// kOnceMax in one launch.
 #include <algorithm>
 
 #include "nbody.h"

@@ -2,9 +2,10 @@
 //
 // fp64 forms follow the reference's arithmetic closely enough for 1e-12 relative agreement:
 // reciprocals and reciprocal square roots are the hardware seeds refined by one third-order step
-// (about 1 ulp, as two Newton steps), exp/cbrt come from the device math library. fp32 forms are the split-precision
-// pair math: one hardware reciprocal (or rsq) per pair, the Gaussian's exp only inside its
-// core (d^2 <= 16 sigma^2), evaluated as an expm1-style series where 1 - e^-x would cancel.
+// (about 1 ulp, as two Newton steps); the Gaussian's velocity takes its own exp (exp_neg_core), its
+// vorticity and shear the device math library's, V3 the library's rcbrt. fp32 forms are the
+// split-precision pair math: one hardware reciprocal (or rsq) per pair, the Gaussian's exp only inside
+// its core (d^2 <= 16 sigma^2), evaluated as an expm1-style series where 1 - e^-x would cancel.
 #pragma once
 
 #include <hip/hip_runtime.h>

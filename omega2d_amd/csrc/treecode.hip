@@ -32,10 +32,12 @@
 //
 // What bounds it: issue of the near pairs and of the moment sums. One wave that popped one cell
 // at a time from its own stack spent most of its time waiting for that cell's record and moments;
-// testing 64 cells at once takes a handful of dependent loads per wave, records of known cells
-// come as scalar loads, and the far cells of 1,024 targets are summed once, not sixteen times.
-// 1M blob particles on themselves plus 65,536 tracers (theta 0.6, order 28): 7.6 -> 3.1 ms, of which
-// the particles' groups 2.0, the tracers' 0.47, the two trees and orders 0.5.
+// testing 64 cells at once takes a handful of dependent loads per wave, a far cell's moments and a
+// leaf's sources come through LDS, and the far cells of 1,024 targets are summed once, not sixteen
+// times. The group kernel is held to 128 registers, four waves per SIMD (the Gaussian's then spills 12
+// to 14 of them, the adjoint's 40 to 43). 1M blob particles on themselves plus 65,536 tracers (theta
+// 0.6, order 28): 7.6 -> 3.2 ms, of which the particles' groups 2.1, the tracers' 0.58, the super groups
+// 0.2, the trees and orders 0.5.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
